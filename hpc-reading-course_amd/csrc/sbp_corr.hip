@@ -3,20 +3,18 @@
 // coarse RK4 step.  Its inputs at each point are eight normalised features of
 // the state and the materials (the fourth-difference terms of the stencil's
 // leading truncation error, the fourth differences of u, v and p, rho and
-// K: pack_state_tiled_kernel / pack_batch_tiled_kernel below).  Training
-// (forward and backward) runs on v_mfma_f32_16x16x16_bf16, inference on
-// v_mfma_f32_16x16x32_bf16 (fused_net_kernel), with FP32 accumulation;
-// master weights and Adam moments are FP32.  No counterpart in the
+// K: pack_state_tiled_kernel / pack_batch_tiled_kernel below).  Every
+// convolution and gradient runs on v_mfma_f32_16x16x32_bf16 with FP32
+// accumulation; master weights and Adam moments are FP32.  No counterpart in the
 // reference: the plain fine-grid solve of the same path is its fallback and
 // reference, and a correction that lifts the discrete energy above the
 // energy the solve started from by more than a set bound is rejected.
 //
-// Activations are channels-last [image][y][x][channel] in bf16, channels
-// padded to a multiple of 4.  A training convolution is a GEMM with M = 16
-// pixels of one image row, N = output channels, K = 9 taps x input channels
-// (padded to a multiple of 16); one wavefront owns a 16-pixel segment.  Backward-data is the same kernel with the weights transposed and
-// the taps mirrored; weight gradients are a GEMM reduced over pixels, written
-// as per-wavefront partials and summed in a fixed order (deterministic).
+// Activations are channels-last [image][y][x][channel] in bf16.  Forward
+// (fused_net_kernel, inference and training) and backward-data
+// (fused_back_kernel) march down windows of an image with all layers in one
+// kernel; weight gradients (wgrad_kernel) are GEMMs reduced over pixels,
+// written as per-block partials and summed in a fixed order (deterministic).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -49,13 +47,12 @@ constexpr int NORM_OUT = 2 * C_IN, NORM_LEN = 2 * C_IN + C_OUT;
 constexpr int KP1 = 80;   // 9*8 = 72 padded to 80
 constexpr int KP2 = 288;  // 9*32
 constexpr int KP3 = 288;
-constexpr int KP3T = 144;  // backward-data of layer 3: 9*16
+constexpr int C_D3 = 8;   // channels of the output gradient in memory (3 real); its transposed weights take KP1
 constexpr int N_W1 = C_H * C_IN * 9, N_B1 = C_H;
 constexpr int N_W2 = C_H * C_H * 9, N_B2 = C_H;
 constexpr int N_W3 = C_OUT * C_H * 9, N_B3 = C_OUT;
 constexpr int OFF_W1 = 0, OFF_B1 = OFF_W1 + N_W1, OFF_W2 = OFF_B1 + N_B1, OFF_B2 = OFF_W2 + N_W2;
 constexpr int OFF_W3 = OFF_B2 + N_B2, OFF_B3 = OFF_W3 + N_W3, N_PARAMS = OFF_B3 + N_B3;
-constexpr int WG_WAVES = 1024;  // wavefronts of the weight-gradient reduction
 
 __device__ __forceinline__ bf16 f2bf(float f)
 {
@@ -67,174 +64,6 @@ __device__ __forceinline__ bf16 f2bf(float f)
 
 __device__ __forceinline__ float bf2f(bf16 h) { return __uint_as_float(((unsigned)h) << 16); }
 
-// --------------------------------------------------------------------------
-// conv3x3 as MFMA GEMM.  MODE 0: + bias, ReLU, bf16 out (COUT_P channels);
-// MODE 1: + bias, fp32 out (first out_ch channels); MODE 2: fp32 out, no bias.
-// wt is [COUT_P][KP] bf16 with k = tap * CIN_P + ci, tap = 3*(dy+1) + (dx+1).
-// --------------------------------------------------------------------------
-template <int CIN_P, int COUT_P, int KP, int MODE>
-__global__ __launch_bounds__(256) void conv3x3_kernel(const bf16 *__restrict__ in, int nimg, int H, int W,
-                                                      const bf16 *__restrict__ wt, const float *__restrict__ bias,
-                                                      bf16 *__restrict__ out_bf, float *__restrict__ out_f, int out_ch)
-{
-  static_assert(CIN_P % 4 == 0 && COUT_P % 16 == 0 && KP % 16 == 0, "MFMA tiling");
-  constexpr int NT = COUT_P / 16, NK = KP / 16;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int m = lane & 15, kg = lane >> 4;
-  // The wavefront's B fragments (all weights it needs) stay in registers
-  // while it walks its 16-pixel segments.
-  bf16x4 bw[NK][NT];
-#pragma unroll
-  for (int ks = 0; ks < NK; ks++)
-#pragma unroll
-    for (int t = 0; t < NT; t++)
-      bw[ks][t] = *reinterpret_cast<const bf16x4 *>(wt + (long)(t * 16 + m) * KP + ks * 16 + kg * 4);
-  float bv[NT];
-#pragma unroll
-  for (int t = 0; t < NT; t++) bv[t] = MODE != 2 ? bias[t * 16 + m] : 0.f;
-  const int segs = (W + 15) / 16;
-  const long nseg = (long)nimg * H * segs;
-  for (long seg = (long)blockIdx.x * 4 + wv; seg < nseg; seg += (long)gridDim.x * 4) {
-    const int sx = (int)(seg % segs);
-    const long row = seg / segs;
-    const int y = (int)(row % H), img = (int)(row / H);
-    const int x0 = sx * 16;
-    f32x4 acc[NT];
-#pragma unroll
-    for (int t = 0; t < NT; t++) acc[t] = f32x4{0, 0, 0, 0};
-    const long img_base = (long)img * H * W;
-#pragma unroll
-    for (int ks = 0; ks < NK; ks++) {
-      const int k0 = ks * 16 + kg * 4;
-      const int tap = k0 / CIN_P, ci = k0 - tap * CIN_P;
-      bf16x4 a = {0, 0, 0, 0};
-      if (tap < 9) {
-        const int yy = y + tap / 3 - 1, xx = x0 + m + tap % 3 - 1;
-        if (yy >= 0 && yy < H && xx >= 0 && xx < W)
-          a = *reinterpret_cast<const bf16x4 *>(in + (img_base + (long)yy * W + xx) * CIN_P + ci);
-      }
-#pragma unroll
-      for (int t = 0; t < NT; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bw[ks][t], acc[t], 0, 0, 0);
-    }
-    // acc[t][i] = C[row 4*kg+i][col m]: pixel x0 + 4*kg + i, output channel 16*t + m
-#pragma unroll
-    for (int t = 0; t < NT; t++) {
-      const int co = t * 16 + m;
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int px = x0 + 4 * kg + i;
-        if (px >= W) continue;
-        const float v = acc[t][i] + bv[t];
-        const long p = img_base + (long)y * W + px;
-        if constexpr (MODE == 0) {
-          out_bf[p * COUT_P + co] = f2bf(v > 0.f ? v : 0.f);
-        } else {
-          if (co < out_ch) out_f[p * out_ch + co] = v;
-        }
-      }
-    }
-  }
-}
-
-// Weight gradient dW[co][k] = sum_p dY[p][co] * patch(X)[p][k]: GEMM with
-// M = output channels, N = K-index, reduced over pixels (16 per MFMA step).
-template <int CIN_P, int COUT_P, int KP>
-__global__ __launch_bounds__(256) void wgrad_kernel(const bf16 *__restrict__ X, const bf16 *__restrict__ dY, int nimg,
-                                                    int H, int W, float *__restrict__ partial)
-{
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const long wid = (long)blockIdx.x * 4 + wv, nw = (long)gridDim.x * 4;
-  constexpr int MT = COUT_P / 16, NT = KP / 16;
-  const int r = lane & 15, kg = lane >> 4;
-  f32x4 acc[MT][NT];
-#pragma unroll
-  for (int a = 0; a < MT; a++)
-#pragma unroll
-    for (int b = 0; b < NT; b++) acc[a][b] = f32x4{0, 0, 0, 0};
-  const int segs = (W + 15) / 16;
-  const long nseg = (long)nimg * H * segs;
-  for (long seg = wid; seg < nseg; seg += nw) {
-    const int sx = (int)(seg % segs);
-    const long row = seg / segs;
-    const int y = (int)(row % H), img = (int)(row / H);
-    const int x0 = sx * 16;
-    const long img_base = (long)img * H * W;
-    bf16x4 a[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int px = x0 + 4 * kg + i;
-        a[mt][i] = px < W ? (short)dY[(img_base + (long)y * W + px) * COUT_P + mt * 16 + r] : (short)0;
-      }
-#pragma unroll
-    for (int nt = 0; nt < NT; nt++) {
-      const int kidx = nt * 16 + r;
-      const int tap = kidx / CIN_P, ci = kidx - tap * CIN_P;
-      bf16x4 b = {0, 0, 0, 0};
-      if (tap < 9) {
-        const int yy = y + tap / 3 - 1;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const int px = x0 + 4 * kg + i, xx = px + tap % 3 - 1;
-          if (px < W && yy >= 0 && yy < H && xx >= 0 && xx < W)
-            b[i] = (short)X[(img_base + (long)yy * W + xx) * CIN_P + ci];
-        }
-      }
-#pragma unroll
-      for (int mt = 0; mt < MT; mt++) acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[mt], b, acc[mt][nt], 0, 0, 0);
-    }
-  }
-  float *P = partial + wid * COUT_P * KP;
-#pragma unroll
-  for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-    for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) P[(mt * 16 + 4 * kg + i) * KP + nt * 16 + r] = acc[mt][nt][i];
-}
-
-// Sum the per-wavefront partials in a fixed order and scatter the real
-// entries into the flat gradient [co][ci][ky][kx].
-__global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float *__restrict__ partial, int nw, int cout,
-                                                           int cin, int cin_p, int cout_p, int kp,
-                                                           float *__restrict__ grad)
-{
-  const int e = blockIdx.x * 256 + threadIdx.x;
-  if (e >= cout * cin * 9) return;
-  const int co = e / (cin * 9), rem = e % (cin * 9), ci = rem / 9, tap = rem % 9;
-  const long idx = (long)co * kp + tap * cin_p + ci;
-  float s = 0.f;
-  for (int w = 0; w < nw; w++) s += partial[(long)w * cout_p * kp + idx];
-  grad[e] = s;
-}
-
-// Bias gradient db[co] = sum_p dY[p][co] (first cout of cout_p channels).
-__global__ __launch_bounds__(256) void bgrad_kernel(const bf16 *__restrict__ dY, long npix, int cout, int cout_p,
-                                                    float *__restrict__ grad)
-{
-  __shared__ float sh[256];
-  const int co = blockIdx.x;
-  float s = 0.f;
-  for (long p = threadIdx.x; p < npix; p += 256) s += bf2f(dY[p * cout_p + co]);
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
-    if (threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) grad[co] = sh[0];
-  (void)cout;
-}
-
-// dPre = dA * (A > 0) in bf16 (A holds post-ReLU activations).
-__global__ __launch_bounds__(256) void relu_back_kernel(const float *__restrict__ dA, const bf16 *__restrict__ A,
-                                                        long n, bf16 *__restrict__ dpre)
-{
-  const long i = blockIdx.x * 256L + threadIdx.x;
-  if (i < n) dpre[i] = f2bf(bf2f(A[i]) > 0.f ? dA[i] : 0.f);
-}
-
 // Whether the correction acts at grid point (i, j) of an H x W image: the
 // points closer than `band` to a wall (the boundary-closure rows) keep the
 // plain scheme's values, and the training loss ignores them.
@@ -244,8 +73,9 @@ __device__ __forceinline__ bool corrected_at(int i, int j, int W, int H, int ban
 }
 
 // MSE loss over the C_OUT real channels and its gradient 2(y - t)/N in bf16
-// (padded channels, and points outside the corrected region, zero; N counts
-// every point).  Per-block partial sums of squares in FP64.
+// (C_D3 channels per pixel; the padded channels, and points outside the
+// corrected region, zero; N counts every point).  Per-block partial sums of
+// squares in FP64.
 __global__ __launch_bounds__(256) void loss_kernel(const float *__restrict__ y, const float *__restrict__ t, long npix,
                                                    int H, int W, int band, double inv_n, bf16 *__restrict__ dY,
                                                    double *__restrict__ partial)
@@ -257,16 +87,16 @@ __global__ __launch_bounds__(256) void loss_kernel(const float *__restrict__ y, 
     const long q = p % npi;
     const int j = (int)(q / W), i = (int)(q - (long)j * W);
     const bool on = corrected_at(i, j, W, H, band);
+    __attribute__((aligned(16))) bf16 g[C_D3] = {0};
 #pragma unroll
-    for (int c = 0; c < C_OUTP; c++) {
-      float g = 0.f;
-      if (c < C_OUT && on) {
-        const float d = y[p * C_OUT + c] - t[p * C_OUT + c];
+    for (int c = 0; c < C_OUT; c++) {
+      const float d = y[p * C_OUT + c] - t[p * C_OUT + c];
+      if (on) {
         s += (double)d * d;
-        g = (float)(2.0 * inv_n) * d;
+        g[c] = f2bf((float)(2.0 * inv_n) * d);
       }
-      dY[p * C_OUTP + c] = f2bf(g);
     }
+    *reinterpret_cast<uint4 *>(dY + p * C_D3) = *reinterpret_cast<const uint4 *>(g);
   }
   sh[threadIdx.x] = s;
   __syncthreads();
@@ -275,15 +105,6 @@ __global__ __launch_bounds__(256) void loss_kernel(const float *__restrict__ y, 
     __syncthreads();
   }
   if (threadIdx.x == 0) partial[blockIdx.x] = sh[0];
-}
-
-__global__ void sum_kernel(const double *__restrict__ partial, int n, double scale, double *__restrict__ out)
-{
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    double s = 0;
-    for (int k = 0; k < n; k++) s += partial[k];
-    out[0] = s * scale;
-  }
 }
 
 // Adam on the FP32 master parameters.
@@ -326,10 +147,10 @@ __global__ __launch_bounds__(256) void prepare_weights_kernel(const float *__res
     const int co = i / KP3, k = i % KP3, tap = k / C_H, ci = k % C_H;
     w3[i] = co < C_OUT ? f2bf(p[OFF_W3 + (co * C_H + ci) * 9 + tap]) : (bf16)0;
   }
-  if (i < C_H * KP3T) {
-    // backward-data of layer 3: W3T[ci][tap'*16 + co] = W3[co][8-tap'][ci]
-    const int ci = i / KP3T, k = i % KP3T, tp = k / C_OUTP, co = k % C_OUTP;
-    w3t[i] = co < C_OUT ? f2bf(p[OFF_W3 + (co * C_H + ci) * 9 + (8 - tp)]) : (bf16)0;
+  if (i < C_H * KP1) {
+    // backward-data of layer 3: W3T[ci][tap'*8 + co] = W3[co][8-tap'][ci]
+    const int ci = i / KP1, k = i % KP1, tp = k / C_D3, co = k % C_D3;
+    w3t[i] = (tp < 9 && co < C_OUT) ? f2bf(p[OFF_W3 + (co * C_H + ci) * 9 + (8 - tp)]) : (bf16)0;
   }
   if (i < C_H) {
     b1[i] = p[OFF_B1 + i];
@@ -382,8 +203,7 @@ __global__ __launch_bounds__(256) void pack_raw_kernel(const float *__restrict__
 // evaluated on all 64 window columns; a value at window column w is exact
 // when its inputs at w-1..w+1 are, so the output is exact on w in [3, 60]: 58
 // output columns per window.  Activations at positions outside the image are
-// zero (the zero padding of the layer-by-layer kernels), so the output equals
-// forward()'s up to the FP32 accumulation order.
+// zero (the network's zero padding).
 // --------------------------------------------------------------------------
 using bf16x8 = __attribute__((ext_vector_type(8))) short;
 using vbf8 = __attribute__((ext_vector_type(8))) __bf16;
@@ -447,13 +267,16 @@ inline long net_blocks_per_image(int H, int W)
 }
 
 // T: type of the state whose corrected energy the epilogue reduces; void for
-// plain inference.
-template <typename T>
+// plain inference.  KEEP: also store the activations of layers 1 and 2 (the
+// training forward; each block its own rows and 58 columns): 78 us for 16
+// images of 257^2 against 289 us for one convolution launch per layer.
+template <typename T, bool KEEP>
 __global__ __launch_bounds__(256) void fused_net_kernel(const bf16 *__restrict__ X, int nimg, int H, int W, int rows,
                                                         const bf16 *__restrict__ w1, const float *__restrict__ b1,
                                                         const bf16 *__restrict__ w2, const float *__restrict__ b2,
                                                         const bf16 *__restrict__ w3, const float *__restrict__ b3,
-                                                        float *__restrict__ out, NetEnergyArgs ea)
+                                                        float *__restrict__ out, bf16 *__restrict__ keep1,
+                                                        bf16 *__restrict__ keep2, NetEnergyArgs ea)
 {
   __shared__ __attribute__((aligned(16))) bf16 s_in[2][FPX * C_INP];
   __shared__ __attribute__((aligned(16))) bf16 s_a1[2][FPX * F1S];
@@ -518,6 +341,12 @@ __global__ __launch_bounds__(256) void fused_net_kernel(const bf16 *__restrict__
   f32x4 q3 = zero;  // layer 3 running sums: register dy of lane (c, pixel)
   __syncthreads();
 
+  // KEEP: this wave's 4 channels of the block's own pixels
+  auto keep_row = [&](bf16 *__restrict__ dst, int r, int w, uint2 v) {
+    if (r >= y0 && r < y1 && w >= 3 && w < FW - 3 && c0 + w < W)
+      *reinterpret_cast<uint2 *>(dst + (ibase + (long)r * W + c0 + w) * C_H + tc * 16 + 4 * kg) = v;
+  };
+
   // Step t with ring slot P = t % 2: X completes its rows, Y is one row
   // behind, Z starts.
   auto step = [&](int t, auto P, FusedRows &Xr, FusedRows &Yr, FusedRows &Zr) {
@@ -542,8 +371,9 @@ __global__ __launch_bounds__(256) void fused_net_kernel(const bf16 *__restrict__
         Yr.l1[u] = mfma32(bw1[1], a, Yr.l1[u]);
         Xr.l1[u] = mfma32(bw1[2], a, Xr.l1[u]);
         const int col = c0 + 16 * sg + m;
-        *reinterpret_cast<uint2 *>(s_a1[ws] + (16 * sg + m + 1) * F1S + tc * 16 + 4 * kg) =
-            relu_pack4(Xr.l1[u], rin && col >= 0 && col < W);
+        const uint2 v = relu_pack4(Xr.l1[u], rin && col >= 0 && col < W);
+        *reinterpret_cast<uint2 *>(s_a1[ws] + (16 * sg + m + 1) * F1S + tc * 16 + 4 * kg) = v;
+        if constexpr (KEEP) keep_row(keep1, r, 16 * sg + m, v);
       }
     }
     // layer 2: layer-1 rows y0-2 .. y1+1 (steps 4 .. rows+7); completes row y0-7+t
@@ -565,8 +395,9 @@ __global__ __launch_bounds__(256) void fused_net_kernel(const bf16 *__restrict__
 #pragma unroll
         for (int dx = 0; dx < 3; dx++) Xr.l2[u] = mfma32(bw2[6 + dx], a[dx], Xr.l2[u]);
         const int col = c0 + 16 * sg + m;
-        *reinterpret_cast<uint2 *>(s_a2[ws] + (16 * sg + m + 1) * F1S + tc * 16 + 4 * kg) =
-            relu_pack4(Xr.l2[u], rin && col >= 0 && col < W);
+        const uint2 v = relu_pack4(Xr.l2[u], rin && col >= 0 && col < W);
+        *reinterpret_cast<uint2 *>(s_a2[ws] + (16 * sg + m + 1) * F1S + tc * 16 + 4 * kg) = v;
+        if constexpr (KEEP) keep_row(keep2, r, 16 * sg + m, v);
       }
     }
     // layer 3: layer-2 rows y0-1 .. y1 (steps 7 .. rows+8); completes output
@@ -659,6 +490,462 @@ __global__ __launch_bounds__(256) void fused_net_kernel(const bf16 *__restrict__
     }
     const double sm = block_sum_256(acc, sh);
     if (threadIdx.x == 0) ea.partial[blockIdx.x] = sm;
+  }
+}
+
+// --------------------------------------------------------------------------
+// Fused backward-data: the ReLU-masked gradients of layers 2 and 1,
+//   dP2 = [A2 > 0] (W3^T * dY3),   dP1 = [A1 > 0] (W2^T * dP2)
+// (* a 3x3 convolution with the mirrored, channel-transposed weights), of one
+// image window in one kernel: the march of fused_net_kernel with two layers.
+// Both are stored (the weight gradients read them), each block its own rows
+// and 58 columns; dP2 also stays in LDS for the second convolution.  The masks
+// are fetched two steps ahead like the input row.
+//
+// Bound: its 290 MB of mask loads and stores and the row march's latency: 80
+// us for 16 images of 257^2 (3.6 TB/s).  One convolution launch per layer, its
+// FP32 output and a masking launch took 391 us.
+// --------------------------------------------------------------------------
+// 4 channels of one pixel: bf16, kept where the activation was positive
+// (positive and not NaN: bit patterns 1 .. 0x7f80), zero outside the image
+__device__ __forceinline__ uint2 mask_pack4(f32x4 acc, uint2 a, bool in)
+{
+  const unsigned lo = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{acc[0], acc[1]}, vbf2));
+  const unsigned hi = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{acc[2], acc[3]}, vbf2));
+  auto keep = [&](unsigned v, unsigned m) {
+    const bool k0 = (m & 0xffffu) - 1u < 0x7f80u, k1 = (m >> 16) - 1u < 0x7f80u;
+    return (in && k0 ? v & 0xffffu : 0u) | (in && k1 ? v & 0xffff0000u : 0u);
+  };
+  return uint2{keep(lo, a.x), keep(hi, a.y)};
+}
+
+constexpr int BACK_HALO = 6;  // row steps beyond the chunk's rows
+
+__global__ __launch_bounds__(256) void fused_back_kernel(const bf16 *__restrict__ dY3, int H, int W, int rows,
+                                                         const bf16 *__restrict__ w3t, const bf16 *__restrict__ w2t,
+                                                         const bf16 *__restrict__ A2, const bf16 *__restrict__ A1,
+                                                         bf16 *__restrict__ dP2, bf16 *__restrict__ dP1)
+{
+  __shared__ __attribute__((aligned(16))) bf16 s_in[2][FPX * C_D3];
+  __shared__ __attribute__((aligned(16))) bf16 s_a[2][FPX * F1S];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int m = lane & 15, kg = lane >> 4;
+  const int strips = (W + FOUT - 1) / FOUT, chunks = (H + rows - 1) / rows;
+  const int b = blockIdx.x;
+  const int img = b / (strips * chunks), rem = b - img * strips * chunks;
+  const int strip = rem / chunks, chunk = rem - strip * chunks;
+  const int c0 = strip * FOUT - 3;
+  const int y0 = chunk * rows, y1 = min(y0 + rows, H);
+  const long ibase = (long)img * H * W;
+  for (int q = threadIdx.x; q < 2 * FPX * F1S; q += 256) (&s_a[0][0])[q] = 0;  // the pad pixels stay zero
+
+  const int tc = wv & 1, sA = wv >> 1;
+  bf16x8 bw3[3], bw2[9];
+#pragma unroll
+  for (int dy = 0; dy < 3; dy++)
+    bw3[dy] = kg < 3 ? *reinterpret_cast<const bf16x8 *>(w3t + (long)(tc * 16 + m) * KP1 + dy * 24 + kg * 8) : bf16x8{};
+#pragma unroll
+  for (int tp = 0; tp < 9; tp++)
+    bw2[tp] = *reinterpret_cast<const bf16x8 *>(w2t + (long)(tc * 16 + m) * KP2 + tp * 32 + kg * 8);
+
+  const int nsteps = (y1 - y0) + BACK_HALO;
+  const int ipx = min((int)threadIdx.x, FIN_PARTS - 1) >> 1, icol = c0 - 1 + ipx;
+  const bool iload = icol >= 0 && icol < W;
+  const long ioff = ibase * C_D3 + (long)min(max(icol, 0), W - 1) * C_D3 + 4 * (threadIdx.x & 1);
+  auto load_in = [&](int ri) {
+    return *reinterpret_cast<const uint2 *>(dY3 + ioff + (long)min(max(ri, 0), H - 1) * W * C_D3);
+  };
+  // this lane's 4 channels of its two pixels, at image row r (clamped: what
+  // lies outside is masked when it is used)
+  const int ch = tc * 16 + 4 * kg;
+  const int col[2] = {c0 + 16 * sA + m, c0 + 16 * (sA + 2) + m};
+  long aoff[2];
+#pragma unroll
+  for (int u = 0; u < 2; u++) aoff[u] = (ibase + min(max(col[u], 0), W - 1)) * C_H + ch;
+  auto load_mask = [&](const bf16 *A, int u, int r) {
+    return *reinterpret_cast<const uint2 *>(A + aoff[u] + (long)min(max(r, 0), H - 1) * W * C_H);
+  };
+  const f32x4 zero = {0, 0, 0, 0};
+  uint2 in_q[2] = {load_in(y0 - 2), load_in(y0 - 1)};  // rows of steps t, t + 1
+  uint2 m2[2][2], m1[2][2];                            // masks of the rows completed in steps t, t + 1
+#pragma unroll
+  for (int k = 0; k < 2; k++)
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      m2[k][u] = load_mask(A2, u, y0 - 4 + k);
+      m1[k][u] = load_mask(A1, u, y0 - 6 + k);
+    }
+  __syncthreads();
+
+  auto step = [&](int t, auto P, FusedRows &Xr, FusedRows &Yr, FusedRows &Zr) {
+    constexpr int ws = decltype(P)::value, rs = ws ^ 1;
+    if (threadIdx.x < FIN_PARTS) {
+      const int ri = y0 - 2 + t;
+      const bool in = iload && ri >= 0 && ri < H;
+      *reinterpret_cast<uint2 *>(s_in[ws] + 4 * threadIdx.x) = uint2{in ? in_q[ws].x : 0u, in ? in_q[ws].y : 0u};
+    }
+    in_q[ws] = load_in(y0 + t);
+    uint2 k2[2], k1[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      k2[u] = m2[ws][u];
+      k1[u] = m1[ws][u];
+      m2[ws][u] = load_mask(A2, u, y0 - 2 + t);
+      m1[ws][u] = load_mask(A1, u, y0 - 4 + t);
+    }
+    // layer 3's transpose: dY3 rows y0-2 .. y1+1 (steps 1 .. rows+4); completes dP2 row y0-4+t
+    if (t >= 1 && t <= nsteps - 2) {
+      const int r = y0 - 4 + t;
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const int w = 16 * (sA + 2 * u) + m;
+        const bf16x8 a = *reinterpret_cast<const bf16x8 *>(s_in[rs] + (w + min(kg, 2)) * C_D3);
+        Zr.l1[u] = mfma32(bw3[0], a, zero);
+        Yr.l1[u] = mfma32(bw3[1], a, Yr.l1[u]);
+        Xr.l1[u] = mfma32(bw3[2], a, Xr.l1[u]);
+        const uint2 v = mask_pack4(Xr.l1[u], k2[u], r >= 0 && r < H && col[u] >= 0 && col[u] < W);
+        *reinterpret_cast<uint2 *>(s_a[ws] + (w + 1) * F1S + ch) = v;
+        if (r >= y0 && r < y1 && w >= 3 && w < FW - 3 && col[u] < W)
+          *reinterpret_cast<uint2 *>(dP2 + (ibase + (long)r * W + col[u]) * C_H + ch) = v;
+      }
+    }
+    // layer 2's transpose: dP2 rows y0-1 .. y1 (steps 4 .. rows+5); completes dP1 row y0-6+t
+    if (t >= 4 && t < nsteps) {
+      const int r = y0 - 6 + t;
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const int w = 16 * (sA + 2 * u) + m;
+        bf16x8 a[3];
+#pragma unroll
+        for (int dx = 0; dx < 3; dx++) a[dx] = *reinterpret_cast<const bf16x8 *>(s_a[rs] + (w + dx) * F1S + kg * 8);
+        Zr.l2[u] = zero;
+#pragma unroll
+        for (int dx = 0; dx < 3; dx++) Zr.l2[u] = mfma32(bw2[dx], a[dx], Zr.l2[u]);
+#pragma unroll
+        for (int dx = 0; dx < 3; dx++) Yr.l2[u] = mfma32(bw2[3 + dx], a[dx], Yr.l2[u]);
+#pragma unroll
+        for (int dx = 0; dx < 3; dx++) Xr.l2[u] = mfma32(bw2[6 + dx], a[dx], Xr.l2[u]);
+        if (r >= y0 && r < y1 && w >= 3 && w < FW - 3 && col[u] < W)
+          *reinterpret_cast<uint2 *>(dP1 + (ibase + (long)r * W + col[u]) * C_H + ch) = mask_pack4(Xr.l2[u], k1[u], true);
+      }
+    }
+    __syncthreads();
+  };
+  FusedRows ra, rb, rc;
+#pragma unroll
+  for (int u = 0; u < 2; u++) ra.l1[u] = rb.l1[u] = rc.l1[u] = ra.l2[u] = rb.l2[u] = rc.l2[u] = zero;
+  for (int t = 0; t < nsteps; t += 6) {
+    step(t, IC<0>{}, ra, rb, rc);
+    step(t + 1, IC<1>{}, rb, rc, ra);
+    step(t + 2, IC<0>{}, rc, ra, rb);
+    step(t + 3, IC<1>{}, ra, rb, rc);
+    step(t + 4, IC<0>{}, rb, rc, ra);
+    step(t + 5, IC<1>{}, rc, ra, rb);
+  }
+}
+
+// --------------------------------------------------------------------------
+// Weight and bias gradients: dW[co][tap][ci] = sum_p dY[p][co] X[p + tap][ci]
+// and db[co] = sum_p dY[p][co], as MFMA GEMMs with M = 16 output channels,
+// N = 16 input channels (8-channel inputs: 8 channels of two row taps) and the
+// sum over pixels as K, 32 per v_mfma_f32_16x16x32_bf16.
+//
+// The operands lie channels-last in memory and the MFMA wants 8 consecutive
+// pixels of one channel per lane, so rows are transposed on their way into
+// LDS ([channel][pixel], pairs of pixels packed into dwords) and read back as
+// 16-byte fragments.  The three column taps of a fragment are one aligned
+// read, its two neighbouring dwords and five v_alignbit; each row of X is
+// transposed once and serves three row taps.  A block takes a strip of at most
+// WG_PX columns and marches down a chunk of rows, two rows per barrier (waves
+// 0, 1 the first, 2, 3 the second; within a pair each wave takes half of the
+// input channels, or of the row taps), the next two rows of both operands
+// in flight meanwhile.  Accumulators stay in registers over all of a block's
+// chunks; the partials are summed in a fixed order (wgrad_reduce_kernel).
+//
+// Bound: the LDS reads and transposing writes around each row's barrier.  16
+// images of 257^2, layers 3 / 2 / 1: 37 / 47 / 28 us; with 2-byte gathers of both operands from global memory and
+// 16-pixel MFMAs 651 / 710 / 278 us, and 1228 us more for each layer's bias
+// gradient in a kernel of its own.  The reduction of all partials takes 9 us
+// (three launches of one serial sum per entry: 271 us each).
+// --------------------------------------------------------------------------
+constexpr int WG_PX = 96;       // columns of a strip, at most: three groups of 32
+constexpr int WG_XS = 120;      // LDS pixels per channel of X: 8 left of the strip, 16-byte rows at an odd multiple
+constexpr int WG_DS = 104;      // the same for dY (no halo)
+constexpr int WG_BLOCKS = 512;  // partials at most: two blocks per CU
+
+// floats of one partial: [co][tap][ci] of the real output channels, then the bias
+constexpr int wg_len(int cin, int cout) { return cout * 9 * cin + cout; }
+
+// how a block's work is cut: strips of `groups` 32-column groups, chunks of `rows` rows
+struct WgradGeom {
+  int groups, strips, rows, chunks, items;
+};
+inline WgradGeom wgrad_geom(int nb, int H, int W)
+{
+  WgradGeom g;
+  const int all = (W + 31) / 32;
+  g.strips = (all + WG_PX / 32 - 1) / (WG_PX / 32);
+  g.groups = (all + g.strips - 1) / g.strips;
+  // about one chunk per block, of an even number of at least 8 rows
+  const int want = std::max(1, WG_BLOCKS / std::max(1, nb * g.strips));
+  g.rows = std::max(8, ((H + want - 1) / want + 1) / 2 * 2);
+  g.chunks = (H + g.rows - 1) / g.rows;
+  g.items = nb * g.strips * g.chunks;
+  return g;
+}
+
+// CIN: channels of X (8 or 32); CD: channels of dY in memory (8 or 32), the
+// first COUT of them real
+template <int CIN, int CD, int COUT>
+__global__ __launch_bounds__(256) void wgrad_kernel(const bf16 *__restrict__ X, const bf16 *__restrict__ dY, int H,
+                                                    int W, WgradGeom g, float *__restrict__ partial)
+{
+  static_assert(CIN == 8 || CIN == 32, "input channel tiling");
+  constexpr int MT = CD == 32 ? 2 : 1;
+  constexpr int NB = CIN == 32 ? 3 : 1;  // B row sets per wave: the three row taps, or one (pair of) row tap(s)
+  constexpr int NP = WG_PX / 2 + 2;      // pixel pairs of an X row: columns -2 .. WG_PX + 1
+  constexpr int XT = 2 * NP * (CIN / 8), XI = (XT + 255) / 256;          // transposing tasks of two X rows
+  constexpr int DT = 2 * (WG_PX / 2) * (CD / 8), DI = (DT + 255) / 256;  // and of two dY rows
+  constexpr int XROW = CIN * WG_XS, DROW = CD * WG_DS;
+  __shared__ __attribute__((aligned(16))) bf16 smem[6 * XROW + 4 * DROW];
+  bf16 *sx = smem, *sd = smem + 6 * XROW;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int m = lane & 15, kg = lane >> 4;
+  const int part = wv & 1, half = wv >> 1;
+
+  f32x4 acc[NB][3][MT], bacc[MT];
+#pragma unroll
+  for (int t = 0; t < MT; t++) {
+    bacc[t] = f32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int d = 0; d < NB; d++)
+#pragma unroll
+      for (int x = 0; x < 3; x++) acc[d][x][t] = f32x4{0, 0, 0, 0};
+  }
+  bf16x8 ones;
+#pragma unroll
+  for (int i = 0; i < 8; i++) ones[i] = (short)0x3f80;  // 1.0
+
+  for (int item = blockIdx.x; item < g.items; item += gridDim.x) {
+    const int chunk = item % g.chunks, rest = item / g.chunks;
+    const int strip = rest % g.strips, img = rest / g.strips;
+    const int x0 = strip * g.groups * 32, wpx = g.groups * 32;
+    const int y0 = chunk * g.rows, y1 = min(y0 + g.rows, H);
+    const long ibase = (long)img * H * W;
+
+    // two pixels of 8 channels of rows r0 and r0 + 1, zero outside the image
+    // (X) or outside this item's pixels (dY)
+    auto load_x = [&](int q, int r0, uint4 v[2]) {
+      const int r = q / (NP * (CIN / 8)), e = q - r * (NP * (CIN / 8));
+      const int row = r0 + r, c = x0 - 2 + 2 * (e / (CIN / 8));
+      const bf16 *p = X + (ibase + (long)row * W + c) * CIN + 8 * (e % (CIN / 8));
+      const bool in = q < XT && row >= 0 && row < H;
+      v[0] = v[1] = uint4{0, 0, 0, 0};
+      if (in && c >= 0 && c < W) v[0] = *reinterpret_cast<const uint4 *>(p);
+      if (in && c + 1 >= 0 && c + 1 < W) v[1] = *reinterpret_cast<const uint4 *>(p + CIN);
+    };
+    auto load_d = [&](int q, int r0, uint4 v[2]) {
+      const int r = q / (WG_PX / 2 * (CD / 8)), e = q - r * (WG_PX / 2 * (CD / 8));
+      const int row = r0 + r, k = 2 * (e / (CD / 8)), c = x0 + k;
+      const bf16 *p = dY + (ibase + (long)row * W + c) * CD + 8 * (e % (CD / 8));
+      const bool in = q < DT && row < y1 && k < wpx;
+      v[0] = v[1] = uint4{0, 0, 0, 0};
+      if (in && c < W) v[0] = *reinterpret_cast<const uint4 *>(p);
+      if (in && c + 1 < W) v[1] = *reinterpret_cast<const uint4 *>(p + CD);
+    };
+    // dword (pixel, pixel + 1) of each of the 8 channels
+    auto store8 = [](bf16 *dst, int stride, const uint4 v[2]) {
+      const unsigned a[4] = {v[0].x, v[0].y, v[0].z, v[0].w}, b[4] = {v[1].x, v[1].y, v[1].z, v[1].w};
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        *reinterpret_cast<unsigned *>(dst + (2 * i) * stride) = (a[i] & 0xffffu) | (b[i] << 16);
+        *reinterpret_cast<unsigned *>(dst + (2 * i + 1) * stride) = (a[i] >> 16) | (b[i] & 0xffff0000u);
+      }
+    };
+    auto store_x = [&](int q, int pair, const uint4 v[2]) {  // slots 2 pair, 2 pair + 1
+      if (q >= XT) return;
+      const int r = q / (NP * (CIN / 8)), e = q - r * (NP * (CIN / 8));
+      store8(sx + (2 * pair + r) * XROW + 8 * (e % (CIN / 8)) * WG_XS + 6 + 2 * (e / (CIN / 8)), WG_XS, v);
+    };
+    auto store_d = [&](int q, int pair, const uint4 v[2]) {
+      if (q >= DT) return;
+      const int r = q / (WG_PX / 2 * (CD / 8)), e = q - r * (WG_PX / 2 * (CD / 8));
+      store8(sd + (2 * pair + r) * DROW + 8 * (e % (CD / 8)) * WG_DS + 2 * (e / (CD / 8)), WG_DS, v);
+    };
+
+    __syncthreads();  // the previous item's rows have been read
+#pragma unroll
+    for (int pr = 0; pr < 2; pr++)
+#pragma unroll
+      for (int n = 0; n < XI; n++) {
+        uint4 v[2];
+        load_x(threadIdx.x + 256 * n, y0 - 1 + 2 * pr, v);
+        store_x(threadIdx.x + 256 * n, pr, v);
+      }
+#pragma unroll
+    for (int n = 0; n < DI; n++) {
+      uint4 v[2];
+      load_d(threadIdx.x + 256 * n, y0, v);
+      store_d(threadIdx.x + 256 * n, 0, v);
+    }
+    __syncthreads();
+
+    // rows y, y + 1 of dY against rows y - 1 .. y + 2 of X: X row pairs xs, xs + 1 (mod 3)
+    int xs = 0, ds = 0;
+    for (int y = y0; y < y1; y += 2) {
+      const bool more = y + 2 < y1;
+      uint4 qx[XI][2], qd[DI][2];
+      if (more) {
+#pragma unroll
+        for (int n = 0; n < XI; n++) load_x(threadIdx.x + 256 * n, y + 3, qx[n]);
+#pragma unroll
+        for (int n = 0; n < DI; n++) load_d(threadIdx.x + 256 * n, y + 2, qd[n]);
+      }
+      const int pn = xs == 2 ? 0 : xs + 1;  // the second row pair
+      const bf16 *dr = sd + (2 * ds + half) * DROW;
+      // X rows of this wave: row tap d of output row y + half is row y - 1 + half + d
+      const bf16 *xr[NB];
+      if constexpr (CIN == 32) {
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+          const int k = half + d;
+          xr[d] = sx + (2 * (k < 2 ? xs : pn) + (k & 1)) * XROW + (part * 16 + m) * WG_XS + 8 + 8 * kg;
+        }
+      } else {  // part 0: row taps 0 (lanes m < 8) and 1; part 1: row tap 2 (twice)
+        const int k = half + (part ? 2 : m >> 3);
+        xr[0] = sx + (2 * (k < 2 ? xs : pn) + (k & 1)) * XROW + (m & 7) * WG_XS + 8 + 8 * kg;
+      }
+      for (int gr = 0; gr < g.groups; gr++) {
+        bf16x8 a[MT];
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+          a[t] = *reinterpret_cast<const bf16x8 *>(dr + (CD == 32 ? t * 16 + m : m & 7) * WG_DS + 32 * gr + 8 * kg);
+        if (part == 0) {
+#pragma unroll
+          for (int t = 0; t < MT; t++) bacc[t] = mfma32(a[t], ones, bacc[t]);
+        }
+#pragma unroll
+        for (int d = 0; d < NB; d++) {
+          const bf16 *p = xr[d] + 32 * gr;
+          const uint4 c = *reinterpret_cast<const uint4 *>(p);
+          const unsigned lo = *reinterpret_cast<const unsigned *>(p - 2);
+          const unsigned hi = *reinterpret_cast<const unsigned *>(p + 8);
+          const unsigned s1 = __builtin_amdgcn_alignbit(c.y, c.x, 16), s2 = __builtin_amdgcn_alignbit(c.z, c.y, 16),
+                         s3 = __builtin_amdgcn_alignbit(c.w, c.z, 16);
+          const uint4 b[3] = {{__builtin_amdgcn_alignbit(c.x, lo, 16), s1, s2, s3},
+                              c,
+                              {s1, s2, s3, __builtin_amdgcn_alignbit(hi, c.w, 16)}};
+#pragma unroll
+          for (int x = 0; x < 3; x++)
+#pragma unroll
+            for (int t = 0; t < MT; t++) acc[d][x][t] = mfma32(a[t], __builtin_bit_cast(bf16x8, b[x]), acc[d][x][t]);
+        }
+      }
+      if (more) {
+        const int pw = pn == 2 ? 0 : pn + 1;
+#pragma unroll
+        for (int n = 0; n < XI; n++) store_x(threadIdx.x + 256 * n, pw, qx[n]);
+#pragma unroll
+        for (int n = 0; n < DI; n++) store_d(threadIdx.x + 256 * n, ds ^ 1, qd[n]);
+      }
+      __syncthreads();
+      xs = pn;
+      ds ^= 1;
+    }
+  }
+
+  // the second row's waves hand their sums to the first's
+  constexpr int NA = NB * 3 * MT * 4 + MT * 4;
+  static_assert(NA * 64 * 2 * (int)sizeof(float) <= (int)sizeof(smem), "accumulators fit the row buffers");
+  float *sf = reinterpret_cast<float *>(smem) + part * NA * 64 + lane;
+  __syncthreads();
+  if (half) {
+    int n = 0;
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        sf[64 * n++] = bacc[t][i];
+#pragma unroll
+        for (int d = 0; d < NB; d++)
+#pragma unroll
+          for (int x = 0; x < 3; x++) sf[64 * n++] = acc[d][x][t][i];
+      }
+  }
+  __syncthreads();
+  if (half) return;
+  float *P = partial + (long)blockIdx.x * wg_len(CIN, COUT);
+  int n = 0;
+#pragma unroll
+  for (int t = 0; t < MT; t++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int co = t * 16 + 4 * kg + i;
+      const float bs = bacc[t][i] + sf[64 * n++];
+      if (part == 0 && m == 0 && co < COUT) P[COUT * 9 * CIN + co] = bs;
+#pragma unroll
+      for (int d = 0; d < NB; d++)
+#pragma unroll
+        for (int x = 0; x < 3; x++) {
+          const float v = acc[d][x][t][i] + sf[64 * n++];
+          const int dy = CIN == 32 ? d : (part ? 2 : m >> 3), ci = CIN == 32 ? part * 16 + m : m & 7;
+          if (co < COUT && (CIN == 32 || part == 0 || m < 8)) P[(co * 9 + 3 * dy + x) * CIN + ci] = v;
+        }
+    }
+}
+
+// Sums the three layers' partials in a fixed order into the flat gradient
+// ([co][ci][ky][kx] weights and biases), and the loss partials.  A block takes
+// 64 consecutive partial entries, its 16 waves every 16th partial each.
+struct WgradReduce {
+  const float *part[3];
+  float *gw[3], *gb[3];
+  int nparts[3], cin[3], cout[3], first[4];  // first: first block of each layer
+  const double *lpart;
+  int nl;
+  double lscale;
+  double *loss;
+};
+
+__global__ __launch_bounds__(1024) void wgrad_reduce_kernel(WgradReduce r)
+{
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  if ((int)blockIdx.x == r.first[3]) {  // the loss: 1024 partials at most, one per thread
+    __shared__ double sl[16];
+    double s = (int)threadIdx.x < r.nl ? r.lpart[threadIdx.x] : 0.0;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+    if (lane == 0) sl[wv] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double t = 0;
+      for (int k = 0; k < 16; k++) t += sl[k];
+      r.loss[0] = t * r.lscale;
+    }
+    return;
+  }
+  __shared__ float sh[16][64];
+  const int l = (int)blockIdx.x >= r.first[2] ? 2 : ((int)blockIdx.x >= r.first[1] ? 1 : 0);
+  const int cin = r.cin[l], cout = r.cout[l], len = wg_len(cin, cout);
+  const int e = ((int)blockIdx.x - r.first[l]) * 64 + lane;
+  float s = 0.f;
+  if (e < len) {
+    const float *p = r.part[l] + e;
+#pragma unroll 4
+    for (int k = wv; k < r.nparts[l]; k += 16) s += p[(long)k * len];
+  }
+  sh[wv][lane] = s;
+  __syncthreads();
+  if (wv || e >= len) return;
+  s = sh[0][lane];
+#pragma unroll
+  for (int k = 1; k < 16; k++) s += sh[k][lane];
+  const int nw = cout * 9 * cin;
+  if (e >= nw) {
+    r.gb[l][e - nw] = s;
+  } else {
+    const int co = e / (9 * cin), rem = e - co * 9 * cin, tap = rem / cin, ci = rem - tap * cin;
+    r.gw[l][(co * cin + ci) * 9 + tap] = s;
   }
 }
 
@@ -986,7 +1273,7 @@ struct sbp_corrector {
   float *b1 = nullptr, *b2 = nullptr, *b3 = nullptr;
   float *norm = nullptr;  // NORM_LEN floats: input shift, input scale, output scale
   bf16 *X0 = nullptr, *A1 = nullptr, *A2 = nullptr, *dY3 = nullptr, *dP2 = nullptr, *dP1 = nullptr;
-  float *Yo = nullptr, *Tg = nullptr, *dA = nullptr, *wpart = nullptr;
+  float *Yo = nullptr, *Tg = nullptr, *wpart = nullptr;
   double *lpart = nullptr, *scalars = nullptr;  // scalars: [0] loss, [1] E_old
   int *rejected = nullptr, *idx = nullptr;
   double *bpart = nullptr, *be_old = nullptr;  // batched energies: per-block partials, reference energies
@@ -1004,7 +1291,7 @@ void release(sbp_corrector *c)
   if (!c) return;
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   void *ptrs[] = {c->params, c->grads, c->m, c->v, c->w1, c->w2, c->w3, c->w2t, c->w3t, c->b1, c->b2, c->b3,
-                  c->norm, c->X0, c->A1, c->A2, c->dY3, c->dP2, c->dP1, c->Yo, c->Tg, c->dA, c->wpart,
+                  c->norm, c->X0, c->A1, c->A2, c->dY3, c->dP2, c->dP1, c->Yo, c->Tg, c->wpart,
                   c->lpart, c->scalars, c->rejected, c->idx, c->ds_raw, c->ds_tgt, c->bpart, c->be_old,
                   c->cpart, c->brej};
   for (void *p : ptrs)
@@ -1029,36 +1316,22 @@ int prepare(sbp_corrector *c)
   return SBP_OK;
 }
 
-// Persistent conv grid: at most 2048 blocks (8 per CU), each wavefront walks
-// several 16-pixel segments with its weights held in registers.
-int conv_grid(int nb, int H, int W)
-{
-  const long blocks = ((long)nb * H * ((W + 15) / 16) + 3) / 4;
-  return (int)std::min<long>(blocks, 2048);
-}
-
-// Forward of nb images already packed in X0: A1, A2 (bf16) and Yo (fp32, 3 ch).
-int forward(sbp_corrector *c, int nb)
-{
-  const int g = conv_grid(nb, c->H, c->W);
-  hipLaunchKernelGGL((conv3x3_kernel<C_INP, C_H, KP1, 0>), dim3(g), dim3(256), 0, c->stream, c->X0, nb, c->H, c->W,
-                     c->w1, c->b1, c->A1, (float *)nullptr, C_H);
-  hipLaunchKernelGGL((conv3x3_kernel<C_H, C_H, KP2, 0>), dim3(g), dim3(256), 0, c->stream, c->A1, nb, c->H, c->W,
-                     c->w2, c->b2, c->A2, (float *)nullptr, C_H);
-  hipLaunchKernelGGL((conv3x3_kernel<C_H, C_OUTP, KP3, 1>), dim3(g), dim3(256), 0, c->stream, c->A2, nb, c->H, c->W,
-                     c->w3, c->b3, (bf16 *)nullptr, c->Yo, C_OUT);
-  HIP_OR_FAIL(hipGetLastError());
-  return SBP_OK;
-}
-
 // Network output Yo of the nb packed images X0 (inference: the fused kernel).
 // T != void: also the corrected candidate's energy partials (NetEnergyArgs).
-template <typename T = void>
+template <typename T = void, bool KEEP = false>
 void launch_infer(sbp_corrector *c, int nb, hipStream_t stream, NetEnergyArgs ea = NetEnergyArgs{})
 {
   const long blocks = (long)nb * net_blocks_per_image(c->H, c->W);
-  hipLaunchKernelGGL(fused_net_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, stream, c->X0, nb, c->H, c->W,
-                     net_chunk_rows(c->H), c->w1, c->b1, c->w2, c->b2, c->w3, c->b3, c->Yo, ea);
+  hipLaunchKernelGGL((fused_net_kernel<T, KEEP>), dim3((unsigned)blocks), dim3(256), 0, stream, c->X0, nb, c->H, c->W,
+                     net_chunk_rows(c->H), c->w1, c->b1, c->w2, c->b2, c->w3, c->b3, c->Yo, c->A1, c->A2, ea);
+}
+
+// Training forward of nb images packed in X0: Yo, and the activations A1, A2.
+int forward(sbp_corrector *c, int nb)
+{
+  launch_infer<void, true>(c, nb, c->stream);
+  HIP_OR_FAIL(hipGetLastError());
+  return SBP_OK;
 }
 
 int infer(sbp_corrector *c, int nb)
@@ -1068,43 +1341,46 @@ int infer(sbp_corrector *c, int nb)
   return SBP_OK;
 }
 
+// One layer's weight and bias gradient partials; returns their number.
+template <int CIN, int CD, int COUT> int launch_wgrad(sbp_corrector *c, const bf16 *X, const bf16 *dY, int nb, float *part)
+{
+  const WgradGeom g = wgrad_geom(nb, c->H, c->W);
+  const int blocks = std::min(g.items, WG_BLOCKS);
+  hipLaunchKernelGGL((wgrad_kernel<CIN, CD, COUT>), dim3(blocks), dim3(256), 0, c->stream, X, dY, c->H, c->W, g, part);
+  return blocks;
+}
+
 // Loss against targets Tg and gradients of every parameter into c->grads.
 int backward(sbp_corrector *c, int nb)
 {
   const long npix = (long)nb * c->H * c->W;
-  const int g = conv_grid(nb, c->H, c->W);
   const int lblocks = (int)std::min<long>(grid_for(npix), 1024);
-  hipLaunchKernelGGL(loss_kernel, dim3(lblocks), dim3(256), 0, c->stream, c->Yo, c->Tg, npix, c->H, c->W, c->band,
-                     1.0 / (double)(npix * C_OUT), c->dY3, c->lpart);
-  hipLaunchKernelGGL(sum_kernel, dim3(1), dim3(64), 0, c->stream, c->lpart, lblocks, 1.0 / (double)(npix * C_OUT),
-                     c->scalars);
-  // layer 3
-  hipLaunchKernelGGL((wgrad_kernel<C_H, C_OUTP, KP3>), dim3(WG_WAVES / 4), dim3(256), 0, c->stream, c->A2, c->dY3, nb,
-                     c->H, c->W, c->wpart);
-  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(grid_for(N_W3)), dim3(256), 0, c->stream, c->wpart, WG_WAVES, C_OUT,
-                     C_H, C_H, C_OUTP, KP3, c->grads + OFF_W3);
-  hipLaunchKernelGGL(bgrad_kernel, dim3(C_OUT), dim3(256), 0, c->stream, c->dY3, npix, C_OUT, C_OUTP,
-                     c->grads + OFF_B3);
-  hipLaunchKernelGGL((conv3x3_kernel<C_OUTP, C_H, KP3T, 2>), dim3(g), dim3(256), 0, c->stream, c->dY3, nb, c->H, c->W,
-                     c->w3t, (const float *)nullptr, (bf16 *)nullptr, c->dA, C_H);
-  hipLaunchKernelGGL(relu_back_kernel, dim3(grid_for(npix * C_H)), dim3(256), 0, c->stream, c->dA, c->A2, npix * C_H,
-                     c->dP2);
-  // layer 2
-  hipLaunchKernelGGL((wgrad_kernel<C_H, C_H, KP2>), dim3(WG_WAVES / 4), dim3(256), 0, c->stream, c->A1, c->dP2, nb,
-                     c->H, c->W, c->wpart);
-  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(grid_for(N_W2)), dim3(256), 0, c->stream, c->wpart, WG_WAVES, C_H, C_H,
-                     C_H, C_H, KP2, c->grads + OFF_W2);
-  hipLaunchKernelGGL(bgrad_kernel, dim3(C_H), dim3(256), 0, c->stream, c->dP2, npix, C_H, C_H, c->grads + OFF_B2);
-  hipLaunchKernelGGL((conv3x3_kernel<C_H, C_H, KP2, 2>), dim3(g), dim3(256), 0, c->stream, c->dP2, nb, c->H, c->W,
-                     c->w2t, (const float *)nullptr, (bf16 *)nullptr, c->dA, C_H);
-  hipLaunchKernelGGL(relu_back_kernel, dim3(grid_for(npix * C_H)), dim3(256), 0, c->stream, c->dA, c->A1, npix * C_H,
-                     c->dP1);
-  // layer 1
-  hipLaunchKernelGGL((wgrad_kernel<C_INP, C_H, KP1>), dim3(WG_WAVES / 4), dim3(256), 0, c->stream, c->X0, c->dP1, nb,
-                     c->H, c->W, c->wpart);
-  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(grid_for(N_W1)), dim3(256), 0, c->stream, c->wpart, WG_WAVES, C_H,
-                     C_IN, C_INP, C_H, KP1, c->grads + OFF_W1);
-  hipLaunchKernelGGL(bgrad_kernel, dim3(C_H), dim3(256), 0, c->stream, c->dP1, npix, C_H, C_H, c->grads + OFF_B1);
+  const double inv_n = 1.0 / (double)(npix * C_OUT);
+  hipLaunchKernelGGL(loss_kernel, dim3(lblocks), dim3(256), 0, c->stream, c->Yo, c->Tg, npix, c->H, c->W, c->band, inv_n,
+                     c->dY3, c->lpart);
+  hipLaunchKernelGGL(fused_back_kernel, dim3((unsigned)(nb * net_blocks_per_image(c->H, c->W))), dim3(256), 0, c->stream,
+                     c->dY3, c->H, c->W, net_chunk_rows(c->H), c->w3t, c->w2t, c->A2, c->A1, c->dP2, c->dP1);
+  WgradReduce r{};
+  r.part[0] = c->wpart;
+  r.part[1] = r.part[0] + (long)WG_BLOCKS * wg_len(C_INP, C_H);
+  r.part[2] = r.part[1] + (long)WG_BLOCKS * wg_len(C_H, C_H);
+  r.nparts[2] = launch_wgrad<C_H, C_D3, C_OUT>(c, c->A2, c->dY3, nb, const_cast<float *>(r.part[2]));
+  r.nparts[1] = launch_wgrad<C_H, C_H, C_H>(c, c->A1, c->dP2, nb, const_cast<float *>(r.part[1]));
+  r.nparts[0] = launch_wgrad<C_INP, C_H, C_H>(c, c->X0, c->dP1, nb, const_cast<float *>(r.part[0]));
+  const int cin[3] = {C_INP, C_H, C_H}, cout[3] = {C_H, C_H, C_OUT};
+  const int ow[3] = {OFF_W1, OFF_W2, OFF_W3}, ob[3] = {OFF_B1, OFF_B2, OFF_B3};
+  for (int l = 0; l < 3; l++) {
+    r.cin[l] = cin[l];
+    r.cout[l] = cout[l];
+    r.gw[l] = c->grads + ow[l];
+    r.gb[l] = c->grads + ob[l];
+    r.first[l + 1] = r.first[l] + (wg_len(cin[l], cout[l]) + 63) / 64;
+  }
+  r.lpart = c->lpart;
+  r.nl = lblocks;
+  r.lscale = inv_n;
+  r.loss = c->scalars;
+  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(r.first[3] + 1), dim3(1024), 0, c->stream, r);
   HIP_OR_FAIL(hipGetLastError());
   return SBP_OK;
 }
@@ -1146,7 +1422,7 @@ int sbp_corr_create(int nx, int ny, int batch, sbp_corrector **out)
   if (!rc) rc = dmalloc(&c->w2, sizeof(bf16) * C_H * KP2);
   if (!rc) rc = dmalloc(&c->w3, sizeof(bf16) * C_OUTP * KP3);
   if (!rc) rc = dmalloc(&c->w2t, sizeof(bf16) * C_H * KP2);
-  if (!rc) rc = dmalloc(&c->w3t, sizeof(bf16) * C_H * KP3T);
+  if (!rc) rc = dmalloc(&c->w3t, sizeof(bf16) * C_H * KP1);
   if (!rc) rc = dmalloc(&c->b1, sizeof(float) * C_H);
   if (!rc) rc = dmalloc(&c->b2, sizeof(float) * C_H);
   if (!rc) rc = dmalloc(&c->b3, sizeof(float) * C_OUTP);
@@ -1154,13 +1430,12 @@ int sbp_corr_create(int nx, int ny, int batch, sbp_corrector **out)
   if (!rc) rc = dmalloc(&c->X0, sizeof(bf16) * npix * C_INP);
   if (!rc) rc = dmalloc(&c->A1, sizeof(bf16) * npix * C_H);
   if (!rc) rc = dmalloc(&c->A2, sizeof(bf16) * npix * C_H);
-  if (!rc) rc = dmalloc(&c->dY3, sizeof(bf16) * npix * C_OUTP);
+  if (!rc) rc = dmalloc(&c->dY3, sizeof(bf16) * npix * C_D3);
   if (!rc) rc = dmalloc(&c->dP2, sizeof(bf16) * npix * C_H);
   if (!rc) rc = dmalloc(&c->dP1, sizeof(bf16) * npix * C_H);
   if (!rc) rc = dmalloc(&c->Yo, sizeof(float) * npix * C_OUT);
   if (!rc) rc = dmalloc(&c->Tg, sizeof(float) * npix * C_OUT);
-  if (!rc) rc = dmalloc(&c->dA, sizeof(float) * npix * C_H);
-  if (!rc) rc = dmalloc(&c->wpart, sizeof(float) * WG_WAVES * C_H * KP2);
+  if (!rc) rc = dmalloc(&c->wpart, sizeof(float) * WG_BLOCKS * (wg_len(C_INP, C_H) + wg_len(C_H, C_H) + wg_len(C_H, C_OUT)));
   if (!rc) rc = dmalloc(&c->lpart, sizeof(double) * 1024);
   if (!rc) rc = dmalloc(&c->scalars, sizeof(double) * 4);
   if (!rc) rc = dmalloc(&c->rejected, sizeof(int));
