@@ -36,7 +36,6 @@ __device__ __forceinline__ StageArgs<T> batch_args(const BatchInst<T> &d)
   a.y2 = d.Y0;
   a.y3 = d.Y1;
   a.third = T(1.0 / 3.0);
-  a.aio = d.A;
   a.uout = d.U;
   a.comp = d.comp;
   a.rinv = d.rinv;

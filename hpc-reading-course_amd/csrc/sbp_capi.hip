@@ -175,10 +175,8 @@ StageArgs<T> make_args(const sbp_ctx *c, int mode, const void *yin, double dt, d
   a.y2 = static_cast<const T *>(c->Y0);
   a.y3 = static_cast<const T *>(c->Y1);
   a.third = T(1.0 / 3.0);
-  a.aio = static_cast<T *>(c->A);
   a.uout = static_cast<T *>(c->U);
   a.comp = static_cast<T *>(c->KC);
-  a.tk = static_cast<T *>(c->TK);
   a.rinv = static_cast<const T *>(c->rinv);
   a.bulk = static_cast<const T *>(c->bulk);
   a.velx = static_cast<const T *>(c->velx);
@@ -215,22 +213,51 @@ StageArgs<T> make_args(const sbp_ctx *c, int mode, const void *yin, double dt, d
   return a;
 }
 
-// Stage operand and output of stage s (1..4).
-//   2D: U -> Y0 (=Y2), Y0 -> Y1 (=Y3), Y1 -> A (=Y4), A -> U (reads Y0, Y1)
-//   1D: U -> Y0, Y0 -> Y1, Y1 -> Y0, Y0 -> U (stage vectors in A and TK)
+// Stage operand and output of stage s (1..4) of the 2D kernels:
+//   U -> Y0 (=Y2), Y0 -> Y1 (=Y3), Y1 -> A (=Y4), A -> U (reads Y0, Y1)
 void stage_io(const sbp_ctx *c, int s, const void **yin, void **yout)
 {
-  if (is1d(c->phys)) {
-    const void *in[4] = {c->U, c->Y0, c->Y1, c->Y0};
-    void *out[4] = {c->Y0, c->Y1, c->Y0, nullptr};
-    *yin = in[s - 1];
-    *yout = out[s - 1];
-  } else {
-    const void *in[4] = {c->U, c->Y0, c->Y1, c->A};
-    void *out[4] = {c->Y0, c->Y1, c->A, nullptr};
-    *yin = in[s - 1];
-    *yout = out[s - 1];
+  const void *in[4] = {c->U, c->Y0, c->Y1, c->A};
+  void *out[4] = {c->Y0, c->Y1, c->A, nullptr};
+  *yin = in[s - 1];
+  *yout = out[s - 1];
+}
+
+// Up to `steps` RK4 steps of a 1D problem in one launch (line_kernel);
+// *taken receives how many it runs.  A line of several tiles leaves the new
+// state in Y0 (its compensation in TK), which then trade places with U (KC).
+template <typename T> hipError_t launch_line_t(sbp_ctx *c, double dt, long steps, long *taken)
+{
+  const LinePlan p = line_plan(c->nx, taps_of(c->order) - c->order / 2 - 1);
+  LineArgs<T> a{};
+  a.u = static_cast<const T *>(c->U);
+  a.comp = static_cast<const T *>(c->KC);
+  a.uo = static_cast<T *>(p.grid > 1 ? c->Y0 : c->U);
+  a.co = static_cast<T *>(p.grid > 1 ? c->TK : c->KC);
+  a.velx = static_cast<const T *>(c->velx);
+  a.plane = c->plane;
+  a.xoff = c->xoff;
+  a.nx = c->nx;
+  a.tile = p.tile;
+  a.halo = p.halo;
+  a.steps = (int)std::min<long>(steps, p.steps);
+  a.hix = T(c->hix);
+  a.ax = T(c->d.ax);
+  a.c12 = T(0.5 * dt);
+  a.c3 = T(dt);
+  a.ca = T(dt / 6);
+  *taken = a.steps;
+  const hipError_t e = c->line_launch(&a, p.nt, p.grid, c->stream);
+  if (e == hipSuccess && p.grid > 1) {
+    std::swap(c->U, c->Y0);
+    if (c->KC) std::swap(c->KC, c->TK);
   }
+  return e;
+}
+
+hipError_t launch_line(sbp_ctx *c, double dt, long steps, long *taken)
+{
+  return c->esz == 8 ? launch_line_t<double>(c, dt, steps, taken) : launch_line_t<float>(c, dt, steps, taken);
 }
 
 // Launch one stage (mode 1..4 of the RK4 step, roles from stage_io) or the
@@ -338,6 +365,10 @@ hipError_t launch_pair_part(sbp_ctx *c, int part, double t, double dt)
 
 hipError_t launch_step(sbp_ctx *c, double t, double dt)
 {
+  if (is1d(c->phys)) {
+    long one;
+    return launch_line(c, dt, 1, &one);
+  }
   if (c->fused) {
     hipError_t e = launch_pair_part(c, 1, t, dt);
     if (e == hipSuccess) e = launch_pair_part(c, 3, t, dt);
@@ -417,7 +448,9 @@ int ensure_graph(sbp_ctx *c, double dt, hipGraphExec_t *out)
 int run_steps(sbp_ctx *c, double t0, double dt, long nsteps, double *t_end = nullptr)
 {
   long n = 0;
-  if (!time_dependent(c) && nsteps >= kGraphSteps) {
+  if (is1d(c->phys)) {
+    for (long k = 0; n < nsteps; n += k) HIP_OR_FAIL(launch_line(c, dt, nsteps - n, &k));
+  } else if (!time_dependent(c) && nsteps >= kGraphSteps) {
     hipGraphExec_t ge = nullptr;
     int rc = ensure_graph(c, dt, &ge);
     if (rc) return rc;
@@ -653,6 +686,15 @@ int build_ctx(const sbp_problem *desc, sbp_ctx *c)
     c->launch = reg(c->phys, c->mat, c->prec == SBP_FP32_KAHAN, kBX);
   }
   if (!c->launch) return fail(SBP_EINVAL, "no kernel for this physics/material/precision");
+  if (is1d(c->phys)) {
+    if (c->prec == SBP_FP64)
+      c->line_launch = (c->order == 2 ? line_launcher_o2_f64
+                                      : (c->order == 4 ? line_launcher_o4_f64 : line_launcher_o6_f64))(c->phys);
+    else
+      c->line_launch = (c->order == 2 ? line_launcher_o2_f32
+                                      : (c->order == 4 ? line_launcher_o4_f32 : line_launcher_o6_f32))(
+          c->phys, c->prec == SBP_FP32_KAHAN);
+  }
   if (c->phys == SBP_ACOUSTIC_2D || c->phys == SBP_ADVECTION_2D) {
     if (c->prec == SBP_FP64)
       c->pair_launch = (c->order == 2 ? pair_launcher_o2_f64
@@ -673,7 +715,7 @@ int build_ctx(const sbp_problem *desc, sbp_ctx *c)
       (rc = dalloc(&c->Y1, reg_bytes)))
     return rc;
   if (c->prec == SBP_FP32_KAHAN && (rc = dalloc(&c->KC, reg_bytes))) return rc;
-  if (is1d(c->phys) && (rc = dalloc(&c->TK, reg_bytes))) return rc;
+  if (is1d(c->phys) && c->KC && (rc = dalloc(&c->TK, reg_bytes))) return rc;
   // Zero the registers once so padding never holds stale bit patterns.
   for (void *p : {c->U, c->A, c->Y0, c->Y1, c->KC, c->TK})
     if (p) HIP_OR_FAIL(hipMemsetAsync(p, 0, reg_bytes, c->stream));
@@ -1119,7 +1161,7 @@ int sbp_time_steps(sbp_ctx *ctx, double t0, double dt, long nsteps, double *ms)
 {
   if (!ctx || !ms) return fail(SBP_EINVAL, "null argument");
   if (!ctx->have_state) return fail(SBP_ESTATE, "no state loaded");
-  if (!time_dependent(ctx) && nsteps >= kGraphSteps) {
+  if (!is1d(ctx->phys) && !time_dependent(ctx) && nsteps >= kGraphSteps) {
     hipGraphExec_t ge = nullptr;
     int rc = ensure_graph(ctx, dt, &ge);  // capture outside the timed region
     if (rc) return rc;
@@ -1142,12 +1184,15 @@ int sbp_time_stages(sbp_ctx *ctx, double dt, long nsteps, double ms_stage[4])
   double acc[4] = {0, 0, 0, 0};
   const double ts[4] = {0, 0.5 * dt, 0.5 * dt, dt};
   // one launch per stage: four timed launches; two-stage: the launches of
-  // stages 1-2 and 3-4 are timed into slots 0 and 2, slots 1 and 3 stay 0
-  const int nl = ctx->fused ? 2 : 4;
+  // stages 1-2 and 3-4 are timed into slots 0 and 2; 1D: whole steps, slot 0;
+  // the other slots stay 0
+  const int nl = is1d(ctx->phys) ? 1 : (ctx->fused ? 2 : 4);
   for (long n = 0; n < nsteps; n++) {
     HIP_OR_FAIL(hipEventRecord(ctx->ev[0], ctx->stream));
     for (int s = 0; s < nl; s++) {
-      if (ctx->fused) {
+      if (nl == 1) {
+        HIP_OR_FAIL(launch_step(ctx, n * dt, dt));
+      } else if (ctx->fused) {
         HIP_OR_FAIL(launch_pair_part(ctx, 2 * s + 1, n * dt, dt));
       } else {
         const void *yin;

@@ -14,6 +14,7 @@ struct sbp_ctx {
   size_t esz = 8;
   double hix = 0, hiy = 0;
   void *U = nullptr, *A = nullptr, *Y0 = nullptr, *Y1 = nullptr, *KC = nullptr, *TK = nullptr;
+  // (TK: 1D Kahan, the compensation of the state in Y0)
   void *rinv = nullptr, *bulk = nullptr;
   void *velx = nullptr, *vely = nullptr;  // advection velocity fields (per-point a, b)
   double *xs = nullptr, *ys = nullptr, *c3x = nullptr, *s3x = nullptr, *c4y = nullptr, *s4y = nullptr;
@@ -22,6 +23,7 @@ struct sbp_ctx {
   int npartials = 0;
   hipStream_t stream = nullptr;
   sbp::StageLaunchFn launch = nullptr;
+  sbp::LineLaunchFn line_launch = nullptr;  // 1D: whole steps
   sbp::LaunchGeom geom{};
   int ty_rows = 32, tiles_x = 0, tiles_y = 0, n_tiles = 0, n_edge = 0, n_edge_blocks = 0;
   bool have_state = false;

@@ -10,8 +10,8 @@ namespace sbp {
 template <typename T, int ORDER, bool KAHAN, int BX>
 StageLaunchFn pick_launcher(int phys, int mat)
 {
-  if (phys == PH_ADV1D) return &Launcher1D<T, ORDER, PH_ADV1D, KAHAN>::launch;
-  if (phys == PH_REFL1D) return &Launcher1D<T, ORDER, PH_REFL1D, KAHAN>::launch;
+  if (phys == PH_ADV1D) return &Launcher1D<T, ORDER, PH_ADV1D>::launch;
+  if (phys == PH_REFL1D) return &Launcher1D<T, ORDER, PH_REFL1D>::launch;
   if (phys == PH_ADV2D) {  // M_ARR: per-point velocity fields
     if (mat == M_ARR) return &Launcher2D<T, ORDER, PH_ADV2D, M_ARR, KAHAN, BX>::launch;
     return &Launcher2D<T, ORDER, PH_ADV2D, M_UNIT, KAHAN, BX>::launch;
@@ -23,6 +23,13 @@ StageLaunchFn pick_launcher(int phys, int mat)
     // tables in every precision, then rounded to T
     if (mat == M_REF) return &Launcher2D<T, ORDER, PH_ACOUSTIC, M_REF, KAHAN, BX>::launch;
   }
+  return nullptr;
+}
+
+template <typename T, int ORDER, bool KAHAN> LineLaunchFn pick_line(int phys)
+{
+  if (phys == PH_ADV1D) return &LineLauncher<T, ORDER, PH_ADV1D, KAHAN>::launch;
+  if (phys == PH_REFL1D) return &LineLauncher<T, ORDER, PH_REFL1D, KAHAN>::launch;
   return nullptr;
 }
 
@@ -57,6 +64,10 @@ PairLaunchFn pick_pair(int phys, int mat)
     if (bx == 256) return pick_launcher<double, ORDER, false, 256>(phys, mat);  \
     return nullptr;                                                             \
   }                                                                             \
+  LineLaunchFn line_launcher_o##ORDER##_f64(int phys)                           \
+  {                                                                             \
+    return pick_line<double, ORDER, false>(phys);                               \
+  }                                                                             \
   PairLaunchFn pair_launcher_o##ORDER##_f64(int phys, int mat)                  \
   {                                                                             \
     return pick_pair<double, ORDER, false>(phys, mat);                          \
@@ -70,6 +81,10 @@ PairLaunchFn pick_pair(int phys, int mat)
     if (bx != 256) return nullptr;                                              \
     return kahan ? pick_launcher<float, ORDER, true, 256>(phys, mat)            \
                  : pick_launcher<float, ORDER, false, 256>(phys, mat);          \
+  }                                                                             \
+  LineLaunchFn line_launcher_o##ORDER##_f32(int phys, bool kahan)               \
+  {                                                                             \
+    return kahan ? pick_line<float, ORDER, true>(phys) : pick_line<float, ORDER, false>(phys); \
   }                                                                             \
   PairLaunchFn pair_launcher_o##ORDER##_f32(int phys, int mat, bool kahan)      \
   {                                                                             \

@@ -17,8 +17,8 @@
 // nearby floating-point numbers is exact).  9 reads + 4 writes per value and
 // step instead of the 16 of a 3-register (U, Y, accumulator) scheme.  The
 // Kahan form compensates the final U += increment with one more register.
-// The 1D kernels keep the stage vectors and follow RK4_custom's operation
-// order exactly.  Large 2D grids run the two-stage schedule further down
+// The 1D kernel (line_kernel) runs whole steps on chip and follows
+// RK4_custom's operation order exactly.  Large 2D grids run the two-stage schedule further down
 // (pair2d_kernel: stages 1-2 and 3-4 in one launch each, the inner stage on
 // chip, 5 words per value and step) with the same arithmetic per point.
 //
@@ -58,11 +58,9 @@ template <typename T> struct StageArgs {
   const T *uin;   // U (stages 2, 3)
   const T *y2;    // Y2 (stage 4 of the 2D kernels)
   const T *y3;    // Y3 (stage 4 of the 2D kernels)
-  T *aio;         // S register of the 1D stage sequence
   T *yout;        // next Y (stages 1-3) or F (RHS mode)
   T *uout;        // U (stage 4, read and written)
   T *comp;        // Kahan compensation of U
-  T *tk;          // k2 register of the 1D stage sequence
   const T *rinv;  // rho^-1 plane (caller material arrays)
   const T *bulk;  // K plane
   const T *velx;  // advection velocity a(i,j) plane (per-point velocity), or null
@@ -216,45 +214,6 @@ __device__ __forceinline__ void rk_store(const StageArgs<T> &a, long o, const T 
         a.uout[q] = U + inc;
       } else {
         const T y = inc - in.C[c];
-        const T t = U + y;
-        a.comp[q] = (t - U) - y;
-        a.uout[q] = t;
-      }
-    }
-  }
-}
-
-// RK4 stage arithmetic of the 1D kernels in exactly RK4_custom's order
-// (time_stepping.h:127-142, rk4_util :267-269): the stage vectors are kept,
-//   stage 1: S = k1            Y = U + dt/2 k1
-//   stage 2: T = k2            Y = U + dt/2 k2
-//   stage 3: S = k1 + 2(k2+k3) Y = U + dt k3
-//   stage 4: U = U + dt/6 (S + k4)   (Kahan form: the increment is compensated)
-// The 1D problems are latency-bound, so the extra register costs nothing.
-template <typename T, int NC, int MODE, bool KAHAN>
-__device__ __forceinline__ void rk_point_exact(const StageArgs<T> &a, long o, const T *K, const T *Ucen)
-{
-#pragma unroll
-  for (int c = 0; c < NC; c++) {
-    const long q = o + c * a.plane;
-    if constexpr (MODE == MODE_RHS) {
-      a.yout[q] = K[c];
-    } else if constexpr (MODE == MODE_S1) {
-      a.aio[q] = K[c];
-      a.yout[q] = Ucen[c] + a.cy * K[c];
-    } else if constexpr (MODE == MODE_S2) {
-      a.tk[q] = K[c];
-      a.yout[q] = a.uin[q] + a.cy * K[c];
-    } else if constexpr (MODE == MODE_S3) {
-      a.aio[q] = a.aio[q] + 2 * (a.tk[q] + K[c]);
-      a.yout[q] = a.uin[q] + a.cy * K[c];
-    } else {
-      const T inc = a.ca * (a.aio[q] + K[c]);
-      const T U = a.uout[q];
-      if constexpr (!KAHAN) {
-        a.uout[q] = U + inc;
-      } else {
-        const T y = inc - a.comp[q];
         const T t = U + y;
         a.comp[q] = (t - U) - y;
         a.uout[q] = t;
@@ -1087,34 +1046,201 @@ __global__ __launch_bounds__(NT) void pair2d_kernel(StageArgs<T> eA, StageArgs<T
 // --------------------------------------------------------------------------
 // 1D problems: one thread per point, table-driven rows.
 // --------------------------------------------------------------------------
-template <typename T, int ORDER, int PHYS, int MODE, bool KAHAN>
-__global__ __launch_bounds__(256) void stage1d_kernel(StageArgs<T> a)
+// K = F at point i of a line: advection_{l,i,r} (advection_rhs.h:13-51) +
+// SAT_bc_{l,r} (:95-119) with the velocity av of this point, or
+// reflection_{l,i,r} (reflection_rhs.h:10-47) + proj_dirichlet_bc_{l,r}
+// (:108-120).  f(c, s) is component c at tap s of this point's row, whose
+// coefficients are cf (dline's sum).
+template <typename T, int ORDER, int PHYS, typename Get>
+__device__ __forceinline__ void line_rhs(const T *cf, Get f, int i, int nx, T hix, T av, const T *Uc, T *K)
 {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= a.nx) return;
-  const int nx = a.nx;
-  const long o = a.xoff + i;
-  const T *f0 = a.yin + a.xoff;
-  const T hq = a.hix * T(Ops<ORDER>::hqinv[0]);
+  constexpr int TAPS = Geom<ORDER>::TAPS;
+  auto der = [&](int c) {
+    T acc = T(0);
+#pragma unroll
+    for (int s = 0; s < TAPS; s++) acc += cf[s] * f(c, s);
+    return hix * acc;
+  };
   if constexpr (PHYS == PH_ADV1D) {
-    // advection_{l,i,r} (advection_rhs.h:13-51) + SAT_bc_{l,r} (:95-119), with
-    // the velocity a(i) of this point (per-point field, or the constant)
-    const T av = a.velx ? a.velx[o] : a.ax;
-    const T u = f0[i];
-    T k = -av * dline<T, ORDER>(f0, 1, nx, i, a.hix);
+    const T hq = hix * T(Ops<ORDER>::hqinv[0]), u = Uc[0];
+    T k = -av * der(0);
     if (i == 0) k += T(0.5) * (T(-0.5) * (av + fabs(av))) * (hq * u);
     if (i == nx - 1) k += T(0.5) * (T(0.5) * (av - fabs(av))) * (hq * u);
-    T K[1] = {k}, Uc[1] = {u};
-    rk_point_exact<T, 1, MODE, KAHAN>(a, o, K, Uc);
+    K[0] = k;
   } else {
-    // reflection_{l,i,r} (reflection_rhs.h:10-47) + proj_dirichlet_bc_{l,r} (:108-120)
-    const T *f1 = f0 + a.plane;
-    T K[2], Uc[2] = {f0[i], f1[i]};
-    K[1] = dline<T, ORDER>(f0, 1, nx, i, a.hix);
-    K[0] = dline<T, ORDER>(f1, 1, nx, i, a.hix);
+    K[1] = der(0);
+    K[0] = der(1);
     if (i == 0 || i == nx - 1) K[0] = T(0);
-    rk_point_exact<T, 2, MODE, KAHAN>(a, o, K, Uc);
   }
+}
+
+// dst = F(src) (RHS mode).
+template <typename T, int ORDER, int PHYS>
+__global__ __launch_bounds__(256) void rhs1d_kernel(StageArgs<T> a)
+{
+  using G = Geom<ORDER>;
+  constexpr int C = PHYS == PH_ADV1D ? 1 : 2;
+  const int i = blockIdx.x * 256 + threadIdx.x, nx = a.nx;
+  if (i >= nx) return;
+  const bool lo = i < G::CLS, hi = i >= nx - G::CLS;
+  const T *cf = c_edge<T, ORDER>.c[lo ? i : (hi ? G::CLS + (nx - 1 - i) : 2 * G::CLS)];
+  const int start = lo ? 0 : (hi ? nx - G::TAPS : i - G::R);
+  const T *f = a.yin + a.xoff;
+  T Uc[C], K[C];
+#pragma unroll
+  for (int c = 0; c < C; c++) Uc[c] = f[c * a.plane + i];
+  T av = a.ax;
+  if constexpr (PHYS == PH_ADV1D)
+    if (a.velx) av = a.velx[a.xoff + i];
+  line_rhs<T, ORDER, PHYS>(cf, [&](int c, int s) { return f[c * a.plane + start + s]; }, i, nx, a.hix, av, Uc, K);
+#pragma unroll
+  for (int c = 0; c < C; c++) a.yout[c * a.plane + a.xoff + i] = K[c];
+}
+
+// Whole RK4 steps of a 1D problem in one launch.  A block holds up to NT
+// consecutive points, one per thread: U, the k-sum and k2 in registers, the
+// stage operand in two LDS buffers (a stage reads one and writes the other,
+// one barrier each).  A line of at most NT points is one block that runs
+// every step asked for, in place; a longer one is cut into tiles of `tile`
+// points, each grown by `halo` = 4 steps RW points per side (RW = TAPS - R - 1:
+// every tap a table row multiplies, zero coefficients included), so the
+// points of the tile itself are exact after `steps` steps, and the new state
+// goes to other arrays.  The arithmetic is RK4_custom's, in its order
+// (time_stepping.h:127-142, rk4_util :267-269):
+//   stage 1: S = k1            Y = U + dt/2 k1
+//   stage 2: k2                Y = U + dt/2 k2
+//   stage 3: S = k1 + 2(k2+k3) Y = U + dt k3
+//   stage 4: U = U + dt/6 (S + k4)   (Kahan form: the increment is compensated)
+// Bound: the latency of one stage (LDS taps, a serial sum, a barrier).
+// One launch per stage took 7.0 us per step on 201 points (order 4 advection)
+// and 10.8 on 5001 (order 6 reflection), launch latency; this takes 0.64 and
+// 1.63.
+template <typename T> struct LineArgs {
+  const T *u, *comp;  // state read
+  T *uo, *co;         // state written (the same arrays when one block holds the line)
+  const T *velx;
+  long plane;
+  int xoff, nx, tile, halo, steps;
+  T hix, ax, c12, c3, ca;  // dt/2, dt, dt/6
+};
+
+template <typename T, int ORDER, int PHYS, bool KAHAN, int NT>
+__global__ __launch_bounds__(NT) void line_kernel(LineArgs<T> a)
+{
+  using G = Geom<ORDER>;
+  constexpr int C = PHYS == PH_ADV1D ? 1 : 2, TAPS = G::TAPS;
+  __shared__ T sy[2][C][NT];
+  const int nx = a.nx, t = threadIdx.x;
+  const int o0 = blockIdx.x * a.tile, o1 = min(o0 + a.tile, nx);          // points written
+  const int e0 = max(o0 - a.halo, 0), n = min(o1 + a.halo, nx) - e0;      // points held: n <= NT
+  const int i = e0 + min(t, n - 1);
+  const bool lo = i < G::CLS, hi = i >= nx - G::CLS;
+  const int row = lo ? i : (hi ? G::CLS + (nx - 1 - i) : 2 * G::CLS);
+  // first tap inside the block (a point whose taps leave it is not exact and
+  // not used by one that is)
+  const int start = min(max((lo ? 0 : (hi ? nx - TAPS : i - G::R)) - e0, 0), n - TAPS);
+  T cf[TAPS];
+#pragma unroll
+  for (int s = 0; s < TAPS; s++) cf[s] = c_edge<T, ORDER>.c[row][s];
+  const long o = a.xoff + i;
+  T av = a.ax;
+  if constexpr (PHYS == PH_ADV1D)
+    if (a.velx) av = a.velx[o];
+  T U[C], cmp[C], S[C], k2[C], K[C], Y[C];
+#pragma unroll
+  for (int c = 0; c < C; c++) {
+    U[c] = Y[c] = a.u[c * a.plane + o];
+    cmp[c] = T(0);
+    if constexpr (KAHAN) cmp[c] = a.comp[c * a.plane + o];
+    sy[0][c][t] = U[c];
+  }
+  __syncthreads();
+  // every tap is read before the first sum: left to itself the compiler waits
+  // for each pair of taps in turn, one LDS latency after the other (5001
+  // points, order 6: 1.63 against 2.23 us per step; with 16 waves per block
+  // the other waves cover them)
+  auto rhs = [&](int b) {
+    T v[C][TAPS];
+#pragma unroll
+    for (int c = 0; c < C; c++)
+#pragma unroll
+      for (int s = 0; s < TAPS; s++) v[c][s] = sy[b][c][start + s];
+    if constexpr (NT == 256) __builtin_amdgcn_sched_barrier(0);
+    line_rhs<T, ORDER, PHYS>(cf, [&](int c, int s) { return v[c][s]; }, i, nx, a.hix, av, Y, K);
+  };
+  for (int step = 0; step < a.steps; step++) {
+    rhs(0);
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+      S[c] = K[c];
+      sy[1][c][t] = Y[c] = U[c] + a.c12 * K[c];
+    }
+    __syncthreads();
+    rhs(1);
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+      k2[c] = K[c];
+      sy[0][c][t] = Y[c] = U[c] + a.c12 * K[c];
+    }
+    __syncthreads();
+    rhs(0);
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+      S[c] = S[c] + 2 * (k2[c] + K[c]);
+      sy[1][c][t] = Y[c] = U[c] + a.c3 * K[c];
+    }
+    __syncthreads();
+    rhs(1);
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+      const T inc = a.ca * (S[c] + K[c]);
+      if constexpr (!KAHAN) {
+        U[c] = U[c] + inc;
+      } else {
+        const T y = inc - cmp[c];
+        const T s = U[c] + y;
+        cmp[c] = (s - U[c]) - y;
+        U[c] = s;
+      }
+      sy[0][c][t] = Y[c] = U[c];
+    }
+    __syncthreads();
+  }
+  if (t >= n || i < o0 || i >= o1) return;
+#pragma unroll
+  for (int c = 0; c < C; c++) {
+    a.uo[c * a.plane + o] = U[c];
+    if constexpr (KAHAN) a.co[c * a.plane + o] = cmp[c];
+  }
+}
+
+// Threads per block and steps per launch of a line of nx points.  Few waves
+// per block keep a stage short and few points per block leave the chip empty,
+// so: 256 threads with halos of about 80 points per side while every tile has
+// a CU of its own (5001 points, order 6: 1.63 us per step; 1024 threads with
+// twice the halo 2.92, 512 threads 1.76; half the steps per launch 2.18);
+// 1024 threads beyond, where halos of 160 points still fit one block per CU
+// (100001 points: 2.93 against 4.06 us), and of 80 on longer lines, whose time
+// is the points' (10^6 points: 15.2 against 16.8 us).
+struct LinePlan {
+  int nt, tile, halo, steps, grid;
+};
+inline LinePlan line_plan(int nx, int rw)
+{
+  constexpr int kCus = 256;
+  LinePlan p{256, nx, 0, 1024, 1};
+  if (nx <= 256) return p;
+  auto set = [&](int nt, int halo) {
+    p.nt = nt;
+    p.steps = halo / (4 * rw);
+    p.halo = 4 * rw * p.steps;
+    p.tile = nt - 2 * p.halo;
+    p.grid = (nx + p.tile - 1) / p.tile;
+  };
+  set(256, 80);
+  if (p.grid > kCus) set(1024, 160);
+  if (p.grid > kCus) set(1024, 80);
+  return p;
 }
 
 // --------------------------------------------------------------------------
@@ -1303,23 +1429,28 @@ struct Launcher2D {
   }
 };
 
-template <typename T, int ORDER, int PHYS, bool KAHAN>
-struct Launcher1D {
-  template <int MODE> static hipError_t go(const StageArgs<T> &a, LaunchGeom g, hipStream_t s)
-  {
-    hipLaunchKernelGGL((stage1d_kernel<T, ORDER, PHYS, MODE, KAHAN>), dim3(g.grid), dim3(256), 0, s, a);
-    return hipGetLastError();
-  }
+// 1D: the RHS mode, and whole steps.
+template <typename T, int ORDER, int PHYS> struct Launcher1D {
   static hipError_t launch(int mode, const void *args, LaunchGeom g, hipStream_t s)
   {
-    const StageArgs<T> &a = *static_cast<const StageArgs<T> *>(args);
-    switch (mode) {
-      case MODE_RHS: return go<MODE_RHS>(a, g, s);
-      case MODE_S1: return go<MODE_S1>(a, g, s);
-      case MODE_S2: return go<MODE_S2>(a, g, s);
-      case MODE_S3: return go<MODE_S3>(a, g, s);
-      default: return go<MODE_S4>(a, g, s);
-    }
+    if (mode != MODE_RHS) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((rhs1d_kernel<T, ORDER, PHYS>), dim3(g.grid), dim3(256), 0, s,
+                       *static_cast<const StageArgs<T> *>(args));
+    return hipGetLastError();
+  }
+};
+
+using LineLaunchFn = hipError_t (*)(const void *args, int nt, int grid, hipStream_t s);
+
+template <typename T, int ORDER, int PHYS, bool KAHAN> struct LineLauncher {
+  static hipError_t launch(const void *args, int nt, int grid, hipStream_t s)
+  {
+    const LineArgs<T> &a = *static_cast<const LineArgs<T> *>(args);
+    if (nt == 256)
+      hipLaunchKernelGGL((line_kernel<T, ORDER, PHYS, KAHAN, 256>), dim3(grid), dim3(256), 0, s, a);
+    else
+      hipLaunchKernelGGL((line_kernel<T, ORDER, PHYS, KAHAN, 1024>), dim3(grid), dim3(1024), 0, s, a);
+    return hipGetLastError();
   }
 };
 
@@ -1363,6 +1494,13 @@ StageLaunchFn launcher_o6_f64(int phys, int mat, int bx);
 StageLaunchFn launcher_o2_f32(int phys, int mat, bool kahan, int bx);
 StageLaunchFn launcher_o4_f32(int phys, int mat, bool kahan, int bx);
 StageLaunchFn launcher_o6_f32(int phys, int mat, bool kahan, int bx);
+// Whole-step launchers of the 1D problems (nullptr for 2D).
+LineLaunchFn line_launcher_o2_f64(int phys);
+LineLaunchFn line_launcher_o4_f64(int phys);
+LineLaunchFn line_launcher_o6_f64(int phys);
+LineLaunchFn line_launcher_o2_f32(int phys, bool kahan);
+LineLaunchFn line_launcher_o4_f32(int phys, bool kahan);
+LineLaunchFn line_launcher_o6_f32(int phys, bool kahan);
 // Two-stage launchers of 2D acoustics (unit, array or reference materials)
 // and 2D advection (constant or per-point velocity); nullptr where none is built.
 PairLaunchFn pair_launcher_o2_f64(int phys, int mat);

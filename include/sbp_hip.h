@@ -213,7 +213,8 @@ int  sbp_time_steps(sbp_ctx *ctx, double t0, double dt, long nsteps, double *ms)
 /* Time each launch of a step separately (HIP events around every launch,
  * nsteps steps); ms_stage[4] receives the mean duration per launch: one per
  * stage, or with two-stage stepping the launches of stages 1-2 and 3-4 in
- * ms_stage[0] and ms_stage[2] (ms_stage[1] = ms_stage[3] = 0). */
+ * ms_stage[0] and ms_stage[2] (ms_stage[1] = ms_stage[3] = 0); a 1D problem
+ * runs whole steps in one launch, timed in ms_stage[0]. */
 int  sbp_time_stages(sbp_ctx *ctx, double dt, long nsteps, double ms_stage[4]);
 
 /* ---- norms ----------------------------------------------------------------
