@@ -32,9 +32,11 @@ def _run(cmd):
 
 
 def extra_flags(src):
-    # FP64 kernels: no FMA contraction, so the right-hand side rounds exactly
-    # like the reference's loops (mul then add, in the same order).
-    if src.endswith("_f64.hip"):
+    # Solver kernels: no FMA contraction.  FP64 right-hand sides round exactly
+    # like the reference's loops (mul then add, in the same order), and FP32
+    # multiply-adds are fused where the source says so (sbp_kernels.hpp mad), the
+    # same way in every kernel.
+    if src.endswith(("_f64.hip", "_f32.hip")):
         return ["-ffp-contract=off"]
     # The corrector's MFMA kernels keep their accumulators in ordinary VGPRs
     # (no AGPR copies before the bias/ReLU/bf16 epilogues); the occupancy of

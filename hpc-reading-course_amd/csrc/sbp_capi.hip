@@ -155,6 +155,17 @@ bool pair_default(const sbp_ctx *c)
   return pair_supported(c) && (long)(c->nx - 2 * D) * (c->ny - 2 * D) >= 450L * 450L;
 }
 
+// Whole steps in one launch (sbp_step.hpp) are the default where they were
+// measured faster than the schedule they replace (us per step, whole /
+// schedule): order 4 FP64 641^2 24.4 / 29.5 and with rho/K arrays 27 / 35,
+// rho = 2 + xy 43 / 48, 2D advection 14.7 / 18.5; 769^2 31.4 / 32.3.  Order 6
+// grows twelve rows and columns per patch: 257^2 13.5 / 19.9, 321^2 21.8 / 20.4.
+bool step_default(const sbp_ctx *c)
+{
+  const long most = c->order == 6 ? 300 : 700;
+  return c->step_launch && c->step_plan.ok && (long)c->nx * c->ny <= most * most;
+}
+
 int default_ty_rows(int nx, int ny, int cls)
 {
   const int wi = nx - 2 * cls, hi = ny - 2 * cls;
@@ -363,12 +374,54 @@ hipError_t launch_pair_part(sbp_ctx *c, int part, double t, double dt)
   return c->esz == 8 ? launch_pair_part_t<double>(c, part, t, dt) : launch_pair_part_t<float>(c, part, t, dt);
 }
 
+// One whole step (step2d_kernel): U -> U' in Y0, which then trade places.
+template <typename T> hipError_t launch_whole_t(sbp_ctx *c, double t, double dt)
+{
+  StepArgs<T> a{};
+  a.u = static_cast<const T *>(c->U);
+  a.uo = static_cast<T *>(c->Y0);
+  a.comp = static_cast<T *>(c->KC);
+  a.rinv = static_cast<const T *>(c->rinv);
+  a.bulk = static_cast<const T *>(c->bulk);
+  a.velx = static_cast<const T *>(c->velx);
+  a.vely = static_cast<const T *>(c->vely);
+  a.xs = c->xs;
+  a.ys = c->ys;
+  a.c3x = c->c3x;
+  a.s3x = c->s3x;
+  a.c4y = c->c4y;
+  a.s4y = c->s4y;
+  const double ts[3] = {t, t + 0.5 * dt, t + dt};
+  for (int k = 0; k < 3; k++) a.c5[k] = std::cos(5 * kPi * ts[k]);
+  a.plane = c->plane;
+  a.pitch = c->pitch;
+  a.xoff = c->xoff;
+  a.nx = c->nx;
+  a.ny = c->ny;
+  a.bc = c->bc;
+  a.hix = T(c->hix);
+  a.hiy = T(c->hiy);
+  a.ax = T(c->d.ax);
+  a.ay = T(c->d.ay);
+  a.c12 = T(0.5 * dt);
+  a.c3 = T(dt);
+  a.ca = T(dt / 6);
+  a.third = T(1.0 / 3.0);
+  a.px = c->step_plan.px;
+  a.pw = c->step_plan.pw;
+  a.ph = c->step_plan.ph;
+  const hipError_t e = c->step_launch(&a, c->step_plan.px * c->step_plan.py, c->stream);
+  if (e == hipSuccess) std::swap(c->U, c->Y0);
+  return e;
+}
+
 hipError_t launch_step(sbp_ctx *c, double t, double dt)
 {
   if (is1d(c->phys)) {
     long one;
     return launch_line(c, dt, 1, &one);
   }
+  if (c->whole) return c->esz == 8 ? launch_whole_t<double>(c, t, dt) : launch_whole_t<float>(c, t, dt);
   if (c->fused) {
     hipError_t e = launch_pair_part(c, 1, t, dt);
     if (e == hipSuccess) e = launch_pair_part(c, 3, t, dt);
@@ -706,6 +759,17 @@ int build_ctx(const sbp_problem *desc, sbp_ctx *c)
           c->phys, c->mat, c->prec == SBP_FP32_KAHAN);
   }
   c->fused = pair_default(c);
+  if (!is1d(c->phys)) {
+    if (c->prec == SBP_FP64)
+      c->step_launch = (c->order == 2 ? step_launcher_o2_f64
+                                      : (c->order == 4 ? step_launcher_o4_f64 : step_launcher_o6_f64))(c->phys, c->mat);
+    else
+      c->step_launch = (c->order == 2 ? step_launcher_o2_f32
+                                      : (c->order == 4 ? step_launcher_o4_f32 : step_launcher_o6_f32))(
+          c->phys, c->mat, c->prec == SBP_FP32_KAHAN);
+    c->step_plan = step_plan(c->order, c->nx, c->ny);
+    c->whole = step_default(c);
+  }
 
   HIP_OR_FAIL(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
   for (hipEvent_t &e : c->ev) HIP_OR_FAIL(hipEventCreate(&e));
@@ -946,6 +1010,7 @@ int sbp_set_fused(sbp_ctx *ctx, int on, int rows)
   HIP_OR_FAIL(hipStreamSynchronize(ctx->stream));
   drop_graph(ctx);
   ctx->fused = on != 0;
+  ctx->whole = false;
   ctx->p_ty_rows = rows > 0 ? rows : default_pair_rows(ctx);
   compute_pair_geometry(ctx);
   return SBP_OK;
@@ -980,15 +1045,10 @@ int sbp_tune_fused(sbp_ctx *ctx, double dt, int *rows)
   hipError_t e = hipMemcpyAsync(save_u, ctx->U, reg, hipMemcpyDeviceToDevice, ctx->stream);
   if (e == hipSuccess && ctx->KC) e = hipMemcpyAsync(save_c, ctx->KC, reg, hipMemcpyDeviceToDevice, ctx->stream);
   const int start_rows = ctx->p_ty_rows;
-  int best = start_rows;
-  float best_ms = 1e30f;
-  for (int t : cand) {
-    if (e != hipSuccess) break;
-    if (t > hi && t != cand[0]) continue;
-    drop_graph(ctx);
-    ctx->p_ty_rows = t;
-    compute_pair_geometry(ctx);
-    e = launch_step(ctx, 0.0, dt);  // warm-up
+  const bool whole = ctx->whole;
+  drop_graph(ctx);
+  auto timed = [&]() {  // three steps, after one to warm up
+    e = launch_step(ctx, 0.0, dt);
     float total = 0;
     for (int rep = 0; rep < 3 && e == hipSuccess; rep++) {
       e = hipEventRecord(ctx->ev[0], ctx->stream);
@@ -999,11 +1059,25 @@ int sbp_tune_fused(sbp_ctx *ctx, double dt, int *rows)
       if (e == hipSuccess) e = hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1]);
       total += ms;
     }
+    return total;
+  };
+  // whole steps stay unless a two-stage tile height beats them
+  const float whole_ms = whole && e == hipSuccess ? timed() : 1e30f;
+  ctx->whole = false;
+  int best = start_rows;
+  float best_ms = 1e30f;
+  for (int t : cand) {
+    if (e != hipSuccess) break;
+    if (t > hi && t != cand[0]) continue;
+    ctx->p_ty_rows = t;
+    compute_pair_geometry(ctx);
+    const float total = timed();
     if (e == hipSuccess && total < best_ms) {
       best_ms = total;
       best = t;
     }
   }
+  ctx->whole = whole && (e != hipSuccess || whole_ms <= best_ms);
   if (e == hipSuccess) e = hipMemcpyAsync(ctx->U, save_u, reg, hipMemcpyDeviceToDevice, ctx->stream);
   if (e == hipSuccess && ctx->KC) e = hipMemcpyAsync(ctx->KC, save_c, reg, hipMemcpyDeviceToDevice, ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
@@ -1184,9 +1258,9 @@ int sbp_time_stages(sbp_ctx *ctx, double dt, long nsteps, double ms_stage[4])
   double acc[4] = {0, 0, 0, 0};
   const double ts[4] = {0, 0.5 * dt, 0.5 * dt, dt};
   // one launch per stage: four timed launches; two-stage: the launches of
-  // stages 1-2 and 3-4 are timed into slots 0 and 2; 1D: whole steps, slot 0;
+  // stages 1-2 and 3-4 are timed into slots 0 and 2; whole steps into slot 0;
   // the other slots stay 0
-  const int nl = is1d(ctx->phys) ? 1 : (ctx->fused ? 2 : 4);
+  const int nl = is1d(ctx->phys) || ctx->whole ? 1 : (ctx->fused ? 2 : 4);
   for (long n = 0; n < nsteps; n++) {
     HIP_OR_FAIL(hipEventRecord(ctx->ev[0], ctx->stream));
     for (int s = 0; s < nl; s++) {

@@ -5,6 +5,7 @@
 
 #include "../../include/sbp_hip.h"
 #include "sbp_kernels.hpp"
+#include "sbp_step.hpp"
 
 struct sbp_ctx {
   sbp_problem d{};
@@ -31,6 +32,11 @@ struct sbp_ctx {
   // launcher, D = CLS + R deep frame, tile geometry of the pair tiles.
   sbp::PairLaunchFn pair_launch = nullptr;
   bool fused = false;
+  // Whole steps in one launch (sbp_step.hpp), in place of either schedule
+  // while nobody has chosen one with sbp_set_fused.
+  sbp::StepLaunchFn step_launch = nullptr;
+  sbp::StepPlan step_plan{};
+  bool whole = false;
   int store_policy = 0;  // two-stage tile stores: 0 by streamed size, 1 cached, 2 nontemporal
   int p_depth = 0, p_ty_rows = 0, p_tiles_x = 0, p_n_tiles = 0, p_n_edge = 0, p_n_edge_blocks = 0;
   // Captured multi-step graphs, keyed by dt and by the array holding U when

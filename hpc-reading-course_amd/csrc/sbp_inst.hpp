@@ -4,6 +4,7 @@
 // built without FMA contraction).
 #pragma once
 #include "sbp_kernels.hpp"
+#include "sbp_step.hpp"
 
 namespace sbp {
 
@@ -30,6 +31,19 @@ template <typename T, int ORDER, bool KAHAN> LineLaunchFn pick_line(int phys)
 {
   if (phys == PH_ADV1D) return &LineLauncher<T, ORDER, PH_ADV1D, KAHAN>::launch;
   if (phys == PH_REFL1D) return &LineLauncher<T, ORDER, PH_REFL1D, KAHAN>::launch;
+  return nullptr;
+}
+
+template <typename T, int ORDER, bool KAHAN> StepLaunchFn pick_step(int phys, int mat)
+{
+  if (phys == PH_ACOUSTIC) {
+    if (mat == M_UNIT) return &StepLauncher<T, ORDER, PH_ACOUSTIC, M_UNIT, KAHAN>::launch;
+    if (mat == M_ARR) return &StepLauncher<T, ORDER, PH_ACOUSTIC, M_ARR, KAHAN>::launch;
+    if (mat == M_REF) return &StepLauncher<T, ORDER, PH_ACOUSTIC, M_REF, KAHAN>::launch;
+  }
+  if (phys == PH_ADV2D)
+    return mat == M_ARR ? &StepLauncher<T, ORDER, PH_ADV2D, M_ARR, KAHAN>::launch
+                        : &StepLauncher<T, ORDER, PH_ADV2D, M_UNIT, KAHAN>::launch;
   return nullptr;
 }
 
@@ -68,6 +82,10 @@ PairLaunchFn pick_pair(int phys, int mat)
   {                                                                             \
     return pick_line<double, ORDER, false>(phys);                               \
   }                                                                             \
+  StepLaunchFn step_launcher_o##ORDER##_f64(int phys, int mat)                  \
+  {                                                                             \
+    return pick_step<double, ORDER, false>(phys, mat);                          \
+  }                                                                             \
   PairLaunchFn pair_launcher_o##ORDER##_f64(int phys, int mat)                  \
   {                                                                             \
     return pick_pair<double, ORDER, false>(phys, mat);                          \
@@ -85,6 +103,10 @@ PairLaunchFn pick_pair(int phys, int mat)
   LineLaunchFn line_launcher_o##ORDER##_f32(int phys, bool kahan)               \
   {                                                                             \
     return kahan ? pick_line<float, ORDER, true>(phys) : pick_line<float, ORDER, false>(phys); \
+  }                                                                             \
+  StepLaunchFn step_launcher_o##ORDER##_f32(int phys, int mat, bool kahan)      \
+  {                                                                             \
+    return kahan ? pick_step<float, ORDER, true>(phys, mat) : pick_step<float, ORDER, false>(phys, mat); \
   }                                                                             \
   PairLaunchFn pair_launcher_o##ORDER##_f32(int phys, int mat, bool kahan)      \
   {                                                                             \

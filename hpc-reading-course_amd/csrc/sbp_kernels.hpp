@@ -81,6 +81,14 @@ template <typename T> struct StageArgs {
 
 template <typename T, int ORDER> __constant__ EdgeTable<T, ORDER> c_edge = make_edge_table<T, ORDER>();
 
+// a * b + c: one rounding in FP32, two in FP64.  Every unit is compiled without
+// contraction and multiply-adds are written with this, so the FP64 kernels
+// round like the reference's loops and every kernel (one launch per stage, two
+// stages, whole steps, ensembles) forms the same FP32 values from the same
+// operands, whatever the compiler makes of the code around them.
+__device__ __forceinline__ double mad(double a, double b, double c) { return a * b + c; }
+__device__ __forceinline__ float mad(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
 // Table-driven derivative at index idx of a strided line of n points.
 template <typename T, int ORDER>
 __device__ __forceinline__ T dline(const T *__restrict__ f, long stride, int n, int idx, T hi)
@@ -92,9 +100,9 @@ __device__ __forceinline__ T dline(const T *__restrict__ f, long stride, int n, 
   const int row = lo ? idx : (hi_side ? G::CLS + (n - 1 - idx) : 2 * G::CLS);
   const int start = lo ? 0 : (hi_side ? n - G::TAPS : idx - G::R);
   const T *c = c_edge<T, ORDER>.c[row];
-  T acc = T(0);
+  T acc = c[0] * f[(long)start * stride];
 #pragma unroll
-  for (int s = 0; s < G::TAPS; s++) acc += c[s] * f[(long)(start + s) * stride];
+  for (int s = 1; s < G::TAPS; s++) acc = mad(c[s], f[(long)(start + s) * stride], acc);
   return hi * acc;
 }
 
@@ -103,10 +111,10 @@ template <typename T, int ORDER, typename Get>
 __device__ __forceinline__ T dint(Get get, T hi)
 {
   using O = Ops<ORDER>;
-  T acc = T(0);
+  T acc = T(O::inner[0]) * get(0);
 #pragma unroll
-  for (int s = 0; s < 2 * O::R + 1; s++)
-    if (O::inner[s] != 0.0) acc += T(O::inner[s]) * get(s);
+  for (int s = 1; s < 2 * O::R + 1; s++)
+    if (O::inner[s] != 0.0) acc = mad(T(O::inner[s]), get(s), acc);
   return hi * acc;
 }
 
@@ -121,8 +129,8 @@ __device__ __forceinline__ void acoustic_F(T dxp, T dyp, T dxu, T dyv, T ri, T K
     Fv = -dyp;
     Fp = -dxu - dyv;
   } else if constexpr (MAT == M_REF) {
-    Fu = -ri * dxp + fu;
-    Fv = -ri * dyp + fv;
+    Fu = mad(-ri, dxp, fu);
+    Fv = mad(-ri, dyp, fv);
     Fp = -dxu - dyv;
   } else {
     Fu = -ri * dxp;
@@ -161,7 +169,7 @@ __device__ __forceinline__ void ref_material_at(double x, double c3x, double s3x
 template <typename T, bool KAHAN>
 __device__ __forceinline__ T stage4_increment(const StageArgs<T> &a, T U, T Y2, T Y3, T Y4, T K)
 {
-  return ((Y2 - U) + 2 * (Y3 - U) + (Y4 - U)) * a.third + a.ca * K;
+  return mad((Y2 - U) + 2 * (Y3 - U) + (Y4 - U), a.third, a.ca * K);
 }
 
 // Pointwise operands of the RK4 update at one edge point: U (stages 2-4), Y2,
@@ -204,9 +212,9 @@ __device__ __forceinline__ void rk_store(const StageArgs<T> &a, long o, const T 
     if constexpr (MODE == MODE_RHS) {
       a.yout[q] = K[c];
     } else if constexpr (MODE == MODE_S1) {
-      a.yout[q] = Ycen[c] + a.cy * K[c];
+      a.yout[q] = mad(a.cy, K[c], Ycen[c]);
     } else if constexpr (MODE == MODE_S2 || MODE == MODE_S3) {
-      a.yout[q] = in.U[c] + a.cy * K[c];
+      a.yout[q] = mad(a.cy, K[c], in.U[c]);
     } else {
       const T U = in.U[c];
       const T inc = stage4_increment<T, KAHAN>(a, U, in.Y2[c], in.Y3[c], Ycen[c], K[c]);
@@ -291,7 +299,7 @@ __device__ __forceinline__ void edge_rhs(const StageArgs<T> &a, const T *f, long
     const T dx = dline<T, ORDER>(f + rowb, 1, nx, i, a.hix);
     const T dy = dline<T, ORDER>(f + colb, fpitch, ny, j, a.hiy);
     Uc[0] = u;
-    T k = -(ax * dx + ay * dy);
+    T k = -mad(ax, dx, ay * dy);
     if (i == 0) k += T(0.5) * (T(-0.5) * (ax + fabs(ax))) * (hqx * u);
     if (j == 0) k += T(0.5) * (T(-0.5) * (ay + fabs(ay))) * (hqy * u);
     if (i == nx - 1) k += T(0.5) * (T(0.5) * (ax - fabs(ax))) * (hqx * u);
@@ -501,7 +509,7 @@ __device__ __forceinline__ void interior_tile(const StageArgs<T> &a, int tile)
       Uc[2] = win[0][R];
     } else {
       const T ax = LD_M ? cur.ri : a.ax, ay = LD_M ? cur.K : a.ay;
-      K[0] = -(ax * d0x + ay * d0y);
+      K[0] = -mad(ax, d0x, ay * d0y);
       Uc[0] = win[0][R];
     }
 
@@ -514,9 +522,9 @@ __device__ __forceinline__ void interior_tile(const StageArgs<T> &a, int tile)
         if constexpr (MODE == MODE_RHS) {
           stg<NS>(a.yout + qo, K[c]);
         } else if constexpr (MODE == MODE_S1) {
-          stg<NS>(a.yout + qo, Uc[c] + a.cy * K[c]);
+          stg<NS>(a.yout + qo, mad(a.cy, K[c], Uc[c]));
         } else if constexpr (MODE == MODE_S2 || MODE == MODE_S3) {
-          stg<NS>(a.yout + qo, cur.U[c] + a.cy * K[c]);
+          stg<NS>(a.yout + qo, mad(a.cy, K[c], cur.U[c]));
         } else {
           const T inc = stage4_increment<T, KAHAN>(a, cur.U[c], cur.Y2[c], cur.Y3[c], Uc[c], K[c]);
           if constexpr (!KAHAN) {
@@ -788,13 +796,13 @@ __device__ __forceinline__ void pair_tile_rw(const PairArgs<T> &a, int tile)
         } else {
           const T dy = dint<T, ORDER>([&](int s) { return win[0][s]; }, a.hiy);
           const T ax = LD_M ? ri : a.ax, ay = LD_M ? Kb : a.ay;
-          F[0] = -(ax * fdx[0][0] + ay * dy);
+          F[0] = -mad(ax, fdx[0][0], ay * dy);
         }
 #pragma unroll
         for (int c = 0; c < NC; c++) {
 #pragma unroll
           for (int s = 0; s < WN - 1; s++) wmid[c][s] = wmid[c][s + 1];
-          wmid[c][WN - 1] = Um[c] + a.c1 * F[c];
+          wmid[c][WN - 1] = mad(a.c1, F[c], Um[c]);
         }
         s_mu[t] = wmid[0][WN - 1];
         if constexpr (AC) s_mp[t] = wmid[2][WN - 1];
@@ -858,12 +866,12 @@ __device__ __forceinline__ void pair_tile_rw(const PairArgs<T> &a, int tile)
           acoustic_F<T, MAT>(gdx[1][0], dyp, gdx[0][0], dyv, fri[0], fK[0], fu, fv, F[0], F[1], F[2]);
         } else {
           const T dy = dint<T, ORDER>([&](int s) { return wmid[0][s]; }, a.hiy);
-          F[0] = -(axo * gdx[0][0] + ayo * dy);
+          F[0] = -mad(axo, gdx[0][0], ayo * dy);
         }
         const long qo = (long)o * pitch + a.xoff + mc;
         if constexpr (PAIR == 1) {
 #pragma unroll
-          for (int c = 0; c < NC; c++) put(a.o2 + c * plane + qo, win[c][0] + a.c2 * F[c]);
+          for (int c = 0; c < NC; c++) put(a.o2 + c * plane + qo, mad(a.c2, F[c], win[c][0]));
         } else {
           // K1 = F(U) at the output row and Y2 = U + dt/2 K1, as pair 1 formed them
           T F1[NC];
@@ -873,14 +881,14 @@ __device__ __forceinline__ void pair_tile_rw(const PairArgs<T> &a, int tile)
             acoustic_F<T, MAT>(hdx[1][0], dyp1, hdx[0][0], dyv1, fri[0], fK[0], fu1, fv1, F1[0], F1[1], F1[2]);
           } else {
             const T dy1 = dint<T, ORDER>([&](int s) { return fU[s][0]; }, a.hiy);
-            F1[0] = -(axo * hdx[0][0] + ayo * dy1);
+            F1[0] = -mad(axo, hdx[0][0], ayo * dy1);
           }
 #pragma unroll
           for (int c = 0; c < NC; c++) {
             const T U = fU[R][c];
-            const T Y2 = U + a.c0 * F1[c];
+            const T Y2 = mad(a.c0, F1[c], U);
             const T Y4 = wmid[c][R];
-            const T inc = ((Y2 - U) + 2 * (win[c][0] - U) + (Y4 - U)) * a.third + a.c2 * F[c];
+            const T inc = mad((Y2 - U) + 2 * (win[c][0] - U) + (Y4 - U), a.third, a.c2 * F[c]);
             if constexpr (!KAHAN) {
               put(a.o1 + c * plane + qo, U + inc);
             } else {
@@ -987,7 +995,7 @@ __device__ __forceinline__ void frame_patch_pair(const StageArgs<T> &eA, const S
     const bool on = ii >= f.i0 && ii < f.i1 && jj >= f.j0 && jj < f.j1;
 #pragma unroll
     for (int c = 0; c < NC; c++) {
-      const T y = (MA == MODE_S1 ? Uc[c] : rin.U[c]) + eA.cy * K[c];
+      const T y = mad(eA.cy, K[c], MA == MODE_S1 ? Uc[c] : rin.U[c]);
       s_f[c][q] = y;
       if (PAIR == 1 && on) eA.yout[o + c * plane] = y;  // Y2 on the frame (stage 4 reads it)
     }
@@ -1056,9 +1064,9 @@ __device__ __forceinline__ void line_rhs(const T *cf, Get f, int i, int nx, T hi
 {
   constexpr int TAPS = Geom<ORDER>::TAPS;
   auto der = [&](int c) {
-    T acc = T(0);
+    T acc = cf[0] * f(c, 0);
 #pragma unroll
-    for (int s = 0; s < TAPS; s++) acc += cf[s] * f(c, s);
+    for (int s = 1; s < TAPS; s++) acc = mad(cf[s], f(c, s), acc);
     return hix * acc;
   };
   if constexpr (PHYS == PH_ADV1D) {
@@ -1173,21 +1181,21 @@ __global__ __launch_bounds__(NT) void line_kernel(LineArgs<T> a)
 #pragma unroll
     for (int c = 0; c < C; c++) {
       S[c] = K[c];
-      sy[1][c][t] = Y[c] = U[c] + a.c12 * K[c];
+      sy[1][c][t] = Y[c] = mad(a.c12, K[c], U[c]);
     }
     __syncthreads();
     rhs(1);
 #pragma unroll
     for (int c = 0; c < C; c++) {
       k2[c] = K[c];
-      sy[0][c][t] = Y[c] = U[c] + a.c12 * K[c];
+      sy[0][c][t] = Y[c] = mad(a.c12, K[c], U[c]);
     }
     __syncthreads();
     rhs(0);
 #pragma unroll
     for (int c = 0; c < C; c++) {
       S[c] = S[c] + 2 * (k2[c] + K[c]);
-      sy[1][c][t] = Y[c] = U[c] + a.c3 * K[c];
+      sy[1][c][t] = Y[c] = mad(a.c3, K[c], U[c]);
     }
     __syncthreads();
     rhs(1);
@@ -1501,6 +1509,14 @@ LineLaunchFn line_launcher_o6_f64(int phys);
 LineLaunchFn line_launcher_o2_f32(int phys, bool kahan);
 LineLaunchFn line_launcher_o4_f32(int phys, bool kahan);
 LineLaunchFn line_launcher_o6_f32(int phys, bool kahan);
+// Whole-step launchers of the 2D problems (sbp_step.hpp; nullptr for 1D).
+using StepLaunchFn = hipError_t (*)(const void *args, int grid, hipStream_t s);
+StepLaunchFn step_launcher_o2_f64(int phys, int mat);
+StepLaunchFn step_launcher_o4_f64(int phys, int mat);
+StepLaunchFn step_launcher_o6_f64(int phys, int mat);
+StepLaunchFn step_launcher_o2_f32(int phys, int mat, bool kahan);
+StepLaunchFn step_launcher_o4_f32(int phys, int mat, bool kahan);
+StepLaunchFn step_launcher_o6_f32(int phys, int mat, bool kahan);
 // Two-stage launchers of 2D acoustics (unit, array or reference materials)
 // and 2D advection (constant or per-point velocity); nullptr where none is built.
 PairLaunchFn pair_launcher_o2_f64(int phys, int mat);

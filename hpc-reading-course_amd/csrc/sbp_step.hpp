@@ -1,0 +1,321 @@
+// sbp_step.hpp -- a whole RK4 step of a 2D problem in one launch, in LDS.
+//
+// A block computes the four stages of one patch of the grid: it loads U on the
+// patch grown by what four stages of stencils reach (closure rows read the
+// first TAPS points of their line, interior rows R points to either side) and
+// evaluates each stage on what the following ones still need.  The region's
+// rows are dealt to the waves in turn, one lane per column, so a point's U,
+// its running sum (Y2-U) + 2(Y3-U) + (Y4-U) and its materials stay in
+// registers, only the stage operand passes through LDS (two buffers, one
+// barrier per stage), and whether a row is a closure row is one decision per
+// wave.  The arithmetic per point is that of the one-stage kernels, term for
+// term, so FP64 results are the same to the bit; U' goes to another array
+// (neighbouring patches read U), whose role the host trades with U's.
+#pragma once
+#include <type_traits>
+
+#include "sbp_kernels.hpp"
+
+namespace sbp {
+
+constexpr int kStepLanes = 64;  // columns of a loaded region, at most
+constexpr int kStepWaves = 8;
+// rows of a loaded region, at most: kStepWaves * step_rows(order)
+constexpr int step_rows(int order) { return order == 6 ? 4 : 3; }
+
+template <typename T> struct StepArgs {
+  const T *u;
+  T *uo, *comp;  // U'; Kahan compensation (read and written at the patch's own points)
+  const T *rinv, *bulk;  // acoustics: rho^-1, K planes (M_ARR)
+  const T *velx, *vely;  // 2D advection: velocity planes (M_ARR)
+  const double *xs, *ys, *c3x, *s3x, *c4y, *s4y;  // rho = 2 + xy and its forcing (M_REF)
+  double c5[3];          // cos(5 pi t) at the times of stage 1, stages 2 and 3, stage 4
+  long plane;
+  int pitch, xoff, nx, ny, bc;
+  T hix, hiy, ax, ay;
+  T c12, c3, ca, third;  // dt/2, dt, dt/6, 1/3
+  int px, pw, ph;        // patches per row, their width and height
+};
+
+// The points the stencils of [lo, hi) read along a line of n points.
+template <int ORDER> __host__ __device__ inline void stencil_reach(int &lo, int &hi, int n)
+{
+  using G = Geom<ORDER>;
+  const bool l = lo < G::CLS, h = hi > n - G::CLS;
+  const int a = l ? 0 : lo - G::R, b = h ? n : hi + G::R;
+  lo = h && n - G::TAPS < a ? n - G::TAPS : a;
+  hi = l && G::TAPS > b ? G::TAPS : b;
+}
+
+template <typename T, int ORDER, int PHYS, int MAT, bool KAHAN>
+__global__ __launch_bounds__(64 * kStepWaves) void step2d_kernel(StepArgs<T> a)
+{
+  using G = Geom<ORDER>;
+  constexpr int R = G::R, CLS = G::CLS, TAPS = G::TAPS, KR = step_rows(ORDER), H = kStepWaves * KR;
+  constexpr bool AC = PHYS == PH_ACOUSTIC;
+  constexpr int C = AC ? 3 : 1;
+  constexpr int FS = H * kStepLanes, BS = C * FS;  // strides of a field and of a buffer
+  __shared__ T s_[2 * BS + 2 * R];
+  T *const s = s_ + R;  // a lane's x taps may reach R slots outside its row: garbage that no used value depends on
+
+  const int nx = a.nx, ny = a.ny;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i0 = (blockIdx.x % a.px) * a.pw, i1 = min(i0 + a.pw, nx);
+  const int j0 = (blockIdx.x / a.px) * a.ph, j1 = min(j0 + a.ph, ny);
+  // regions evaluated in stages 1 .. 4 ([4]: the patch), and loaded ([0])
+  int xl[5], xh[5], yl[5], yh[5];
+  xl[4] = i0, xh[4] = i1, yl[4] = j0, yh[4] = j1;
+#pragma unroll
+  for (int k = 3; k >= 0; k--) {
+    xl[k] = xl[k + 1], xh[k] = xh[k + 1], yl[k] = yl[k + 1], yh[k] = yh[k + 1];
+    stencil_reach<ORDER>(xl[k], xh[k], nx);
+    stencil_reach<ORDER>(yl[k], yh[k], ny);
+  }
+  const bool xedge = xl[1] < CLS || xh[1] > nx - CLS;  // closure columns among the region's
+  const bool yedge = yl[1] < CLS || yh[1] > ny - CLS;
+
+  const int i = min(xl[0] + lane, xh[0] - 1);
+  const long col = a.xoff + i;
+  // x taps of this lane: closure columns read a table row from their end of
+  // the line; interior ones the interior row, whose padding taps re-read the
+  // centre (a point that is certainly valid) with coefficient zero
+  T cf[TAPS];
+  int xt = lane - R, xpad = lane;
+  if (xedge) {
+    const bool lo = i < CLS, hi = i >= nx - CLS;
+    const int row = lo ? i : (hi ? CLS + (nx - 1 - i) : 2 * CLS);
+#pragma unroll
+    for (int t = 0; t < TAPS; t++) cf[t] = c_edge<T, ORDER>.c[row][t];
+    if (lo || hi) {
+      xt = min(max((lo ? 0 : nx - TAPS) - xl[0], 0), kStepLanes - TAPS);
+      xpad = -1;
+    }
+  }
+
+  T U[KR][C], P[KR][C], Y[KR][C], ri[KR], Kb[KR], cmp[KR][C];
+  double xc = 0, c3c = 0, s3c = 0;
+  if constexpr (MAT == M_REF) {
+    xc = a.xs[i];
+    c3c = a.c3x[i];
+    s3c = a.s3x[i];
+  }
+#pragma unroll
+  for (int k = 0; k < KR; k++) {
+    const int j = min(yl[0] + wv + kStepWaves * k, yh[0] - 1);
+    const long o = (long)j * a.pitch + col;
+#pragma unroll
+    for (int c = 0; c < C; c++) U[k][c] = a.u[c * a.plane + o];
+    ri[k] = Kb[k] = T(1);
+    if constexpr (MAT == M_ARR) {
+      ri[k] = (AC ? a.rinv : a.velx)[o];
+      Kb[k] = (AC ? a.bulk : a.vely)[o];
+    }
+    if constexpr (KAHAN) {
+#pragma unroll
+      for (int c = 0; c < C; c++) cmp[k][c] = a.comp[c * a.plane + o];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < KR; k++)
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+      Y[k][c] = U[k][c];
+      P[k][c] = T(0);
+      s[c * FS + (wv + kStepWaves * k) * kStepLanes + lane] = U[k][c];
+    }
+  __syncthreads();
+
+  // Right-hand side at row j = region row r of buffer b, centre values Yc.
+  auto rhs = [&](auto XE, int b, int r, int j, const T *Yc, T rik, T Kk, double c5, T *K) {
+    constexpr bool xe = decltype(XE)::value;
+    constexpr int NX = xe ? TAPS : 2 * R + 1;
+    const T *f = s + b * BS, *fp = AC ? f + 2 * FS : f;
+    const T *fx = f + r * kStepLanes, *px = fp + r * kStepLanes;
+    const bool yc = yedge && (j < CLS || j >= ny - CLS);  // closure row
+    const int ry = yc ? (j < CLS ? 0 : ny - TAPS) - yl[0] : r - R;
+    const T *py = fp + ry * kStepLanes + lane, *vy = f + FS + ry * kStepLanes + lane;
+    T ax[NX], bx[NX], ay[TAPS], by[TAPS];  // p (or the one field) and u in x; p and v in y
+#pragma unroll
+    for (int t = 0; t < NX; t++) {
+      const int q = xe ? (t < 2 * R + 1 || xpad < 0 ? xt + t : xpad) : lane - R + t;
+      ax[t] = px[q];
+      if constexpr (AC) bx[t] = fx[q];
+    }
+#pragma unroll
+    for (int t = 0; t < 2 * R + 1; t++) {
+      ay[t] = py[t * kStepLanes];
+      if constexpr (AC) by[t] = vy[t * kStepLanes];
+    }
+    if (yc) {
+#pragma unroll
+      for (int t = 2 * R + 1; t < TAPS; t++) {
+        ay[t] = py[t * kStepLanes];
+        if constexpr (AC) by[t] = vy[t * kStepLanes];
+      }
+    }
+    auto ddx = [&](const T *v) {
+      if constexpr (xe) {
+        T acc = cf[0] * v[0];
+#pragma unroll
+        for (int t = 1; t < TAPS; t++) acc = mad(cf[t], v[t], acc);
+        return a.hix * acc;
+      } else {
+        return dint<T, ORDER>([&](int t) { return v[t]; }, a.hix);
+      }
+    };
+    auto ddy = [&](const T *v) {
+      if (yc) {
+        const T *cy = c_edge<T, ORDER>.c[j < CLS ? j : CLS + (ny - 1 - j)];
+        T acc = cy[0] * v[0];
+#pragma unroll
+        for (int t = 1; t < TAPS; t++) acc = mad(cy[t], v[t], acc);
+        return a.hiy * acc;
+      }
+      return dint<T, ORDER>([&](int t) { return v[t]; }, a.hiy);
+    };
+    if constexpr (AC) {
+      const T dxp = ddx(ax), dyp = ddy(ay), dxu = ddx(bx), dyv = ddy(by);
+      T fu = T(0), fv = T(0);
+      if constexpr (MAT == M_REF) ref_material_at<T>(xc, c3c, s3c, a.ys, a.c4y, a.s4y, j, c5, rik, fu, fv);
+      acoustic_F<T, MAT>(dxp, dyp, dxu, dyv, rik, Kk, fu, fv, K[0], K[1], K[2]);
+      if (xe || yc) {  // boundary terms, as in edge_rhs
+        const T qinv0 = T(Ops<ORDER>::hqinv[0]);
+        const T hqx = a.hix * qinv0, hqy = a.hiy * qinv0;
+        const int bc = a.bc == B_DEFAULT ? B_FSREF : a.bc;
+        const T u = Yc[0], v = Yc[1], p = Yc[2];
+        if (bc == B_FSREF) {
+          if (i == 0) K[0] -= hqx * p;
+          if (j == 0) K[1] -= hqy * p;
+          if (i == nx - 1) K[0] += hqx * p;
+          if (j == ny - 1) K[1] += hqy * p;
+        } else if (bc == B_FS) {
+          if (i == 0) K[0] -= rik * (hqx * p);
+          if (j == 0) K[1] -= rik * (hqy * p);
+          if (i == nx - 1) K[0] += rik * (hqx * p);
+          if (j == ny - 1) K[1] += rik * (hqy * p);
+        } else {
+          if (i == 0) K[2] -= Kk * (hqx * u);
+          if (j == 0) K[2] -= Kk * (hqy * v);
+          if (i == nx - 1) K[2] += Kk * (hqx * u);
+          if (j == ny - 1) K[2] += Kk * (hqy * v);
+        }
+      }
+    } else {
+      const T va = MAT == M_ARR ? rik : a.ax, vb = MAT == M_ARR ? Kk : a.ay;
+      T k = -mad(va, ddx(ax), vb * ddy(ay));
+      if (xe || yc) {
+        const T qinv0 = T(Ops<ORDER>::hqinv[0]);
+        const T hqx = a.hix * qinv0, hqy = a.hiy * qinv0, u = Yc[0];
+        if (i == 0) k += T(0.5) * (T(-0.5) * (va + fabs(va))) * (hqx * u);
+        if (j == 0) k += T(0.5) * (T(-0.5) * (vb + fabs(vb))) * (hqy * u);
+        if (i == nx - 1) k += T(0.5) * (T(0.5) * (va - fabs(va))) * (hqx * u);
+        if (j == ny - 1) k += T(0.5) * (T(0.5) * (vb - fabs(vb))) * (hqy * u);
+      }
+      K[0] = k;
+    }
+  };
+
+  // (unrolled: fewer registers, so two blocks per CU; 513^2 18.9 against 27 us)
+  auto stages = [&](auto XE) {
+    const int y1l = yl[1], y1h = yh[1], y2l = yl[2], y2h = yh[2], y3l = yl[3], y3h = yh[3];
+#pragma unroll
+    for (int st = 1; st <= 4; st++) {
+      const int b = (st - 1) & 1;
+      const double c5 = st == 1 ? a.c5[0] : (st == 4 ? a.c5[2] : a.c5[1]);
+      const T cy = st == 3 ? a.c3 : a.c12, w = st == 2 ? T(2) : T(1);
+      const int ylo = st == 1 ? y1l : (st == 2 ? y2l : (st == 3 ? y3l : j0));
+      const int yhi = st == 1 ? y1h : (st == 2 ? y2h : (st == 3 ? y3h : j1));
+#pragma unroll
+      for (int k = 0; k < KR; k++) {
+        const int r = wv + kStepWaves * k, j = yl[0] + r;
+        if (j < ylo || j >= yhi) continue;  // (the whole wave)
+        T K[C];
+        rhs(XE, b, r, j, Y[k], ri[k], Kb[k], c5, K);
+        if (st < 4) {
+#pragma unroll
+          for (int c = 0; c < C; c++) {
+            const T y = mad(cy, K[c], U[k][c]);
+            P[k][c] = P[k][c] + w * (y - U[k][c]);  // exact products: Y2-U, + 2 (Y3-U), + (Y4-U)
+            Y[k][c] = y;
+            s[(b ^ 1) * BS + c * FS + r * kStepLanes + lane] = y;
+          }
+        } else if (xl[0] + lane >= i0 && xl[0] + lane < i1) {
+          const long o = (long)j * a.pitch + col;
+#pragma unroll
+          for (int c = 0; c < C; c++) {
+            const T inc = mad(P[k][c], a.third, a.ca * K[c]);
+            if constexpr (!KAHAN) {
+              a.uo[c * a.plane + o] = U[k][c] + inc;
+            } else {
+              const T y = inc - cmp[k][c];
+              const T t = U[k][c] + y;
+              a.comp[c * a.plane + o] = (t - U[k][c]) - y;
+              a.uo[c * a.plane + o] = t;
+            }
+          }
+        }
+      }
+      __syncthreads();
+    }
+  };
+  if (xedge) stages(std::true_type{});
+  else stages(std::false_type{});
+}
+
+// The cut of an nx x ny grid into patches; ok: every region fits a block.
+// Patches are as low as gives each a CU of its own, since a block's time is
+// its rows' (101^2, order 4: 7.4 us per step at 2 rows, 9.0 at 8), and as high
+// as the rows of a block allow on grids that fill the chip anyway (513^2: 18.9
+// us at 8 rows, 22.5 at 4).
+struct StepPlan {
+  bool ok;
+  int px, pw, py, ph;
+};
+template <int ORDER> inline StepPlan step_plan_t(int nx, int ny)
+{
+  constexpr int rows = kStepWaves * step_rows(ORDER);
+  // parts of `len` points of a line of n whose four-stage regions hold at most `most`
+  auto fits = [](int n, int len, int most) {
+    for (int p = 0; p < n; p += len) {
+      int lo = p, hi = p + len < n ? p + len : n;
+      for (int k = 0; k < 4; k++) stencil_reach<ORDER>(lo, hi, n);
+      if (hi - lo > most) return false;
+    }
+    return true;
+  };
+  StepPlan p{};
+  p.px = (nx + kStepLanes - 1) / kStepLanes;
+  for (;; p.px++) {
+    p.pw = (nx + p.px - 1) / p.px;
+    if (p.pw < 1 || fits(nx, p.pw, kStepLanes)) break;
+    if (p.pw == 1) return p;
+  }
+  p.px = (nx + p.pw - 1) / p.pw;
+  constexpr int kCus = 256;
+  int best = 0;
+  for (p.ph = 1; p.ph <= 8; p.ph++) {
+    if (!fits(ny, p.ph, rows)) continue;
+    best = p.ph;
+    if ((long)p.px * ((ny + p.ph - 1) / p.ph) <= kCus) break;
+  }
+  if (!best) return p;
+  p.ph = best;
+  p.py = (ny + p.ph - 1) / p.ph;
+  p.ok = true;
+  return p;
+}
+inline StepPlan step_plan(int order, int nx, int ny)
+{
+  return order == 2 ? step_plan_t<2>(nx, ny) : (order == 4 ? step_plan_t<4>(nx, ny) : step_plan_t<6>(nx, ny));
+}
+
+template <typename T, int ORDER, int PHYS, int MAT, bool KAHAN> struct StepLauncher {
+  static hipError_t launch(const void *args, int grid, hipStream_t s)
+  {
+    hipLaunchKernelGGL((step2d_kernel<T, ORDER, PHYS, MAT, KAHAN>), dim3(grid), dim3(64 * kStepWaves), 0, s,
+                       *static_cast<const StepArgs<T> *>(args));
+    return hipGetLastError();
+  }
+};
+
+}  // namespace sbp

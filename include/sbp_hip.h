@@ -117,12 +117,15 @@ int  sbp_set_tile_rows(sbp_ctx *ctx, int rows);
  * measured faster).  rows: tile height of the two-stage tiles
  * (0 = chosen from the grid).  A performance knob with no reference
  * counterpart: it changes how ts_rk4's steps are scheduled on the device
- * (ts_rk.cpp:54-65), not what they compute. */
+ * (ts_rk.cpp:54-65), not what they compute.  Until this is called a context
+ * runs whole steps in one launch where that was measured faster than the
+ * schedule sbp_get_fused reports; the call chooses one of the two schedules. */
 int  sbp_set_fused(sbp_ctx *ctx, int on, int rows);
 int  sbp_get_fused(const sbp_ctx *ctx);
 /* Time the two-stage schedule's candidate tile heights (8 .. 136 rows) on
  * this grid for step dt and keep the fastest; *rows (optional) receives it
- * (0 when the context runs one launch per stage).  The resident state is
+ * (0 when sbp_get_fused is 0).  A context that runs whole steps keeps doing so
+ * unless that tile height is faster.  The resident state is
  * saved and restored, so tuning leaves it untouched; a tuning knob with no
  * reference counterpart, results do not depend on it. */
 int  sbp_tune_fused(sbp_ctx *ctx, double dt, int *rows);
@@ -213,8 +216,8 @@ int  sbp_time_steps(sbp_ctx *ctx, double t0, double dt, long nsteps, double *ms)
 /* Time each launch of a step separately (HIP events around every launch,
  * nsteps steps); ms_stage[4] receives the mean duration per launch: one per
  * stage, or with two-stage stepping the launches of stages 1-2 and 3-4 in
- * ms_stage[0] and ms_stage[2] (ms_stage[1] = ms_stage[3] = 0); a 1D problem
- * runs whole steps in one launch, timed in ms_stage[0]. */
+ * ms_stage[0] and ms_stage[2] (ms_stage[1] = ms_stage[3] = 0); whole steps in
+ * one launch (1D problems, and 2D ones that run them) in ms_stage[0]. */
 int  sbp_time_stages(sbp_ctx *ctx, double dt, long nsteps, double ms_stage[4]);
 
 /* ---- norms ----------------------------------------------------------------
