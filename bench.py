@@ -4,13 +4,13 @@
 Default workload (the throughput target of the path): 2D first-order acoustics
 [u,v,p] on the unit square, 4097 x 4097 points, order-4 SBP, wall SATs,
 rho = c = 1, seeded Gaussian pressure pulse, CFL 0.25, FP64.  A step is one
-classical RK4 step (four fused stage kernels) over the whole grid with the
-state resident in HBM.
+classical RK4 step over the whole grid with the state resident in HBM (by
+default one march2d_kernel launch that reads U and writes U').
 
 Prints one JSON line:
   value       DOF-updates/s (nx*ny*3 values advanced one RK4 step per update)
   roofline    HBM roofline of the dominant kernel: the step's longest launch
-              (at 4097^2 the pair2d_kernel launch of RK4 stages 3-4), its
+              (at 4097^2 the whole step's march2d_kernel), its
               algorithmic bytes per launch (each value it must read or write
               once: launch_bytes) over its mean duration (HIP events on the
               library's stream), against the 8 TB/s peak; `traffic` is the
@@ -37,14 +37,12 @@ sys.path.insert(0, ROOT)
 
 PEAK_HBM_GBS = 8000.0
 # HBM bytes per launch of the dominant kernel of the default workload (4097^2,
-# order 4, rho = K = 1, FP64, two-stage schedule: the pair2d_kernel launch of
-# RK4 stages 3-4), from rocprofv3 as FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0 KiB
-# (the factors that turn the counters of a 1 GiB plain copy in the same runs
-# into the bytes it reads and writes), with the commit and the tile height it
-# was measured at: profiles/pair2d_acoustic_4097sq_order4_fp64_hbm_counters.md.
-MEASURED_TRAFFIC = {(4097, 4, 0, "two-stage", 3): (491316 * 2.0 + 404713 * 1.0) * 1024}
-MEASURED_AT = "84c602f"
-MEASURED_TILE_ROWS = 40
+# order 4, rho = K = 1, FP64: march2d_kernel), from rocprofv3 as FETCH_SIZE x
+# 2.0 + WRITE_SIZE x 1.0 KiB (the factors that turn the counters of a 1 GiB
+# plain copy in the same runs into the bytes it reads and writes):
+# profiles/march2d_acoustic_4097sq_order4_fp64_hbm_counters.md.
+MEASURED_TRAFFIC = {}
+MEASURED_AT = None
 
 
 def pkg(sub):
@@ -68,9 +66,20 @@ def bytes_per_dof(precision, materials=False, C=3):
     return (words + extra) * w
 
 
-def launch_bytes(spec, fused):
+WHOLE, TWO, ONE = "whole step", "two-stage", "one stage per launch"
+
+
+def schedule_of(fused, stage_ms):
+    """A context's schedule: a whole step is timed into the first slot alone."""
+    if stage_ms[0] > 0 and not np.any(np.asarray(stage_ms[1:]) > 0):
+        return WHOLE
+    return TWO if fused else ONE
+
+
+def launch_bytes(spec, schedule):
     """Algorithmic HBM bytes of each of a step's four stage slots: every value
     a launch must read or write, once.  Per DOF (point and component), words:
+      whole step (slot 1): U -> U' (2; Kahan + compensation R/W 2)
       one stage per launch: U -> Y2 (2), Y2, U -> Y3 (3), Y3, U -> Y4 (3),
                             Y4, U, Y2, Y3 -> U (5; Kahan + compensation R/W 2)
       two-stage (two launches; slots 2 and 4 are empty):
@@ -79,14 +88,17 @@ def launch_bytes(spec, fused):
                   launch 3  interior Y3, U -> U' (3; Kahan +2; Y2 is
                             recomputed); frame Y3, U, Y2 -> U' (4; Kahan +2)
     Stored rho^-1 and K add 2 words per point to every launch that differentiates
-    with them (two-stage: per interior or frame point a launch covers)."""
+    with them (two-stage: per interior or frame point a launch covers; whole
+    step: once)."""
     w = 8 if spec.precision == 0 else 4
     kahan = spec.precision == 2
     mat = spec.material == 2
     C = spec.components
     order = spec.order
     npts = spec.nx * spec.ny
-    if not fused:
+    if schedule == WHOLE:
+        return [float(npts * (C * (4 if kahan else 2) + (2 if mat else 0)) * w), 0.0, 0.0, 0.0]
+    if schedule == ONE:
         words = [2, 3, 3, 5 + (2 if kahan else 0)]
         return [float(npts * (C * k + (2 if mat else 0)) * w) for k in words]
     cls, r = {2: 1, 4: 4, 6: 6}[order], order // 2
@@ -100,14 +112,16 @@ def launch_bytes(spec, fused):
     return [float(b1 * w), 0.0, float(b3 * w), 0.0]
 
 
-def launch_planes(spec, fused, slot):
+def launch_planes(spec, schedule, slot):
     """(planes read, planes written) per interior point of the launch in stage
     slot `slot` (1-4), one plane being one component or material array: the
     byte mix launch_bytes counts, for the flat streaming ceiling."""
     kahan = spec.precision == 2
     m = 2 if spec.material == 2 else 0
     C = spec.components
-    if fused:
+    if schedule == WHOLE:
+        return C * (2 if kahan else 1) + m, C * (2 if kahan else 1)
+    if schedule == TWO:
         if slot == 1:
             return C + m, C
         return (3 if kahan else 2) * C + m, (2 if kahan else 1) * C
@@ -152,7 +166,8 @@ def measure(spec, v0, dt, steps, warmup, fused=None):
     bpd = bytes_per_dof(spec.precision, mat, spec.components)
     step_kernel_s = float(np.sum(stage_ms)) * 1e-3
     achieved = dofs * bpd / step_kernel_s / 1e9
-    lb = launch_bytes(spec, fused)
+    schedule = schedule_of(fused, stage_ms)
+    lb = launch_bytes(spec, schedule)
     k_achieved = sum(lb) / step_kernel_s / 1e9
     dom = int(np.argmax(stage_ms))
     dom_gbs = lb[dom] / (float(stage_ms[dom]) * 1e-3) / 1e9
@@ -162,7 +177,7 @@ def measure(spec, v0, dt, steps, warmup, fused=None):
         bytes_per_dof=bpd, achieved_gbs=achieved, frac=achieved / PEAK_HBM_GBS, energy=energy,
         kernel_bytes_per_dof=sum(lb) / dofs, kernel_achieved_gbs=k_achieved, kernel_frac=k_achieved / PEAK_HBM_GBS,
         launch_bytes=lb, dominant_launch=dom + 1, dominant_gbs=dom_gbs, dominant_frac=dom_gbs / PEAK_HBM_GBS,
-        schedule="two-stage" if fused else "one stage per launch", tile_rows=rows)
+        schedule=schedule, tile_rows=rows if schedule == TWO else None)
 
 
 def batched(count=256, steps=500, warmup=10, prec=1):
@@ -189,7 +204,7 @@ def batched(count=256, steps=500, warmup=10, prec=1):
     dofs = sum(sp.nx * sp.ny * 3 for sp in specs)
     bpd = bytes_per_dof(prec, materials=True)
     achieved = dofs * bpd * steps / (ev_ms * 1e-3) / 1e9
-    kbpd = sum(sum(launch_bytes(sp, cfg.get("two_stage", False))) for sp in specs) / dofs
+    kbpd = sum(sum(launch_bytes(sp, TWO if cfg.get("two_stage", False) else ONE)) for sp in specs) / dofs
     return {"instances": count, "dofs": dofs, "steps": steps, "precision": ["fp64", "fp32", "fp32_kahan"][prec],
             "dof_updates_per_s": dofs * steps / wall, "ms_per_step": wall / steps * 1e3,
             "event_ms_per_step": ev_ms / steps, "bytes_per_dof": bpd, "achieved_gbs": achieved,
@@ -220,13 +235,14 @@ def reflection_2d(steps=2000, warmup=0):
             fused = ctx.fused
         dofs = spec.nx * spec.ny * 3
         bpd = bytes_per_dof(prec, True)
-        lb = launch_bytes(spec, fused)
+        schedule = schedule_of(fused, stage_ms)
+        lb = launch_bytes(spec, schedule)
         kbpd = sum(lb) / dofs
         step_s = float(np.sum(stage_ms)) * 1e-3
         # the dominant launch against the flat stream of its own byte mix
         dom = int(np.argmax(stage_ms))
         dom_gbs = lb[dom] / (float(stage_ms[dom]) * 1e-3) / 1e9
-        nr, nw = launch_planes(spec, fused, dom + 1)
+        nr, nw = launch_planes(spec, schedule, dom + 1)
         stream_gbs = capi.stream_bandwidth(spec.nx * spec.ny * (8 if prec == 0 else 4), nr, nw, 3)
         out[name] = {"dof_updates_per_s": dofs * steps / wall, "ms_per_step": wall / steps * 1e3,
                      "bytes_per_dof": bpd, "frac": dofs * bpd / step_s / 1e9 / PEAK_HBM_GBS,
@@ -235,7 +251,7 @@ def reflection_2d(steps=2000, warmup=0):
                      "dominant_frac": dom_gbs / PEAK_HBM_GBS,
                      "stream_ceiling": {"planes_read": nr, "planes_written": nw, "gbs": stream_gbs,
                                         "frac": dom_gbs / stream_gbs},
-                     "schedule": "two-stage" if fused else "one stage per launch"}
+                     "schedule": schedule}
         del v0
     ref = finals["fp64"]
     scale = float(np.max(np.abs(ref)))
@@ -392,12 +408,14 @@ def main():
     dom = main_m["dominant_launch"]
     # the dominant launch's byte mix in a flat elementwise kernel (no stencil,
     # halo or tiles): the rate those bytes reach as a plain stream
-    nr, nw = launch_planes(spec, main_m["schedule"] == "two-stage", dom)
+    nr, nw = launch_planes(spec, main_m["schedule"], dom)
     plane_bytes = spec.nx * spec.ny * (8 if spec.precision == 0 else 4)
     stream_gbs = capi.stream_bandwidth(plane_bytes, nr, nw, 5)
     log("flat stream, %d planes read + %d written: %.0f GB/s" % (nr, nw, stream_gbs))
     traffic = MEASURED_TRAFFIC.get((spec.nx, spec.order, spec.precision, main_m["schedule"], dom))
-    if main_m["schedule"] == "two-stage":
+    if main_m["schedule"] == WHOLE:
+        names = {1: "march2d_kernel, a whole RK4 step (strips and frame patches)"}
+    elif main_m["schedule"] == TWO:
         names = {1: "pair2d_kernel, RK4 stages 1-2 (interior tiles and frame patches)", 2: "(no launch)",
                  3: "pair2d_kernel, RK4 stages 3-4 (interior tiles and frame patches)", 4: "(no launch)"}
     else:
@@ -428,7 +446,7 @@ def main():
                      "traffic_unit": "HBM bytes per launch of that kernel (rocprofv3 FETCH_SIZE x 2.0 + "
                                      "WRITE_SIZE x 1.0 KiB, copy-calibrated)",
                      "traffic_measured_at": MEASURED_AT,
-                     "traffic_tile_rows": MEASURED_TILE_ROWS, "tile_rows": main_m.get("tile_rows"),
+                     "tile_rows": main_m.get("tile_rows"),
                      "launch_bytes": main_m["launch_bytes"], "stage_ms": main_m["stage_ms"],
                      "step": {"bytes": sum(main_m["launch_bytes"]), "bytes_per_dof": main_m["kernel_bytes_per_dof"],
                               "kernel_ms": float(np.sum(main_m["stage_ms"])),
@@ -436,7 +454,7 @@ def main():
                      "rate_16word_basis": {"bytes_per_dof": main_m["bytes_per_dof"],
                                            "achieved": main_m["achieved_gbs"], "frac_of_peak": main_m["frac"],
                                            "note": "3-register RK4 with one launch per stage (16 words); "
-                                                   "the two-stage schedule needs fewer bytes, so this rate "
+                                                   "other schedules need fewer bytes, so this rate "
                                                    "is not bounded by the peak"},
                      "copy_ceiling_gbs": copy_gbs,
                      "stream_ceiling": {"planes_read": nr, "planes_written": nw, "plane_bytes": plane_bytes,

@@ -166,6 +166,21 @@ bool step_default(const sbp_ctx *c)
   return c->step_launch && c->step_plan.ok && (long)c->nx * c->ny <= most * most;
 }
 
+// Marched steps (sbp_march.hpp) replace both from the sizes where their lead-in
+// and frame cost less than the passes they save (us per step, march / before):
+// order 4 FP64 301^2 12.8 / 11.5, 401^2 13.2 / 15.4, 1025^2 30.8 / 47.5, 4097^2
+// 251 / 452; FP32 401^2 10.1 / 9.7, 513^2 11.9 / 14.2, 4097^2 121 / 236; order 2
+// FP64 201^2 6.3 / 5.8, 257^2 6.5 / 7.3; order 6 FP64 301^2 21.9 / 20.1, 513^2
+// 30.3 / 36.7, FP32 301^2 15.2 / 17.2.  Ribbons leave most of a strip's columns
+// or rows to the lead-in: 64 x 4096 31.7 / 16.1, 2048 x 128 19.1 / 17.8, 128 x
+// 2048 22.8 / 20.6, 2000 x 200 22.1 / 23.4; longer ones are still better
+// marched (64 x 60000 201 / 338, 60000 x 64 87 / 176).
+bool march_default(const sbp_ctx *c)
+{
+  const long least = std::min(c->nx, c->ny) <= 128 ? 700 : (c->order == 2 ? 260 : 380);
+  return c->march_plan.ok && (long)c->nx * c->ny >= least * least;
+}
+
 int default_ty_rows(int nx, int ny, int cls)
 {
   const int wi = nx - 2 * cls, hi = ny - 2 * cls;
@@ -374,7 +389,8 @@ hipError_t launch_pair_part(sbp_ctx *c, int part, double t, double dt)
   return c->esz == 8 ? launch_pair_part_t<double>(c, part, t, dt) : launch_pair_part_t<float>(c, part, t, dt);
 }
 
-// One whole step (step2d_kernel): U -> U' in Y0, which then trade places.
+// One whole step (march2d_kernel or step2d_kernel): U -> U' in Y0, which then
+// trade places.
 template <typename T> hipError_t launch_whole_t(sbp_ctx *c, double t, double dt)
 {
   StepArgs<T> a{};
@@ -410,7 +426,11 @@ template <typename T> hipError_t launch_whole_t(sbp_ctx *c, double t, double dt)
   a.px = c->step_plan.px;
   a.pw = c->step_plan.pw;
   a.ph = c->step_plan.ph;
-  const hipError_t e = c->step_launch(&a, c->step_plan.px * c->step_plan.py, c->stream);
+  a.strips = c->march_plan.strips;
+  a.segs = c->march_plan.segs;
+  a.seg_rows = c->march_plan.seg_rows;
+  const hipError_t e = c->march ? c->march_fns.launch(&a, c->stream)
+                                : c->step_launch(&a, c->step_plan.px * c->step_plan.py, c->stream);
   if (e == hipSuccess) std::swap(c->U, c->Y0);
   return e;
 }
@@ -769,6 +789,20 @@ int build_ctx(const sbp_problem *desc, sbp_ctx *c)
           c->phys, c->mat, c->prec == SBP_FP32_KAHAN);
     c->step_plan = step_plan(c->order, c->nx, c->ny);
     c->whole = step_default(c);
+    if (c->prec == SBP_FP64)
+      c->march_fns = (c->order == 2 ? march_launcher_o2_f64
+                                    : (c->order == 4 ? march_launcher_o4_f64 : march_launcher_o6_f64))(c->phys, c->mat);
+    else
+      c->march_fns = (c->order == 2 ? march_launcher_o2_f32
+                                    : (c->order == 4 ? march_launcher_o4_f32 : march_launcher_o6_f32))(
+          c->phys, c->mat, c->prec == SBP_FP32_KAHAN);
+    if (c->march_fns.launch) {
+      int resident = 0;
+      HIP_OR_FAIL(c->march_fns.resident(&resident));
+      if (c->step_plan.ok) c->march_plan = march_plan(c->order, c->nx, c->ny, c->step_plan.px, resident);
+      c->march = march_default(c);
+      c->whole = c->whole || c->march;
+    }
   }
 
   HIP_OR_FAIL(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));

@@ -37,6 +37,10 @@ struct sbp_ctx {
   sbp::StepLaunchFn step_launch = nullptr;
   sbp::StepPlan step_plan{};
   bool whole = false;
+  // whole steps march along the grid (sbp_march.hpp)
+  sbp::MarchFns march_fns{};
+  sbp::MarchPlan march_plan{};
+  bool march = false;
   int store_policy = 0;  // two-stage tile stores: 0 by streamed size, 1 cached, 2 nontemporal
   int p_depth = 0, p_ty_rows = 0, p_tiles_x = 0, p_n_tiles = 0, p_n_edge = 0, p_n_edge_blocks = 0;
   // Captured multi-step graphs, keyed by dt and by the array holding U when

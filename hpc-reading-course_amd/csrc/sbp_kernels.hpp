@@ -1517,6 +1517,18 @@ StepLaunchFn step_launcher_o6_f64(int phys, int mat);
 StepLaunchFn step_launcher_o2_f32(int phys, int mat, bool kahan);
 StepLaunchFn step_launcher_o4_f32(int phys, int mat, bool kahan);
 StepLaunchFn step_launcher_o6_f32(int phys, int mat, bool kahan);
+// Marched whole steps (sbp_march.hpp; null where none is built): launch, and the
+// blocks a CU holds.
+struct MarchFns {
+  hipError_t (*launch)(const void *args, hipStream_t s);
+  hipError_t (*resident)(int *blocks);
+};
+MarchFns march_launcher_o2_f64(int phys, int mat);
+MarchFns march_launcher_o4_f64(int phys, int mat);
+MarchFns march_launcher_o6_f64(int phys, int mat);
+MarchFns march_launcher_o2_f32(int phys, int mat, bool kahan);
+MarchFns march_launcher_o4_f32(int phys, int mat, bool kahan);
+MarchFns march_launcher_o6_f32(int phys, int mat, bool kahan);
 // Two-stage launchers of 2D acoustics (unit, array or reference materials)
 // and 2D advection (constant or per-point velocity); nullptr where none is built.
 PairLaunchFn pair_launcher_o2_f64(int phys, int mat);

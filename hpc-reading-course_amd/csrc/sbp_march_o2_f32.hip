@@ -1,0 +1,8 @@
+// FP32 and FP32+Kahan marched whole steps of the order-2 SBP operators.
+#include "sbp_march.hpp"
+namespace sbp {
+MarchFns march_launcher_o2_f32(int phys, int mat, bool kahan)
+{
+  return kahan ? pick_march<float, 2, true>(phys, mat) : pick_march<float, 2, false>(phys, mat);
+}
+}  // namespace sbp

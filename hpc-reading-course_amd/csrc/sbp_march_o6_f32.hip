@@ -1,0 +1,8 @@
+// FP32 and FP32+Kahan marched whole steps of the order-6 SBP operators.
+#include "sbp_march.hpp"
+namespace sbp {
+MarchFns march_launcher_o6_f32(int phys, int mat, bool kahan)
+{
+  return kahan ? pick_march<float, 6, true>(phys, mat) : pick_march<float, 6, false>(phys, mat);
+}
+}  // namespace sbp

@@ -1,0 +1,5 @@
+// FP64 marched whole steps of the order-6 SBP operators (built without FMA contraction).
+#include "sbp_march.hpp"
+namespace sbp {
+MarchFns march_launcher_o6_f64(int phys, int mat) { return pick_march<double, 6, false>(phys, mat); }
+}  // namespace sbp

@@ -23,6 +23,9 @@ constexpr int kStepWaves = 8;
 // rows of a loaded region, at most: kStepWaves * step_rows(order)
 constexpr int step_rows(int order) { return order == 6 ? 4 : 3; }
 
+// values of a patch's LDS array: two buffers of every component, and R slots at either end
+constexpr int step_lds(int order, int comps, int rows) { return 2 * comps * rows * kStepLanes + order; }
+
 template <typename T> struct StepArgs {
   const T *u;
   T *uo, *comp;  // U'; Kahan compensation (read and written at the patch's own points)
@@ -35,6 +38,7 @@ template <typename T> struct StepArgs {
   T hix, hiy, ax, ay;
   T c12, c3, ca, third;  // dt/2, dt, dt/6, 1/3
   int px, pw, ph;        // patches per row, their width and height
+  int strips, segs, seg_rows;  // marched strips (sbp_march.hpp): columns, segments of rows, rows of a segment
 };
 
 // The points the stencils of [lo, hi) read along a line of n points.
@@ -47,21 +51,25 @@ template <int ORDER> __host__ __device__ inline void stencil_reach(int &lo, int 
   hi = l && G::TAPS > b ? G::TAPS : b;
 }
 
-template <typename T, int ORDER, int PHYS, int MAT, bool KAHAN>
-__global__ __launch_bounds__(64 * kStepWaves) void step2d_kernel(StepArgs<T> a)
+// The step on columns [i0, i1) and rows [j0, j1), by a block of NW waves
+// whose patches load at most H rows.  TR: "columns" and "rows" are the grid's rows and columns (a narrow
+// strip along the left or right boundary fills the lanes that way; it must
+// not reach the closure rows at the lanes' ends).
+template <typename T, int ORDER, int PHYS, int MAT, bool KAHAN, bool TR, int NW, int H>
+__device__ __forceinline__ void step_patch(const StepArgs<T> &a, T *s_, int i0, int i1, int j0, int j1)
 {
   using G = Geom<ORDER>;
-  constexpr int R = G::R, CLS = G::CLS, TAPS = G::TAPS, KR = step_rows(ORDER), H = kStepWaves * KR;
+  constexpr int R = G::R, CLS = G::CLS, TAPS = G::TAPS, KR = H / NW;
   constexpr bool AC = PHYS == PH_ACOUSTIC;
   constexpr int C = AC ? 3 : 1;
-  constexpr int FS = H * kStepLanes, BS = C * FS;  // strides of a field and of a buffer
-  __shared__ T s_[2 * BS + 2 * R];
+  constexpr int FS = H * kStepLanes, BS = C * FS;  // strides of a field and of a buffer of the LDS array s_
+  static_assert(H % NW == 0 && 2 * BS + 2 * R == step_lds(ORDER, C, H), "rows and LDS of a patch");
   T *const s = s_ + R;  // a lane's x taps may reach R slots outside its row: garbage that no used value depends on
 
-  const int nx = a.nx, ny = a.ny;
+  static_assert(!TR || MAT != M_REF, "the forcing's tables are per grid column");
+  const int nx = TR ? a.ny : a.nx, ny = TR ? a.nx : a.ny;
+  const T hl = TR ? a.hiy : a.hix, hr = TR ? a.hix : a.hiy;  // of the lane and row axes
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int i0 = (blockIdx.x % a.px) * a.pw, i1 = min(i0 + a.pw, nx);
-  const int j0 = (blockIdx.x / a.px) * a.ph, j1 = min(j0 + a.ph, ny);
   // regions evaluated in stages 1 .. 4 ([4]: the patch), and loaded ([0])
   int xl[5], xh[5], yl[5], yh[5];
   xl[4] = i0, xh[4] = i1, yl[4] = j0, yh[4] = j1;
@@ -75,7 +83,8 @@ __global__ __launch_bounds__(64 * kStepWaves) void step2d_kernel(StepArgs<T> a)
   const bool yedge = yl[1] < CLS || yh[1] > ny - CLS;
 
   const int i = min(xl[0] + lane, xh[0] - 1);
-  const long col = a.xoff + i;
+  // offset of this lane's point of row j
+  auto at = [&](int j) { return TR ? (long)i * a.pitch + a.xoff + j : (long)j * a.pitch + a.xoff + i; };
   // x taps of this lane: closure columns read a table row from their end of
   // the line; interior ones the interior row, whose padding taps re-read the
   // centre (a point that is certainly valid) with coefficient zero
@@ -101,8 +110,8 @@ __global__ __launch_bounds__(64 * kStepWaves) void step2d_kernel(StepArgs<T> a)
   }
 #pragma unroll
   for (int k = 0; k < KR; k++) {
-    const int j = min(yl[0] + wv + kStepWaves * k, yh[0] - 1);
-    const long o = (long)j * a.pitch + col;
+    const int j = min(yl[0] + wv + NW * k, yh[0] - 1);
+    const long o = at(j);
 #pragma unroll
     for (int c = 0; c < C; c++) U[k][c] = a.u[c * a.plane + o];
     ri[k] = Kb[k] = T(1);
@@ -121,7 +130,7 @@ __global__ __launch_bounds__(64 * kStepWaves) void step2d_kernel(StepArgs<T> a)
     for (int c = 0; c < C; c++) {
       Y[k][c] = U[k][c];
       P[k][c] = T(0);
-      s[c * FS + (wv + kStepWaves * k) * kStepLanes + lane] = U[k][c];
+      s[c * FS + (wv + NW * k) * kStepLanes + lane] = U[k][c];
     }
   __syncthreads();
 
@@ -130,11 +139,12 @@ __global__ __launch_bounds__(64 * kStepWaves) void step2d_kernel(StepArgs<T> a)
     constexpr bool xe = decltype(XE)::value;
     constexpr int NX = xe ? TAPS : 2 * R + 1;
     const T *f = s + b * BS, *fp = AC ? f + 2 * FS : f;
-    const T *fx = f + r * kStepLanes, *px = fp + r * kStepLanes;
+    // u differentiated in x, v in y, p in both
+    const T *fx = f + (TR && AC ? FS : 0) + r * kStepLanes, *px = fp + r * kStepLanes;
     const bool yc = yedge && (j < CLS || j >= ny - CLS);  // closure row
     const int ry = yc ? (j < CLS ? 0 : ny - TAPS) - yl[0] : r - R;
-    const T *py = fp + ry * kStepLanes + lane, *vy = f + FS + ry * kStepLanes + lane;
-    T ax[NX], bx[NX], ay[TAPS], by[TAPS];  // p (or the one field) and u in x; p and v in y
+    const T *py = fp + ry * kStepLanes + lane, *vy = f + (TR ? 0 : FS) + ry * kStepLanes + lane;
+    T ax[NX], bx[NX], ay[TAPS], by[TAPS];  // p (or the one field) and u / v along the lanes; p and v / u across
 #pragma unroll
     for (int t = 0; t < NX; t++) {
       const int q = xe ? (t < 2 * R + 1 || xpad < 0 ? xt + t : xpad) : lane - R + t;
@@ -153,28 +163,30 @@ __global__ __launch_bounds__(64 * kStepWaves) void step2d_kernel(StepArgs<T> a)
         if constexpr (AC) by[t] = vy[t * kStepLanes];
       }
     }
-    auto ddx = [&](const T *v) {
+    const int gi = TR ? j : i, gj = TR ? i : j;  // grid column and row
+    auto dlane = [&](const T *v) {
       if constexpr (xe) {
         T acc = cf[0] * v[0];
 #pragma unroll
         for (int t = 1; t < TAPS; t++) acc = mad(cf[t], v[t], acc);
-        return a.hix * acc;
+        return hl * acc;
       } else {
-        return dint<T, ORDER>([&](int t) { return v[t]; }, a.hix);
+        return dint<T, ORDER>([&](int t) { return v[t]; }, hl);
       }
     };
-    auto ddy = [&](const T *v) {
+    auto drow = [&](const T *v) {
       if (yc) {
         const T *cy = c_edge<T, ORDER>.c[j < CLS ? j : CLS + (ny - 1 - j)];
         T acc = cy[0] * v[0];
 #pragma unroll
         for (int t = 1; t < TAPS; t++) acc = mad(cy[t], v[t], acc);
-        return a.hiy * acc;
+        return hr * acc;
       }
-      return dint<T, ORDER>([&](int t) { return v[t]; }, a.hiy);
+      return dint<T, ORDER>([&](int t) { return v[t]; }, hr);
     };
     if constexpr (AC) {
-      const T dxp = ddx(ax), dyp = ddy(ay), dxu = ddx(bx), dyv = ddy(by);
+      const T lp = dlane(ax), rp = drow(ay), lf = dlane(bx), rf = drow(by);
+      const T dxp = TR ? rp : lp, dyp = TR ? lp : rp, dxu = TR ? rf : lf, dyv = TR ? lf : rf;
       T fu = T(0), fv = T(0);
       if constexpr (MAT == M_REF) ref_material_at<T>(xc, c3c, s3c, a.ys, a.c4y, a.s4y, j, c5, rik, fu, fv);
       acoustic_F<T, MAT>(dxp, dyp, dxu, dyv, rik, Kk, fu, fv, K[0], K[1], K[2]);
@@ -184,32 +196,33 @@ __global__ __launch_bounds__(64 * kStepWaves) void step2d_kernel(StepArgs<T> a)
         const int bc = a.bc == B_DEFAULT ? B_FSREF : a.bc;
         const T u = Yc[0], v = Yc[1], p = Yc[2];
         if (bc == B_FSREF) {
-          if (i == 0) K[0] -= hqx * p;
-          if (j == 0) K[1] -= hqy * p;
-          if (i == nx - 1) K[0] += hqx * p;
-          if (j == ny - 1) K[1] += hqy * p;
+          if (gi == 0) K[0] -= hqx * p;
+          if (gj == 0) K[1] -= hqy * p;
+          if (gi == a.nx - 1) K[0] += hqx * p;
+          if (gj == a.ny - 1) K[1] += hqy * p;
         } else if (bc == B_FS) {
-          if (i == 0) K[0] -= rik * (hqx * p);
-          if (j == 0) K[1] -= rik * (hqy * p);
-          if (i == nx - 1) K[0] += rik * (hqx * p);
-          if (j == ny - 1) K[1] += rik * (hqy * p);
+          if (gi == 0) K[0] -= rik * (hqx * p);
+          if (gj == 0) K[1] -= rik * (hqy * p);
+          if (gi == a.nx - 1) K[0] += rik * (hqx * p);
+          if (gj == a.ny - 1) K[1] += rik * (hqy * p);
         } else {
-          if (i == 0) K[2] -= Kk * (hqx * u);
-          if (j == 0) K[2] -= Kk * (hqy * v);
-          if (i == nx - 1) K[2] += Kk * (hqx * u);
-          if (j == ny - 1) K[2] += Kk * (hqy * v);
+          if (gi == 0) K[2] -= Kk * (hqx * u);
+          if (gj == 0) K[2] -= Kk * (hqy * v);
+          if (gi == a.nx - 1) K[2] += Kk * (hqx * u);
+          if (gj == a.ny - 1) K[2] += Kk * (hqy * v);
         }
       }
     } else {
       const T va = MAT == M_ARR ? rik : a.ax, vb = MAT == M_ARR ? Kk : a.ay;
-      T k = -mad(va, ddx(ax), vb * ddy(ay));
+      const T l = dlane(ax), w = drow(ay);
+      T k = -mad(va, TR ? w : l, vb * (TR ? l : w));
       if (xe || yc) {
         const T qinv0 = T(Ops<ORDER>::hqinv[0]);
         const T hqx = a.hix * qinv0, hqy = a.hiy * qinv0, u = Yc[0];
-        if (i == 0) k += T(0.5) * (T(-0.5) * (va + fabs(va))) * (hqx * u);
-        if (j == 0) k += T(0.5) * (T(-0.5) * (vb + fabs(vb))) * (hqy * u);
-        if (i == nx - 1) k += T(0.5) * (T(0.5) * (va - fabs(va))) * (hqx * u);
-        if (j == ny - 1) k += T(0.5) * (T(0.5) * (vb - fabs(vb))) * (hqy * u);
+        if (gi == 0) k += T(0.5) * (T(-0.5) * (va + fabs(va))) * (hqx * u);
+        if (gj == 0) k += T(0.5) * (T(-0.5) * (vb + fabs(vb))) * (hqy * u);
+        if (gi == a.nx - 1) k += T(0.5) * (T(0.5) * (va - fabs(va))) * (hqx * u);
+        if (gj == a.ny - 1) k += T(0.5) * (T(0.5) * (vb - fabs(vb))) * (hqy * u);
       }
       K[0] = k;
     }
@@ -227,7 +240,7 @@ __global__ __launch_bounds__(64 * kStepWaves) void step2d_kernel(StepArgs<T> a)
       const int yhi = st == 1 ? y1h : (st == 2 ? y2h : (st == 3 ? y3h : j1));
 #pragma unroll
       for (int k = 0; k < KR; k++) {
-        const int r = wv + kStepWaves * k, j = yl[0] + r;
+        const int r = wv + NW * k, j = yl[0] + r;
         if (j < ylo || j >= yhi) continue;  // (the whole wave)
         T K[C];
         rhs(XE, b, r, j, Y[k], ri[k], Kb[k], c5, K);
@@ -240,7 +253,7 @@ __global__ __launch_bounds__(64 * kStepWaves) void step2d_kernel(StepArgs<T> a)
             s[(b ^ 1) * BS + c * FS + r * kStepLanes + lane] = y;
           }
         } else if (xl[0] + lane >= i0 && xl[0] + lane < i1) {
-          const long o = (long)j * a.pitch + col;
+          const long o = at(j);
 #pragma unroll
           for (int c = 0; c < C; c++) {
             const T inc = mad(P[k][c], a.third, a.ca * K[c]);
@@ -258,8 +271,18 @@ __global__ __launch_bounds__(64 * kStepWaves) void step2d_kernel(StepArgs<T> a)
       __syncthreads();
     }
   };
-  if (xedge) stages(std::true_type{});
+  if (!TR && xedge) stages(std::integral_constant<bool, !TR>{});
   else stages(std::false_type{});
+}
+
+template <typename T, int ORDER, int PHYS, int MAT, bool KAHAN>
+__global__ __launch_bounds__(64 * kStepWaves) void step2d_kernel(StepArgs<T> a)
+{
+  constexpr int H = kStepWaves * step_rows(ORDER);
+  __shared__ T s[step_lds(ORDER, PHYS == PH_ACOUSTIC ? 3 : 1, H)];
+  const int i0 = (blockIdx.x % a.px) * a.pw, j0 = (blockIdx.x / a.px) * a.ph;
+  step_patch<T, ORDER, PHYS, MAT, KAHAN, false, kStepWaves, H>(a, s, i0, min(i0 + a.pw, a.nx), j0,
+                                                               min(j0 + a.ph, a.ny));
 }
 
 // The cut of an nx x ny grid into patches; ok: every region fits a block.
@@ -307,6 +330,55 @@ template <int ORDER> inline StepPlan step_plan_t(int nx, int ny)
 inline StepPlan step_plan(int order, int nx, int ny)
 {
   return order == 2 ? step_plan_t<2>(nx, ny) : (order == 4 ? step_plan_t<4>(nx, ny) : step_plan_t<6>(nx, ny));
+}
+
+// Marched steps (sbp_march.hpp): output columns of a strip, depth of the frame
+// around the strips, the frame's patches (px along the bottom and top each,
+// one per kStepLanes - 4 order rows at either side).
+constexpr int kMarchThreads = 256;
+constexpr int march_cols(int order) { return kMarchThreads - 4 * order; }
+constexpr int march_depth(int order) { return order == 2 ? 4 : (order == 4 ? 10 : 15); }
+constexpr int step_cols(int order) { return kStepLanes - 4 * order; }
+__host__ __device__ inline int march_frame(int order, int px, int ny)
+{
+  return 2 * px + 2 * ((ny - 2 * march_depth(order) + step_cols(order) - 1) / step_cols(order));
+}
+
+// The cut of the marched region into strips and segments.  A segment costs its
+// rows and the 4 order rows it leads in with, and each further block per CU
+// slows the others down by about a quarter of what one alone takes (4097^2
+// FP32 190 / 130 / 128 / 126 us per step at 1 .. 4 per CU, 2049^2 58 / 43 / 41
+// / 45, 1025^2 21 / 17 / 17 / 19): as many blocks per CU, at most `resident`,
+// as make (rows + lead) (1 + w / 4) smallest.  A frame of few patches takes
+// its place within them, so that all blocks of a launch run at once (1025^2
+// FP64: 31 us per step, 36 with another 88 blocks to wait for); a larger one is
+// worth a longer launch (4097^2 FP64 255 / 288).
+struct MarchPlan {
+  bool ok;
+  int strips, segs, seg_rows;
+};
+inline MarchPlan march_plan(int order, int nx, int ny, int px, int resident)
+{
+  constexpr int kCus = 256;
+  const int D = march_depth(order), w = nx - 2 * D, h = ny - 2 * D;
+  MarchPlan p{};
+  if (w < 1 || h < 1 || px < 1 || resident < 1) return p;
+  p.strips = (w + march_cols(order) - 1) / march_cols(order);
+  const int nf = march_frame(order, px, ny);
+  double least = 1e300;
+  for (int per = 1; per <= resident; per++) {
+    const int all = kCus * per, blocks = 4 * nf <= all ? all - nf : all;
+    const int segs = blocks > p.strips ? blocks / p.strips : 1;
+    const int rows = (h + segs - 1) / segs;
+    const double cost = (rows + 4.0 * order) * (4 + per);
+    if (cost < least) {
+      least = cost;
+      p.seg_rows = rows;
+    }
+  }
+  p.segs = (h + p.seg_rows - 1) / p.seg_rows;
+  p.ok = true;
+  return p;
 }
 
 template <typename T, int ORDER, int PHYS, int MAT, bool KAHAN> struct StepLauncher {
