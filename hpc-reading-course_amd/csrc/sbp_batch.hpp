@@ -1,8 +1,9 @@
 // sbp_batch.hpp -- persistent kernels of the batched acoustic ensemble.
 //
 // Many independent 2D acoustic problems of different sizes share one launch
-// per RK4 stage (batch_stage_kernel) or, in the two-stage configurations, one
-// per pair of stages (batch_pair_kernel).  The host flattens the work of every
+// per RK4 stage (batch_stage_kernel), in the two-stage configurations one per
+// pair of stages (batch_pair_kernel), in the whole-step ones one per step
+// (batch_march_kernel, sbp_march.hpp).  The host flattens the work of every
 // instance into one list of (instance, item) pairs -- the boundary-frame
 // blocks (frame patches) and the interior tiles (pair tiles) of
 // sbp_kernels.hpp -- and a fixed grid of persistent blocks walks that list.  The list is cut into one chunk per XCD: whole instances,
@@ -26,6 +27,8 @@ template <typename T> struct BatchInst {
   // two-stage configurations: the (CLS+R)-deep frame and the pair tiles
   int p_depth, p_tiles_x, p_ty_rows, p_n_tiles, p_n_edge, p_n_edge_blocks;
   int p_nts;  // pair tiles' store policy (PairArgs::nts), one for the whole ensemble
+  // whole-step configurations: strips and segment rows, patches of the frame
+  int m_strips, m_seg_rows, m_px, m_pw, m_frame;
 };
 
 template <typename T, int MODE>
@@ -257,5 +260,12 @@ BatchLaunchFn batch_launcher_f32(int order, int mat, bool kahan, int bx, int pf)
 // two-stage configurations (the launch's `mode` argument is the part, 1..4)
 BatchLaunchFn batch_pair_launcher_f64(int order, int mat);
 BatchLaunchFn batch_pair_launcher_f32(int order, int mat, bool kahan);
+// whole-step configurations (sbp_march_o*.hip; the launch's grid is a block per item)
+BatchLaunchFn batch_march_launcher_o2_f64(int mat);
+BatchLaunchFn batch_march_launcher_o4_f64(int mat);
+BatchLaunchFn batch_march_launcher_o6_f64(int mat);
+BatchLaunchFn batch_march_launcher_o2_f32(int mat, bool kahan);
+BatchLaunchFn batch_march_launcher_o4_f32(int mat, bool kahan);
+BatchLaunchFn batch_march_launcher_o6_f32(int mat, bool kahan);
 
 }  // namespace sbp

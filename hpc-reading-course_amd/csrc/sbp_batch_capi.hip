@@ -6,7 +6,7 @@
 // of the persistent stage kernel over the flattened work list (one-stage
 // configurations) or two of the persistent pair kernel (two-stage
 // configurations: stages 1-2 and 3-4, each over every instance's frame
-// patches and pair tiles); nsteps are replayed from a captured hipGraph.  The
+// patches and pair tiles) or one (whole-step configurations); nsteps are replayed from a captured hipGraph.  The
 // schedule, tile shape and number of persistent blocks come from a small
 // table of candidates, chosen by sbp_batch_autotune on the ensemble at hand.
 #include <hip/hip_runtime.h>
@@ -22,6 +22,7 @@
 #include "sbp_batch.hpp"
 #include "sbp_batch_impl.hpp"
 #include "sbp_host.hpp"
+#include "sbp_step.hpp"
 
 using namespace sbp;
 using sbp::host::fail;
@@ -32,15 +33,25 @@ namespace {
 
 struct BatchConfig {
   int bx, ty, blocks_per_cu, pf;  // pf: rows of loads in flight per tile
-  int pair;                        // 1: two RK4 stages per interior launch (bx from pair_nt)
+  int kind;                        // one of the following
+};
+enum {
+  ONE_STAGE,
+  TWO_STAGE,  // two RK4 stages per launch (bx from pair_nt)
+  WHOLE       // a step per launch (march_cols wide, ty: rows of a segment; a block per item)
 };
 
 // Candidate launch shapes of the autotuner.
 // Short tiles (4, 8 rows) are for ensembles of small grids, where tall tiles
 // leave most of the persistent blocks without work.
-// The last nine are two-stage configurations (sbp_kernels.hpp pair2d_kernel);
-// they need every instance to have an interior beyond its (CLS+R)-deep frame.
-// Their tiles are pair_nt wide; bx only sizes the unused one-stage fields.
+// Nine are two-stage configurations (sbp_kernels.hpp pair2d_kernel); they need
+// every instance to have an interior beyond its (CLS+R)-deep frame.  Their
+// tiles are pair_nt wide; bx only sizes the unused one-stage fields.
+// The last ones march whole steps (sbp_march.hpp), where every instance has an
+// interior beyond its (CLS+3R)-deep frame: low segments fill the chip where
+// there are few instances, high ones lead in less often (FP32 with rho/K
+// arrays, us per step at 8, 32 and 128 rows, best two-stage: 16 x 257^2 25 / 33
+// / 90, 37; 48 of 129^2 .. 1025^2 298 / 224 / 199, 421).
 constexpr BatchConfig kConfigs[] = {
     {256, 32, 4, 1, 0}, {256, 64, 4, 1, 0}, {256, 16, 4, 1, 0}, {256, 32, 2, 1, 0}, {256, 32, 8, 1, 0},
     {256, 64, 2, 1, 0}, {128, 32, 8, 1, 0}, {128, 64, 8, 1, 0}, {128, 16, 8, 1, 0}, {128, 32, 4, 1, 0},
@@ -48,6 +59,9 @@ constexpr BatchConfig kConfigs[] = {
     {128, 4, 8, 1, 0},  {256, 8, 4, 4, 0},  {256, 4, 4, 4, 0},  {128, 8, 8, 4, 0},  {128, 4, 8, 4, 0},
     {256, 16, 4, 0, 1}, {256, 8, 4, 0, 1},  {256, 32, 4, 0, 1}, {256, 16, 2, 0, 1}, {256, 16, 3, 0, 1},
     {256, 24, 3, 0, 1}, {256, 12, 3, 0, 1}, {256, 24, 2, 0, 1}, {256, 32, 2, 0, 1},
+    {256, 8, 0, 0, WHOLE},  {256, 12, 0, 0, WHOLE}, {256, 16, 0, 0, WHOLE}, {256, 24, 0, 0, WHOLE},
+    {256, 32, 0, 0, WHOLE}, {256, 48, 0, 0, WHOLE}, {256, 64, 0, 0, WHOLE}, {256, 96, 0, 0, WHOLE},
+    {256, 128, 0, 0, WHOLE},
 };
 constexpr int kNumConfigs = sizeof(kConfigs) / sizeof(kConfigs[0]);
 constexpr int kAlignB = 64;
@@ -69,7 +83,7 @@ void drop_graph(sbp_batch *b)
   }
 }
 
-// Bring the state back to the U pool (after an odd number of two-stage steps
+// Bring the state back to the U pool (after an odd number of two-stage or whole steps
 // it sits in Y0); the one-stage kernels, tuning and configuration changes
 // start from there.
 int normalize_parity(sbp_batch *b)
@@ -80,7 +94,7 @@ int normalize_parity(sbp_batch *b)
   return SBP_OK;
 }
 
-template <typename T> bool fill_inst(const sbp_batch *b, std::vector<BatchInst<T>> &out, int bx, int ty, bool pair)
+template <typename T> bool fill_inst(const sbp_batch *b, std::vector<BatchInst<T>> &out, int bx, int ty, int kind)
 {
   bool ok = true;
   out.resize(b->count);
@@ -119,13 +133,28 @@ template <typename T> bool fill_inst(const sbp_batch *b, std::vector<BatchInst<T
     // two-stage geometry: pair_nt-thread tiles inside a (CLS+R)-deep frame
     const int nt = pair_nt((int)b->esz, b->order), R = b->order / 2, D = b->cls + R;
     const int pw = h.nx - 2 * D, ph = h.ny - 2 * D;
-    if (pair && (pw <= 0 || ph <= 0)) ok = false;
+    if (kind == TWO_STAGE && (pw <= 0 || ph <= 0)) ok = false;
     d.p_depth = D;
     d.p_tiles_x = pw > 0 ? (pw + nt - 2 * R - 1) / (nt - 2 * R) : 0;
     d.p_ty_rows = ty;
     d.p_n_tiles = (pw > 0 && ph > 0) ? d.p_tiles_x * ((ph + ty - 1) / ty) : 0;
     d.p_n_edge = 2 * D * h.nx + 2 * D * (h.ny - 2 * D);
     d.p_n_edge_blocks = pw > 0 && ph > 0 ? frame_patch_count(h.nx, h.ny, D) : 0;  // frame patches
+    d.m_strips = d.m_seg_rows = d.m_px = d.m_pw = d.m_frame = 0;
+    if (kind == WHOLE) {
+      const int MD = march_depth(b->order), mh = h.ny - 2 * MD, mw = h.nx - 2 * MD;
+      const StepPlan sp = step_plan(b->order, h.nx, h.ny);
+      if (mw <= 0 || mh <= 0 || !sp.ok) {
+        ok = false;
+        continue;
+      }
+      const int segs = (mh + ty - 1) / ty;
+      d.m_strips = (mw + march_cols(b->order) - 1) / march_cols(b->order);
+      d.m_seg_rows = (mh + segs - 1) / segs;
+      d.m_px = sp.px;
+      d.m_pw = sp.pw;
+      d.m_frame = march_frame(b->order, sp.px, h.ny);
+    }
   }
   return ok;
 }
@@ -136,7 +165,14 @@ int apply_config(sbp_batch *b, int cfg)
   const BatchConfig c = kConfigs[cfg];
   const bool kahan = b->prec == SBP_FP32_KAHAN;
   BatchLaunchFn fn;
-  if (c.pair)
+  if (c.kind == WHOLE)
+    fn = b->prec == SBP_FP64
+             ? (b->order == 2 ? batch_march_launcher_o2_f64
+                              : (b->order == 4 ? batch_march_launcher_o4_f64 : batch_march_launcher_o6_f64))(b->mat)
+             : (b->order == 2 ? batch_march_launcher_o2_f32
+                              : (b->order == 4 ? batch_march_launcher_o4_f32 : batch_march_launcher_o6_f32))(b->mat,
+                                                                                                            kahan);
+  else if (c.kind == TWO_STAGE)
     fn = b->prec == SBP_FP64 ? batch_pair_launcher_f64(b->order, b->mat)
                              : batch_pair_launcher_f32(b->order, b->mat, kahan);
   else
@@ -150,13 +186,52 @@ int apply_config(sbp_batch *b, int cfg)
   // patches), so long items start early and short ones fill the tail on every
   // XCD alike.
   std::vector<int2> work;
+  int most = 0;  // items of the longest chunk
+  // Whole steps: every instance's segments in turn are cut into chunks of
+  // equal work, and the frame patches after them likewise (neighbours stay
+  // together, instances need not: few large ones still load every XCD alike).
+  auto build_whole = [&](auto &desc) {
+    const int lead = 4 * b->order, MD = march_depth(b->order);
+    std::vector<std::vector<int2>> on(kNumXcd);
+    for (int frames = 0; frames < 2; frames++) {
+      std::vector<int2> items;
+      std::vector<double> weight;
+      for (int k = 0; k < b->count; k++) {
+        const auto &d = desc[k];
+        if (frames) {
+          for (int e = 0; e < d.m_frame; e++) items.push_back(make_int2(k, e)), weight.push_back(1);
+        } else {
+          const int h = d.ny - 2 * MD, segs = (h + d.m_seg_rows - 1) / d.m_seg_rows;
+          for (int t = 0; t < d.m_strips * segs; t++) {
+            const int rows = std::min(d.m_seg_rows, h - t / d.m_strips * d.m_seg_rows);
+            items.push_back(make_int2(k, d.m_frame + t)), weight.push_back(rows + lead);
+          }
+        }
+      }
+      double total = 0, sum = 0;
+      for (double v : weight) total += v;
+      for (size_t i = 0; i < items.size(); i++) {
+        on[std::min(kNumXcd - 1, (int)((sum + 0.5 * weight[i]) / total * kNumXcd))].push_back(items[i]);
+        sum += weight[i];
+      }
+    }
+    std::vector<int2> items;
+    work.assign(kNumXcd, make_int2(0, 0));
+    for (int x = 0; x < kNumXcd; x++) {
+      work[x] = make_int2((int)items.size(), (int)on[x].size());
+      items.insert(items.end(), on[x].begin(), on[x].end());
+      most = std::max(most, (int)on[x].size());
+    }
+    work.insert(work.end(), items.begin(), items.end());
+  };
   auto build = [&](auto &desc) {
+    if (c.kind == WHOLE) return build_whole(desc);
     const int R = b->order / 2;
-    auto tiles = [&](int k) { return c.pair ? desc[k].p_n_tiles : desc[k].n_tiles; };
-    auto eblocks = [&](int k) { return c.pair ? desc[k].p_n_edge_blocks : desc[k].n_edge_blocks; };
+    auto tiles = [&](int k) { return c.kind == TWO_STAGE ? desc[k].p_n_tiles : desc[k].n_tiles; };
+    auto eblocks = [&](int k) { return c.kind == TWO_STAGE ? desc[k].p_n_edge_blocks : desc[k].n_edge_blocks; };
     std::vector<double> weight(b->count);  // in 256-point rows (a frame patch: about 4, two stages on its grown points)
     for (int k = 0; k < b->count; k++)
-      weight[k] = c.pair ? (double)tiles(k) * (c.ty + 4 * R) + 4.0 * eblocks(k)
+      weight[k] = c.kind == TWO_STAGE ? (double)tiles(k) * (c.ty + 4 * R) + 4.0 * eblocks(k)
                          : (double)tiles(k) * (c.ty + 2 * R) * c.bx / 256.0 + eblocks(k);
     std::vector<int> order(b->count);
     for (int k = 0; k < b->count; k++) order[k] = k;
@@ -194,19 +269,22 @@ int apply_config(sbp_batch *b, int cfg)
   std::vector<BatchInst<float>> df;
   bool fits;
   if (b->esz == 8) {
-    fits = fill_inst(b, dd, c.bx, c.ty, c.pair);
-    build(dd);
+    fits = fill_inst(b, dd, c.bx, c.ty, c.kind);
+    if (fits) build(dd);
     desc_bytes = dd.size() * sizeof(BatchInst<double>);
     const auto sw = swapped(dd);
     dd.insert(dd.end(), sw.begin(), sw.end());
   } else {
-    fits = fill_inst(b, df, c.bx, c.ty, c.pair);
-    build(df);
+    fits = fill_inst(b, df, c.bx, c.ty, c.kind);
+    if (fits) build(df);
     desc_bytes = df.size() * sizeof(BatchInst<float>);
     const auto sw = swapped(df);
     df.insert(df.end(), sw.begin(), sw.end());
   }
-  if (!fits) return fail(SBP_EINVAL, "two-stage configurations need every instance larger than 2(CLS+R) points");
+  if (!fits)
+    return fail(SBP_EINVAL, c.kind == WHOLE
+                                ? "whole-step configurations need every instance larger than 2(CLS+3R) points"
+                                : "two-stage configurations need every instance larger than 2(CLS+R) points");
   int rc = normalize_parity(b);
   if (rc) return rc;
   HIP_OR_FAIL(hipStreamSynchronize(b->stream));
@@ -222,10 +300,11 @@ int apply_config(sbp_batch *b, int cfg)
                         hipMemcpyHostToDevice));
   b->desc_bytes = desc_bytes;
   b->nwork = (int)work.size();
-  b->pair = c.pair != 0;
+  b->kind = c.kind;
   b->auto_nts = b->esz == 8 ? dd[0].p_nts : df[0].p_nts;
   b->pair_nts = b->store_policy == 0 ? b->auto_nts : (b->store_policy == 2 ? 1 : 0);
-  b->grid = std::max(kNumXcd, (b->num_cus * c.blocks_per_cu + kNumXcd - 1) / kNumXcd * kNumXcd);
+  b->grid = c.kind == WHOLE ? kNumXcd * most
+                            : std::max(kNumXcd, (b->num_cus * c.blocks_per_cu + kNumXcd - 1) / kNumXcd * kNumXcd);
   b->launch = fn;
   b->config = cfg;
   return SBP_OK;
@@ -256,7 +335,12 @@ int upload_dt(sbp_batch *b, const double *dt)
 hipError_t launch_step(sbp_batch *b)
 {
   hipError_t e = hipSuccess;
-  if (b->pair) {  // parts 1 and 3 on the descriptors of the current parity
+  if (b->kind == WHOLE) {
+    e = b->launch(0, sbp::host::batch_inst(b), b->work_dev, b->nwork, b->grid, b->stream);
+    if (e == hipSuccess) b->par ^= 1;
+    return e;
+  }
+  if (b->kind == TWO_STAGE) {  // parts 1 and 3 on the descriptors of the current parity
     const void *inst = sbp::host::batch_inst(b);
     for (int p = 1; p <= 3 && e == hipSuccess; p += 2)
       e = b->launch(p | (b->pair_nts ? 0 : kBatchCachedStores), inst, b->work_dev, b->nwork, b->grid, b->stream);
@@ -268,7 +352,7 @@ hipError_t launch_step(sbp_batch *b)
   return e;
 }
 
-// kBatchGraphSteps is even: a two-stage capture ends at the parity it began.
+// kBatchGraphSteps is even: a capture of two-stage or whole steps ends at the parity it began.
 int ensure_graph(sbp_batch *b)
 {
   if (b->gexec[b->par]) return SBP_OK;
@@ -629,10 +713,11 @@ int sbp_batch_get_config(const sbp_batch *b, int *config, int *tile_width, int *
   if (!b) return fail(SBP_EINVAL, "null batch");
   const BatchConfig c = kConfigs[b->config];
   if (config) *config = b->config;
-  if (tile_width) *tile_width = c.pair ? pair_nt((int)b->esz, b->order) : c.bx;
+  if (tile_width) *tile_width = c.kind == WHOLE ? march_cols(b->order)
+                                             : (c.kind == TWO_STAGE ? pair_nt((int)b->esz, b->order) : c.bx);
   if (tile_rows) *tile_rows = c.ty;
   if (blocks_per_cu) *blocks_per_cu = c.blocks_per_cu;
-  if (two_stage) *two_stage = c.pair;
+  if (two_stage) *two_stage = c.kind == TWO_STAGE;
   return SBP_OK;
 }
 
@@ -657,7 +742,7 @@ int sbp_batch_autotune(sbp_batch *b, const double *dt, int *choice)
   float best_ms = 1e30f;
   for (int cfg = 0; cfg < kNumConfigs && rc == SBP_OK; cfg++) {
     const int arc = apply_config(b, cfg);
-    if (arc == SBP_EINVAL && kConfigs[cfg].pair) continue;  // instances too small for a two-stage tile
+    if (arc == SBP_EINVAL && kConfigs[cfg].kind != ONE_STAGE) continue;  // instances too small for it
     if ((rc = arc)) break;
     for (int s = 0; s < 2 && rc == SBP_OK; s++)
       if (launch_step(b) != hipSuccess) rc = fail(SBP_EHIP, "autotune warm-up launch failed");

@@ -34,8 +34,8 @@ struct sbp_batch {
   int pair_nts = 1;          // two-stage: nontemporal (1) or cached (0) pair-tile stores
   int auto_nts = 1;          // the same chosen from the streamed bytes
   int store_policy = 0;      // 0: auto_nts, 1: cached, 2: nontemporal
-  bool pair = false;         // the configuration runs two RK4 stages per interior launch
-  int par = 0;               // 1: a two-stage step left the state in the Y0 pool
+  int kind = 0;              // the configuration's schedule (BatchConfig)
+  int par = 0;               // 1: a two-stage or whole step left the state in the Y0 pool
   double *aos = nullptr, *partials = nullptr, *scalar = nullptr;
   hipStream_t stream = nullptr;
   hipGraphExec_t gexec[2] = {nullptr, nullptr};  // captured steps, by starting parity

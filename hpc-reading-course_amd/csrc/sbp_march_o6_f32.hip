@@ -5,4 +5,8 @@ MarchFns march_launcher_o6_f32(int phys, int mat, bool kahan)
 {
   return kahan ? pick_march<float, 6, true>(phys, mat) : pick_march<float, 6, false>(phys, mat);
 }
+BatchLaunchFn batch_march_launcher_o6_f32(int mat, bool kahan)
+{
+  return kahan ? pick_batch_march<float, 6, true>(mat) : pick_batch_march<float, 6, false>(mat);
+}
 }  // namespace sbp

@@ -252,7 +252,8 @@ int  sbp_error_norms_noalloc(const double *v, const double *w, long n, double hx
  * Many independent 2D acoustic problems (uneven sizes, own materials, own dt)
  * advanced together: one persistent kernel per RK4 stage (or, in the
  * two-stage configurations, per pair of stages) walks a flattened list of
- * every instance's tiles and boundary blocks, and nsteps are replayed from a
+ * every instance's tiles and boundary blocks; whole-step configurations take
+ * a block per item of such a list and one launch per step; nsteps are replayed from a
  * captured hipGraph.  No counterpart in the reference, which runs one problem per MPI
  * job (code/batch.sh:1-7); each instance's arithmetic is the single-problem
  * path's (sbp_rk4_advance).  All instances share order, precision and
@@ -272,7 +273,10 @@ int  sbp_batch_energy(sbp_batch *b, int k, double *E);
 /* Launch-shape candidates (tile width, tile rows, persistent blocks per CU,
  * and whether the step runs two RK4 stages per launch: the schedule of
  * sbp_set_fused, which needs every instance larger than 2(CLS+R) points;
- * sbp_batch_set_config fails with SBP_EINVAL otherwise). */
+ * sbp_batch_set_config fails with SBP_EINVAL otherwise).  Whole-step
+ * candidates (strip width, segment rows, 0 blocks per CU, two_stage 0) need
+ * more than 2(CLS+3R) points and give the one-stage candidates' results bit
+ * for bit. */
 int  sbp_batch_num_configs(void);
 int  sbp_batch_set_config(sbp_batch *b, int config);
 int  sbp_batch_get_config(const sbp_batch *b, int *config, int *tile_width, int *tile_rows,
