@@ -396,11 +396,16 @@ void release(sbp_batch *b)
   for (void *p : {b->U, b->A, b->Y0, b->Y1, b->KC, b->RI, b->BK, b->inst_dev, (void *)b->work_dev, (void *)b->aos,
                   (void *)b->partials, (void *)b->scalar})
     if (p) (void)hipFree(p);
+  if (b->aos_pin) (void)hipHostFree(b->aos_pin);
   if (b->ev0) (void)hipEventDestroy(b->ev0);
   if (b->ev1) (void)hipEventDestroy(b->ev1);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   delete b;
 }
+
+// where a vector of so many bytes lies on its way to or from the caller
+bool in_host(size_t bytes) { return bytes <= sbp::host::kZeroCopyBytes; }
+double *aos_of(const sbp_batch *b, size_t bytes) { return in_host(bytes) ? b->aos_pin : b->aos; }
 
 int check_index(const sbp_batch *b, int k)
 {
@@ -458,7 +463,10 @@ int build_batch(const sbp_problem *descs, int count, sbp_batch *b)
     HIP_OR_FAIL(hipMalloc(&b->KC, reg));
     HIP_OR_FAIL(hipMemsetAsync(b->KC, 0, reg, b->stream));
   }
-  HIP_OR_FAIL(hipMalloc(&b->aos, sizeof(double) * 3 * (size_t)b->max_pts));
+  const size_t aos_bytes = sizeof(double) * 3 * (size_t)b->max_pts;
+  if (aos_bytes > sbp::host::kZeroCopyBytes) HIP_OR_FAIL(hipMalloc(&b->aos, aos_bytes));
+  HIP_OR_FAIL(hipHostMalloc(reinterpret_cast<void **>(&b->aos_pin), std::min(aos_bytes, sbp::host::kZeroCopyBytes),
+                            hipHostMallocDefault));
   HIP_OR_FAIL(hipMalloc(&b->partials, sizeof(double) * 1024));
   HIP_OR_FAIL(hipMalloc(&b->scalar, sizeof(double)));
   if (b->mat == SBP_MAT_ARRAYS) {
@@ -468,15 +476,17 @@ int build_batch(const sbp_problem *descs, int count, sbp_batch *b)
       const InstHost &h = b->inst[k];
       const long n = (long)h.nx * h.ny;
       const int grid = (int)((n + 255) / 256);
+      const size_t bytes = sizeof(double) * n;
+      double *aos = aos_of(b, bytes);
       for (int which = 0; which < 2; which++) {
         const double *src = which == 0 ? descs[k].rho_inv : descs[k].bulk;
         void *dst = which == 0 ? b->RI : b->BK;
-        HIP_OR_FAIL(hipMemcpyAsync(b->aos, src, sizeof(double) * n, hipMemcpyHostToDevice, b->stream));
+        HIP_OR_FAIL(sbp::host::put(aos, in_host(bytes), src, bytes, b->stream));
         if (b->esz == 8)
-          hipLaunchKernelGGL(matrix_to_plane_kernel<double>, dim3(grid), dim3(256), 0, b->stream, b->aos,
+          hipLaunchKernelGGL(matrix_to_plane_kernel<double>, dim3(grid), dim3(256), 0, b->stream, aos,
                              static_cast<double *>(dst) + h.off, h.nx, h.ny, h.pitch, h.xoff);
         else
-          hipLaunchKernelGGL(matrix_to_plane_kernel<float>, dim3(grid), dim3(256), 0, b->stream, b->aos,
+          hipLaunchKernelGGL(matrix_to_plane_kernel<float>, dim3(grid), dim3(256), 0, b->stream, aos,
                              static_cast<float *>(dst) + h.off, h.nx, h.ny, h.pitch, h.xoff);
         HIP_OR_FAIL(hipGetLastError());
         HIP_OR_FAIL(hipStreamSynchronize(b->stream));
@@ -586,15 +596,17 @@ int sbp_batch_set_state(sbp_batch *b, int k, const double *v)
   if (rc) return rc;
   if (!v) return fail(SBP_EINVAL, "null vector");
   const InstHost &h = b->inst[k];
-  const long n = (long)h.nx * h.ny;
-  HIP_OR_FAIL(hipMemcpyAsync(b->aos, v, sizeof(double) * 3 * n, hipMemcpyHostToDevice, b->stream));
+  const long n = 3L * h.nx * h.ny;
+  const size_t bytes = sizeof(double) * n;
+  double *aos = aos_of(b, bytes);
+  HIP_OR_FAIL(sbp::host::put(aos, in_host(bytes), v, bytes, b->stream));
   const int grid = (int)((n + 255) / 256);
   if (b->esz == 8)
-    hipLaunchKernelGGL(aos_to_planar_kernel<double>, dim3(grid), dim3(256), 0, b->stream, b->aos,
+    hipLaunchKernelGGL(aos_to_planar_kernel<double>, dim3(grid), dim3(256), 0, b->stream, aos,
                        static_cast<double *>(sbp::host::batch_state(b)) + 3 * h.off, (double *)nullptr, h.nx, h.ny, 3,
                        h.pitch, h.xoff, h.plane);
   else
-    hipLaunchKernelGGL(aos_to_planar_kernel<float>, dim3(grid), dim3(256), 0, b->stream, b->aos,
+    hipLaunchKernelGGL(aos_to_planar_kernel<float>, dim3(grid), dim3(256), 0, b->stream, aos,
                        static_cast<float *>(sbp::host::batch_state(b)) + 3 * h.off,
                        b->KC ? static_cast<float *>(b->KC) + 3 * h.off : nullptr, h.nx, h.ny, 3, h.pitch, h.xoff,
                        h.plane);
@@ -611,20 +623,21 @@ int sbp_batch_get_state(sbp_batch *b, int k, double *v)
   if (!v) return fail(SBP_EINVAL, "null vector");
   if (!b->have_state[k]) return fail(SBP_ESTATE, "no state loaded for this instance");
   const InstHost &h = b->inst[k];
-  const long n = (long)h.nx * h.ny;
+  const long n = 3L * h.nx * h.ny;
   const int grid = (int)((n + 255) / 256);
+  const size_t bytes = sizeof(double) * n;
+  double *aos = aos_of(b, bytes);
   if (b->esz == 8)
     hipLaunchKernelGGL(planar_to_aos_kernel<double>, dim3(grid), dim3(256), 0, b->stream,
-                       static_cast<const double *>(sbp::host::batch_state(b)) + 3 * h.off, (const double *)nullptr, b->aos, h.nx, h.ny,
+                       static_cast<const double *>(sbp::host::batch_state(b)) + 3 * h.off, (const double *)nullptr, aos, h.nx, h.ny,
                        3, h.pitch, h.xoff, h.plane);
   else
     hipLaunchKernelGGL(planar_to_aos_kernel<float>, dim3(grid), dim3(256), 0, b->stream,
                        static_cast<const float *>(sbp::host::batch_state(b)) + 3 * h.off,
-                       b->KC ? static_cast<const float *>(b->KC) + 3 * h.off : nullptr, b->aos, h.nx, h.ny, 3,
+                       b->KC ? static_cast<const float *>(b->KC) + 3 * h.off : nullptr, aos, h.nx, h.ny, 3,
                        h.pitch, h.xoff, h.plane);
   HIP_OR_FAIL(hipGetLastError());
-  HIP_OR_FAIL(hipMemcpyAsync(v, b->aos, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, b->stream));
-  HIP_OR_FAIL(hipStreamSynchronize(b->stream));
+  HIP_OR_FAIL(sbp::host::get(b->staging, v, aos, in_host(bytes), bytes, b->stream));
   return SBP_OK;
 }
 
@@ -636,20 +649,21 @@ int sbp_batch_get_state_strided(sbp_batch *b, int k, int stride, double *v)
   if (!b->have_state[k]) return fail(SBP_ESTATE, "no state loaded for this instance");
   const InstHost &h = b->inst[k];
   const int cx = (h.nx - 1) / stride + 1, cy = (h.ny - 1) / stride + 1;
-  const long n = (long)cx * cy;
+  const long n = 3L * cx * cy;
   const int grid = (int)((n + 255) / 256);
+  const size_t bytes = sizeof(double) * n;
+  double *aos = aos_of(b, bytes);
   if (b->esz == 8)
     hipLaunchKernelGGL(planar_to_aos_strided_kernel<double>, dim3(grid), dim3(256), 0, b->stream,
-                       static_cast<const double *>(sbp::host::batch_state(b)) + 3 * h.off, (const double *)nullptr, b->aos, h.nx, h.ny, 3,
+                       static_cast<const double *>(sbp::host::batch_state(b)) + 3 * h.off, (const double *)nullptr, aos, h.nx, h.ny, 3,
                        h.pitch, h.xoff, h.plane, stride);
   else
     hipLaunchKernelGGL(planar_to_aos_strided_kernel<float>, dim3(grid), dim3(256), 0, b->stream,
                        static_cast<const float *>(sbp::host::batch_state(b)) + 3 * h.off,
-                       b->KC ? static_cast<const float *>(b->KC) + 3 * h.off : nullptr, b->aos, h.nx, h.ny, 3, h.pitch,
+                       b->KC ? static_cast<const float *>(b->KC) + 3 * h.off : nullptr, aos, h.nx, h.ny, 3, h.pitch,
                        h.xoff, h.plane, stride);
   HIP_OR_FAIL(hipGetLastError());
-  HIP_OR_FAIL(hipMemcpyAsync(v, b->aos, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, b->stream));
-  HIP_OR_FAIL(hipStreamSynchronize(b->stream));
+  HIP_OR_FAIL(sbp::host::get(b->staging, v, aos, in_host(bytes), bytes, b->stream));
   return SBP_OK;
 }
 

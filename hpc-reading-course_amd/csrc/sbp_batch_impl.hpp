@@ -7,6 +7,7 @@
 
 #include "../../include/sbp_hip.h"
 #include "sbp_batch.hpp"
+#include "sbp_xfer.hpp"
 
 namespace sbp {
 namespace host {
@@ -36,7 +37,9 @@ struct sbp_batch {
   int store_policy = 0;      // 0: auto_nts, 1: cached, 2: nontemporal
   int kind = 0;              // the configuration's schedule (BatchConfig)
   int par = 0;               // 1: a two-stage or whole step left the state in the Y0 pool
-  double *aos = nullptr, *partials = nullptr, *scalar = nullptr;
+  double *aos = nullptr, *aos_pin = nullptr;  // an instance's vector in device or, small ones, host memory (sbp_xfer.hpp)
+  sbp::host::Staging staging;
+  double *partials = nullptr, *scalar = nullptr;
   hipStream_t stream = nullptr;
   hipGraphExec_t gexec[2] = {nullptr, nullptr};  // captured steps, by starting parity
   hipEvent_t ev0 = nullptr, ev1 = nullptr;

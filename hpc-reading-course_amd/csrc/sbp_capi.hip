@@ -543,21 +543,20 @@ int run_steps(sbp_ctx *c, double t0, double dt, long nsteps, double *t_end = nul
 int upload_aos(sbp_ctx *c, const double *v)
 {
   const size_t bytes = sizeof(double) * (size_t)c->C * c->nx * c->ny;
-  HIP_OR_FAIL(hipMemcpyAsync(c->aos, v, bytes, hipMemcpyHostToDevice, c->stream));
+  HIP_OR_FAIL(host::put(c->aos, c->aos_host, v, bytes, c->stream));
   return SBP_OK;
 }
 
 int download_aos(sbp_ctx *c, double *v)
 {
   const size_t bytes = sizeof(double) * (size_t)c->C * c->nx * c->ny;
-  HIP_OR_FAIL(hipMemcpyAsync(v, c->aos, bytes, hipMemcpyDeviceToHost, c->stream));
-  HIP_OR_FAIL(hipStreamSynchronize(c->stream));
+  HIP_OR_FAIL(host::get(c->staging, v, c->aos, c->aos_host, bytes, c->stream));
   return SBP_OK;
 }
 
 int aos_to_planar(sbp_ctx *c, void *dst, void *comp)
 {
-  const long n = (long)c->nx * c->ny;
+  const long n = (long)c->C * c->nx * c->ny;
   const int grid = (int)((n + 255) / 256);
   if (c->esz == 8)
     hipLaunchKernelGGL(aos_to_planar_kernel<double>, dim3(grid), dim3(256), 0, c->stream, c->aos,
@@ -571,7 +570,7 @@ int aos_to_planar(sbp_ctx *c, void *dst, void *comp)
 
 int planar_to_aos(sbp_ctx *c, const void *src, const void *comp)
 {
-  const long n = (long)c->nx * c->ny;
+  const long n = (long)c->C * c->nx * c->ny;
   const int grid = (int)((n + 255) / 256);
   if (c->esz == 8)
     hipLaunchKernelGGL(planar_to_aos_kernel<double>, dim3(grid), dim3(256), 0, c->stream,
@@ -677,7 +676,7 @@ int upload_plane(sbp_ctx *c, const double *m, void **dst)
   const size_t n = (size_t)c->nx * c->ny;
   int rc = dalloc(dst, c->esz * (size_t)c->plane);
   if (rc) return rc;
-  HIP_OR_FAIL(hipMemcpyAsync(c->aos, m, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
+  HIP_OR_FAIL(host::put(c->aos, c->aos_host, m, sizeof(double) * n, c->stream));
   const int grid = (int)((n + 255) / 256);
   if (c->esz == 8)
     hipLaunchKernelGGL(matrix_to_plane_kernel<double>, dim3(grid), dim3(256), 0, c->stream, c->aos,
@@ -704,7 +703,8 @@ void release(sbp_ctx *c)
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   drop_graph(c);
   void *ptrs[] = {c->U,   c->A,   c->Y0,  c->Y1,  c->KC,  c->TK,  c->rinv,     c->bulk,     c->velx, c->vely,
-                  c->xs,  c->ys,  c->c3x, c->s3x, c->c4y, c->s4y, c->aos,      c->aos2,     c->partials, c->scalar};
+                  c->xs,  c->ys,  c->c3x, c->s3x, c->c4y, c->s4y, c->aos2, c->partials, c->scalar, c->aos_host ? nullptr : c->aos};
+  if (c->aos_host && c->aos) (void)hipHostFree(c->aos);
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   for (void *p : c->rkw)
@@ -817,7 +817,13 @@ int build_ctx(const sbp_problem *desc, sbp_ctx *c)
   // Zero the registers once so padding never holds stale bit patterns.
   for (void *p : {c->U, c->A, c->Y0, c->Y1, c->KC, c->TK})
     if (p) HIP_OR_FAIL(hipMemsetAsync(p, 0, reg_bytes, c->stream));
-  if ((rc = dalloc(&c->aos, sizeof(double) * (size_t)c->C * c->nx * c->ny))) return rc;
+  const size_t aos_bytes = sizeof(double) * (size_t)c->C * c->nx * c->ny;
+  c->aos_host = aos_bytes <= host::kZeroCopyBytes;
+  if (!c->aos_host) {
+    if ((rc = dalloc(&c->aos, aos_bytes))) return rc;
+  } else {
+    HIP_OR_FAIL(hipHostMalloc(reinterpret_cast<void **>(&c->aos), aos_bytes, hipHostMallocDefault));
+  }
   c->npartials = 1024;
   if ((rc = dalloc(&c->partials, sizeof(double) * c->npartials)) || (rc = dalloc(&c->scalar, 2 * sizeof(double))))
     return rc;
@@ -1167,7 +1173,7 @@ int sbp_get_state_strided(sbp_ctx *ctx, int stride, double *v)
   if (!ctx || !v || stride < 1) return fail(SBP_EINVAL, "bad argument");
   if (!ctx->have_state) return fail(SBP_ESTATE, "no state loaded");
   const int cx = (ctx->nx - 1) / stride + 1, cy = (ctx->ny - 1) / stride + 1;
-  const long n = (long)cx * cy;
+  const long n = (long)ctx->C * cx * cy;
   const int grid = (int)((n + 255) / 256);
   if (ctx->esz == 8)
     hipLaunchKernelGGL(planar_to_aos_strided_kernel<double>, dim3(grid), dim3(256), 0, ctx->stream,
@@ -1178,8 +1184,7 @@ int sbp_get_state_strided(sbp_ctx *ctx, int stride, double *v)
                        (const float *)ctx->U, (const float *)ctx->KC, ctx->aos, ctx->nx, ctx->ny, ctx->C, ctx->pitch,
                        ctx->xoff, ctx->plane, stride);
   HIP_OR_FAIL(hipGetLastError());
-  HIP_OR_FAIL(hipMemcpyAsync(v, ctx->aos, sizeof(double) * ctx->C * n, hipMemcpyDeviceToHost, ctx->stream));
-  HIP_OR_FAIL(hipStreamSynchronize(ctx->stream));
+  HIP_OR_FAIL(host::get(ctx->staging, v, ctx->aos, ctx->aos_host, sizeof(double) * n, ctx->stream));
   return SBP_OK;
 }
 
@@ -1355,7 +1360,7 @@ int sbp_error_norms(sbp_ctx *ctx, const double *v, const double *w, double *l2, 
     int rc = dalloc(&ctx->aos2, sizeof(double) * (size_t)n);
     if (rc) return rc;
   }
-  HIP_OR_FAIL(hipMemcpyAsync(ctx->aos, v, sizeof(double) * n, hipMemcpyHostToDevice, ctx->stream));
+  HIP_OR_FAIL(host::put(ctx->aos, ctx->aos_host, v, sizeof(double) * n, ctx->stream));
   HIP_OR_FAIL(hipMemcpyAsync(ctx->aos2, w, sizeof(double) * n, hipMemcpyHostToDevice, ctx->stream));
   const int grid = (int)std::max<long>(1, std::min<long>((n + 255) / 256, ctx->npartials / 2));
   hipLaunchKernelGGL(diff_norms_kernel, dim3(grid), dim3(256), 0, ctx->stream, ctx->aos, ctx->aos2, n, ctx->partials);

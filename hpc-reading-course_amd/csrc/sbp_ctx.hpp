@@ -6,6 +6,7 @@
 #include "../../include/sbp_hip.h"
 #include "sbp_kernels.hpp"
 #include "sbp_step.hpp"
+#include "sbp_xfer.hpp"
 
 struct sbp_ctx {
   sbp_problem d{};
@@ -19,7 +20,10 @@ struct sbp_ctx {
   void *rinv = nullptr, *bulk = nullptr;
   void *velx = nullptr, *vely = nullptr;  // advection velocity fields (per-point a, b)
   double *xs = nullptr, *ys = nullptr, *c3x = nullptr, *s3x = nullptr, *c4y = nullptr, *s4y = nullptr;
-  double *aos = nullptr, *aos2 = nullptr;  // AoS FP64 staging (aos2: second operand, on first use)
+  // AoS FP64 staging: pinned host memory (aos_host) or device memory (sbp_xfer.hpp); aos2: second operand, on first use
+  double *aos = nullptr, *aos2 = nullptr;
+  bool aos_host = false;
+  sbp::host::Staging staging;
   double *partials = nullptr, *scalar = nullptr;
   int npartials = 0;
   hipStream_t stream = nullptr;

@@ -1344,23 +1344,23 @@ static __global__ __launch_bounds__(256) void norm_final_kernel(const double *pa
 }
 
 // --------------------------------------------------------------------------
-// AoS (reference layout, double) <-> planar device state.
+// AoS (reference layout, double) <-> planar device state.  A thread per AoS
+// value, so that the vector, which may lie in host memory, is read and written
+// in whole lines.
 // --------------------------------------------------------------------------
 template <typename T>
 __global__ __launch_bounds__(256) void aos_to_planar_kernel(const double *__restrict__ aos, T *__restrict__ U,
                                                             T *__restrict__ comp, int nx, int ny, int nc,
                                                             int pitch, int xoff, long plane)
 {
-  const long k = blockIdx.x * 256L + threadIdx.x;
-  if (k >= (long)nx * ny) return;
-  const int j = (int)(k / nx), i = (int)(k - (long)j * nx);
-  const long o = (long)j * pitch + xoff + i;
-  for (int c = 0; c < nc; c++) {
-    const double v = aos[k * nc + c];
-    const T t = (T)v;
-    U[c * plane + o] = t;
-    if (comp) comp[c * plane + o] = (T)((double)t - v);  // value = U - comp
-  }
+  const unsigned m = blockIdx.x * 256u + threadIdx.x;  // (nx ny <= 2^30 points of at most 3 values)
+  if (m >= (unsigned)nx * ny * nc) return;
+  const unsigned k = m / nc, c = m - k * nc, j = k / nx, i = k - j * nx;
+  const long o = c * plane + (long)j * pitch + xoff + i;
+  const double v = aos[m];
+  const T t = (T)v;
+  U[o] = t;
+  if (comp) comp[o] = (T)((double)t - v);  // value = U - comp
 }
 
 template <typename T>
@@ -1368,15 +1368,13 @@ __global__ __launch_bounds__(256) void planar_to_aos_kernel(const T *__restrict_
                                                             double *__restrict__ aos, int nx, int ny, int nc,
                                                             int pitch, int xoff, long plane)
 {
-  const long k = blockIdx.x * 256L + threadIdx.x;
-  if (k >= (long)nx * ny) return;
-  const int j = (int)(k / nx), i = (int)(k - (long)j * nx);
-  const long o = (long)j * pitch + xoff + i;
-  for (int c = 0; c < nc; c++) {
-    double v = (double)U[c * plane + o];
-    if (comp) v -= (double)comp[c * plane + o];
-    aos[k * nc + c] = v;
-  }
+  const unsigned m = blockIdx.x * 256u + threadIdx.x;
+  if (m >= (unsigned)nx * ny * nc) return;
+  const unsigned k = m / nc, c = m - k * nc, j = k / nx, i = k - j * nx;
+  const long o = c * plane + (long)j * pitch + xoff + i;
+  double v = (double)U[o];
+  if (comp) v -= (double)comp[o];
+  aos[m] = v;
 }
 
 // Every stride-th point in both directions (injection onto a nested grid).
@@ -1385,16 +1383,14 @@ __global__ __launch_bounds__(256) void planar_to_aos_strided_kernel(const T *__r
                                                                     double *__restrict__ aos, int nx, int ny, int nc,
                                                                     int pitch, int xoff, long plane, int stride)
 {
-  const int cx = (nx - 1) / stride + 1, cy = (ny - 1) / stride + 1;
-  const long k = blockIdx.x * 256L + threadIdx.x;
-  if (k >= (long)cx * cy) return;
-  const int cj = (int)(k / cx), ci = (int)(k - (long)cj * cx);
-  const long o = (long)cj * stride * pitch + xoff + (long)ci * stride;
-  for (int c = 0; c < nc; c++) {
-    double v = (double)U[c * plane + o];
-    if (comp) v -= (double)comp[c * plane + o];
-    aos[k * nc + c] = v;
-  }
+  const unsigned cx = (nx - 1) / stride + 1, cy = (ny - 1) / stride + 1;
+  const unsigned m = blockIdx.x * 256u + threadIdx.x;
+  if (m >= cx * cy * nc) return;
+  const unsigned k = m / nc, c = m - k * nc, cj = k / cx, ci = k - cj * cx;
+  const long o = c * plane + (long)cj * stride * pitch + xoff + (long)ci * stride;
+  double v = (double)U[o];
+  if (comp) v -= (double)comp[o];
+  aos[m] = v;
 }
 
 template <typename T>
