@@ -389,13 +389,10 @@ hipError_t launch_pair_part(sbp_ctx *c, int part, double t, double dt)
   return c->esz == 8 ? launch_pair_part_t<double>(c, part, t, dt) : launch_pair_part_t<float>(c, part, t, dt);
 }
 
-// One whole step (march2d_kernel or step2d_kernel): U -> U' in Y0, which then
-// trade places.
-template <typename T> hipError_t launch_whole_t(sbp_ctx *c, double t, double dt)
+// The grid, fields and parameters that steps on chip take.
+template <typename T> StepArgs<T> step_args_t(const sbp_ctx *c)
 {
   StepArgs<T> a{};
-  a.u = static_cast<const T *>(c->U);
-  a.uo = static_cast<T *>(c->Y0);
   a.comp = static_cast<T *>(c->KC);
   a.rinv = static_cast<const T *>(c->rinv);
   a.bulk = static_cast<const T *>(c->bulk);
@@ -407,8 +404,6 @@ template <typename T> hipError_t launch_whole_t(sbp_ctx *c, double t, double dt)
   a.s3x = c->s3x;
   a.c4y = c->c4y;
   a.s4y = c->s4y;
-  const double ts[3] = {t, t + 0.5 * dt, t + dt};
-  for (int k = 0; k < 3; k++) a.c5[k] = std::cos(5 * kPi * ts[k]);
   a.plane = c->plane;
   a.pitch = c->pitch;
   a.xoff = c->xoff;
@@ -419,6 +414,18 @@ template <typename T> hipError_t launch_whole_t(sbp_ctx *c, double t, double dt)
   a.hiy = T(c->hiy);
   a.ax = T(c->d.ax);
   a.ay = T(c->d.ay);
+  return a;
+}
+
+// One whole step (march2d_kernel or step2d_kernel): U -> U' in Y0, which then
+// trade places.
+template <typename T> hipError_t launch_whole_t(sbp_ctx *c, double t, double dt)
+{
+  StepArgs<T> a = step_args_t<T>(c);
+  a.u = static_cast<const T *>(c->U);
+  a.uo = static_cast<T *>(c->Y0);
+  const double ts[3] = {t, t + 0.5 * dt, t + dt};
+  for (int k = 0; k < 3; k++) a.c5[k] = std::cos(5 * kPi * ts[k]);
   a.c12 = T(0.5 * dt);
   a.c3 = T(dt);
   a.ca = T(dt / 6);
@@ -709,6 +716,7 @@ void release(sbp_ctx *c)
     if (p) (void)hipFree(p);
   for (void *p : c->rkw)
     if (p) (void)hipFree(p);
+  if (c->rk_host) (void)hipHostFree(c->rk_host);
   for (hipEvent_t &e : c->ev)
     if (e) (void)hipEventDestroy(e);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -993,6 +1001,7 @@ hipError_t sbp::host::launch_rhs(sbp_ctx *c, double t, const void *src, void *ds
 {
   return ::launch_stage(c, MODE_RHS, 0.0, t, src, dst);
 }
+StepArgs<double> sbp::host::step_args(const sbp_ctx *c) { return step_args_t<double>(c); }
 void sbp::host::drop_step_graph(sbp_ctx *c) { ::drop_graph(c); }
 
 int sbp::host::energy_of(sbp_ctx *c, const void *u, const void *comp, double *out)

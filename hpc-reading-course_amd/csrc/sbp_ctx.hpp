@@ -39,7 +39,7 @@ struct sbp_ctx {
   // Whole steps in one launch (sbp_step.hpp), in place of either schedule
   // while nobody has chosen one with sbp_set_fused.
   sbp::StepLaunchFn step_launch = nullptr;
-  sbp::StepPlan step_plan{};
+  sbp::StepPlan step_plan{}, rkf_plan{};
   bool whole = false;
   // whole steps march along the grid (sbp_march.hpp)
   sbp::MarchFns march_fns{};
@@ -59,6 +59,7 @@ struct sbp_ctx {
   hipEvent_t ev[5] = {};
   int device = 0;
   void *rkw[8] = {};  // adaptive RK workspace (K1..K6, stage input, candidate), allocated on first use
+  double *rk_host = nullptr;  // sums of squared scaled errors of an attempt (pinned host memory)
 };
 
 
@@ -72,6 +73,8 @@ hipError_t launch_step(sbp_ctx *c, double t, double dt);
 int energy_of(sbp_ctx *c, const void *u, const void *comp, double *out);
 // dst = F(t, src) on planar registers of the context (the RHS stage kernels).
 hipError_t launch_rhs(sbp_ctx *c, double t, const void *src, void *dst);
+// What steps on chip take of an FP64 context.
+StepArgs<double> step_args(const sbp_ctx *c);
 // Forget the captured step graph (after the state register moved).
 void drop_step_graph(sbp_ctx *c);
 }  // namespace host

@@ -11,9 +11,10 @@
 //   MATCHSTEP rule stretches or halves the next step near t_end; more than 10
 //   rejections of one step, or a non-finite enorm, fail with SBP_EDIVERGED.
 //
-// Every attempt is six right-hand-side launches (the RHS mode of the stage
-// kernels) plus combination kernels and one weighted-norm reduction, whose
-// scalar the host reads to decide.  Built without FMA contraction (file
+// An attempt on a small 2D grid is one launch (sbp_rkf.hpp); otherwise six
+// right-hand-side launches (the RHS mode of the stage kernels) plus combination
+// kernels and one weighted-norm reduction.  The host reads the sum of squared
+// scaled errors to decide; the kernels leave it in pinned host memory.  Built without FMA contraction (file
 // suffix _f64) with the oracle's operation order, so the stage values match
 // the CPU restatement bit for bit.
 #include <hip/hip_runtime.h>
@@ -26,6 +27,7 @@
 #include "../../include/sbp_hip.h"
 #include "sbp_ctx.hpp"
 #include "sbp_host.hpp"
+#include "sbp_rkf.hpp"
 #include "sbp_ts.hpp"
 
 using sbp::host::fail;
@@ -33,16 +35,10 @@ using sbp::host::fail;
 
 namespace {
 
-// Fehlberg's coefficients (E. Fehlberg, NASA TR R-315, 1969).
-constexpr double kC[6] = {0.0, 1.0 / 4.0, 3.0 / 8.0, 12.0 / 13.0, 1.0, 1.0 / 2.0};
-constexpr double kA[6][5] = {{0, 0, 0, 0, 0},
-                             {1.0 / 4.0, 0, 0, 0, 0},
-                             {3.0 / 32.0, 9.0 / 32.0, 0, 0, 0},
-                             {1932.0 / 2197.0, -7200.0 / 2197.0, 7296.0 / 2197.0, 0, 0},
-                             {439.0 / 216.0, -8.0, 3680.0 / 513.0, -845.0 / 4104.0, 0},
-                             {-8.0 / 27.0, 2.0, -3544.0 / 2565.0, 1859.0 / 4104.0, -11.0 / 40.0}};
-constexpr double kB5[6] = {16.0 / 135.0, 0.0, 6656.0 / 12825.0, 28561.0 / 56430.0, -9.0 / 50.0, 2.0 / 55.0};
-constexpr double kB4[6] = {25.0 / 216.0, 0.0, 1408.0 / 2565.0, 2197.0 / 4104.0, -1.0 / 5.0, 0.0};
+using sbp::kRkfA;
+using sbp::kRkfB4;
+using sbp::kRkfB5;
+using sbp::kRkfC;
 
 struct Regs {
   const double *K[6];
@@ -112,10 +108,13 @@ __global__ __launch_bounds__(256) void rkf_sum_kernel(const double *__restrict__
   if (threadIdx.x == 0) out[0] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
 
-int ensure_workspace(sbp_ctx *c)
+// The registers an attempt works in: the candidate (the last), and where the
+// stages are launches of their own K1 .. K6 and a stage's operand.
+int ensure_workspace(sbp_ctx *c, bool one_launch)
 {
   const size_t bytes = c->esz * (size_t)c->C * (size_t)c->plane;
-  for (void *&p : c->rkw) {
+  for (int q = one_launch ? 7 : 0; q < 8; q++) {
+    void *&p = c->rkw[q];
     if (p) continue;
     hipError_t e = hipMalloc(&p, bytes);
     if (e != hipSuccess) {
@@ -126,7 +125,21 @@ int ensure_workspace(sbp_ctx *c)
     // become the state register, padding included)
     HIP_OR_FAIL(hipMemsetAsync(p, 0, bytes, c->stream));
   }
+  const int n = std::max(1, c->rkf_plan.px * c->rkf_plan.py);
+  if (!c->rk_host)
+    HIP_OR_FAIL(hipHostMalloc(reinterpret_cast<void **>(&c->rk_host), sizeof(double) * n, hipHostMallocDefault));
   return SBP_OK;
+}
+
+// One launch per attempt where that was measured faster (us per attempt, one
+// launch / thirteen): order 4 201^2 27 / 70, 1025^2 173 / 228, with rho = 2 +
+// xy 226 / 244, 2D advection 82 / 113; order 2 1025^2 78 / 253.  Order 6 loads
+// 64 x 40 points for 28 x 4 and spills: 101^2 32 / 69, 151^2 48 / 71, with rho
+// = 2 + xy 68 / 75 (201^2 97 / 76), 2D advection 27 / 57.
+bool one_launch_default(const sbp_ctx *c)
+{
+  const long most = c->order == 6 ? 160 : 1100;
+  return c->rkf_plan.ok && (long)c->nx * c->ny <= most * most;
 }
 
 }  // namespace
@@ -141,7 +154,14 @@ int sbp_rk45(sbp_ctx *ctx, double t0, double t_end, double dt0, double atol, dou
   if (!ctx->have_state) return fail(SBP_ESTATE, "no state loaded");
   if (!(dt0 > 0) || !(t_end >= t0) || !std::isfinite(t_end) || !(atol > 0) || !(rtol >= 0) || max_steps < 1)
     return fail(SBP_EINVAL, "bad time span, step or tolerance");
-  int rc = ensure_workspace(ctx);
+  sbp::RkfLaunchFn one = nullptr;
+  if (ctx->phys == SBP_ACOUSTIC_2D || ctx->phys == SBP_ADVECTION_2D) {
+    one = (ctx->order == 2 ? sbp::rkf_launcher_o2 : (ctx->order == 4 ? sbp::rkf_launcher_o4 : sbp::rkf_launcher_o6))(
+        ctx->phys, ctx->mat);
+    ctx->rkf_plan = sbp::rkf_plan(ctx->order, ctx->nx, ctx->ny);
+    if (!one_launch_default(ctx)) one = nullptr;
+  }
+  int rc = ensure_workspace(ctx, one != nullptr);
   if (rc) return rc;
   double *K[6], *Y = static_cast<double *>(ctx->rkw[6]), *U5 = static_cast<double *>(ctx->rkw[7]);
   for (int q = 0; q < 6; q++) K[q] = static_cast<double *>(ctx->rkw[q]);
@@ -155,13 +175,24 @@ int sbp_rk45(sbp_ctx *ctx, double t0, double t_end, double dt0, double atol, dou
   r.xoff = ctx->xoff;
   Row b{}, e{};
   for (int q = 0; q < 6; q++) {
-    b.c[q] = kB5[q];
-    e.c[q] = kB5[q] - kB4[q];
+    b.c[q] = kRkfB5[q];
+    e.c[q] = kRkfB5[q] - kRkfB4[q];
   }
   const long npts = (long)ctx->nx * ctx->ny;
   const int pgrid = (int)((npts + 255) / 256);
   const int fgrid = std::min(pgrid, ctx->npartials);
   hipStream_t s = ctx->stream;
+  sbp::RkfArgs ra{};
+  if (one) {
+    ra.g = sbp::host::step_args(ctx);
+    ra.g.px = ctx->rkf_plan.px;
+    ra.g.pw = ctx->rkf_plan.pw;
+    ra.g.ph = ctx->rkf_plan.ph;
+    ra.atol = atol;
+    ra.rtol = rtol;
+    ra.partial = ctx->rk_host;
+  }
+  const int blocks = ctx->rkf_plan.px * ctx->rkf_plan.py;
   namespace ts = sbp::ts;
   // TSSolve: the first step does not overshoot t_end
   double t = t0, h = ts::first_step(t0, dt0, t_end);
@@ -180,21 +211,29 @@ int sbp_rk45(sbp_ctx *ctx, double t0, double t_end, double dt0, double atol, dou
         return fail(SBP_EINVAL, "step budget exhausted before t_end");
       }
       double *U = static_cast<double *>(ctx->U);
-      HIP_OR_FAIL(sbp::host::launch_rhs(ctx, t, U, K[0]));
-      for (int st = 1; st < 6; st++) {
-        Row a{};
-        for (int q = 0; q < st; q++) a.c[q] = kA[st][q];
-        hipLaunchKernelGGL(rkf_stage_kernel, dim3(pgrid), dim3(256), 0, s, r, st, a, h, U, Y);
+      if (one) {
+        ra.g.u = U;
+        ra.g.uo = U5;
+        ra.h = h;
+        for (int st = 0; st < 6; st++) ra.c5[st] = std::cos(5 * sbp::kPi * (t + kRkfC[st] * h));
+        HIP_OR_FAIL(one(ra, blocks, s));
+      } else {
+        HIP_OR_FAIL(sbp::host::launch_rhs(ctx, t, U, K[0]));
+        for (int st = 1; st < 6; st++) {
+          Row a{};
+          for (int q = 0; q < st; q++) a.c[q] = kRkfA[st][q];
+          hipLaunchKernelGGL(rkf_stage_kernel, dim3(pgrid), dim3(256), 0, s, r, st, a, h, U, Y);
+          HIP_OR_FAIL(hipGetLastError());
+          HIP_OR_FAIL(sbp::host::launch_rhs(ctx, t + kRkfC[st] * h, Y, K[st]));
+        }
+        hipLaunchKernelGGL(rkf_finish_kernel, dim3(fgrid), dim3(256), 0, s, r, b, e, h, atol, rtol, U, U5,
+                           ctx->partials);
+        hipLaunchKernelGGL(rkf_sum_kernel, dim3(1), dim3(256), 0, s, ctx->partials, fgrid, ctx->rk_host);
         HIP_OR_FAIL(hipGetLastError());
-        HIP_OR_FAIL(sbp::host::launch_rhs(ctx, t + kC[st] * h, Y, K[st]));
       }
-      hipLaunchKernelGGL(rkf_finish_kernel, dim3(fgrid), dim3(256), 0, s, r, b, e, h, atol, rtol, U, U5,
-                         ctx->partials);
-      hipLaunchKernelGGL(rkf_sum_kernel, dim3(1), dim3(256), 0, s, ctx->partials, fgrid, ctx->scalar);
-      HIP_OR_FAIL(hipGetLastError());
-      double ss = 0;
-      HIP_OR_FAIL(hipMemcpyAsync(&ss, ctx->scalar, sizeof(double), hipMemcpyDeviceToHost, s));
       HIP_OR_FAIL(hipStreamSynchronize(s));
+      double ss = 0;
+      for (int q = 0; q < (one ? blocks : 1); q++) ss += ctx->rk_host[q];
       const double enorm = std::sqrt(ss / (double)(npts * ctx->C));
       if (!std::isfinite(enorm)) {  // TSErrorWeightedNorm: PETSC_ERR_FP
         report();

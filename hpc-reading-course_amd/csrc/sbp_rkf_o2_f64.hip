@@ -1,0 +1,5 @@
+// One-launch RKF4(5) attempts of the order-2 SBP operators (built without FMA contraction).
+#include "sbp_rkf.hpp"
+namespace sbp {
+RkfLaunchFn rkf_launcher_o2(int phys, int mat) { return pick_rkf<2>(phys, mat); }
+}  // namespace sbp

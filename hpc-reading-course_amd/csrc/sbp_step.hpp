@@ -51,92 +51,81 @@ template <int ORDER> __host__ __device__ inline void stencil_reach(int &lo, int 
   hi = l && G::TAPS > b ? G::TAPS : b;
 }
 
-// The step on columns [i0, i1) and rows [j0, j1), by a block of NW waves
-// whose patches load at most H rows.  TR: "columns" and "rows" are the grid's rows and columns (a narrow
-// strip along the left or right boundary fills the lanes that way; it must
-// not reach the closure rows at the lanes' ends).
-template <typename T, int ORDER, int PHYS, int MAT, bool KAHAN, bool TR, int NW, int H>
-__device__ __forceinline__ void step_patch(const StepArgs<T> &a, T *s_, int i0, int i1, int j0, int j1)
-{
+// A patch of the grid in a block's LDS array s_: columns [i0, i1) and rows
+// [j0, j1), for a method of NST stages, by NW waves, at most H rows loaded.
+// TR: "columns" and "rows" are the grid's rows and columns (a narrow strip
+// along the left or right boundary fills the lanes that way; it must not reach
+// the closure rows at the lanes' ends).
+template <typename T, int ORDER, int PHYS, int MAT, bool TR, int NW, int H, int NST> struct Patch {
   using G = Geom<ORDER>;
-  constexpr int R = G::R, CLS = G::CLS, TAPS = G::TAPS, KR = H / NW;
-  constexpr bool AC = PHYS == PH_ACOUSTIC;
-  constexpr int C = AC ? 3 : 1;
-  constexpr int FS = H * kStepLanes, BS = C * FS;  // strides of a field and of a buffer of the LDS array s_
+  static constexpr int R = G::R, CLS = G::CLS, TAPS = G::TAPS, KR = H / NW;
+  static constexpr bool AC = PHYS == PH_ACOUSTIC;
+  static constexpr int C = AC ? 3 : 1;
+  static constexpr int FS = H * kStepLanes, BS = C * FS;  // strides of a field and of a buffer of the LDS array
   static_assert(H % NW == 0 && 2 * BS + 2 * R == step_lds(ORDER, C, H), "rows and LDS of a patch");
-  T *const s = s_ + R;  // a lane's x taps may reach R slots outside its row: garbage that no used value depends on
-
   static_assert(!TR || MAT != M_REF, "the forcing's tables are per grid column");
-  const int nx = TR ? a.ny : a.nx, ny = TR ? a.nx : a.ny;
-  const T hl = TR ? a.hiy : a.hix, hr = TR ? a.hix : a.hiy;  // of the lane and row axes
-  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // regions evaluated in stages 1 .. 4 ([4]: the patch), and loaded ([0])
-  int xl[5], xh[5], yl[5], yh[5];
-  xl[4] = i0, xh[4] = i1, yl[4] = j0, yh[4] = j1;
-#pragma unroll
-  for (int k = 3; k >= 0; k--) {
-    xl[k] = xl[k + 1], xh[k] = xh[k + 1], yl[k] = yl[k + 1], yh[k] = yh[k + 1];
-    stencil_reach<ORDER>(xl[k], xh[k], nx);
-    stencil_reach<ORDER>(yl[k], yh[k], ny);
-  }
-  const bool xedge = xl[1] < CLS || xh[1] > nx - CLS;  // closure columns among the region's
-  const bool yedge = yl[1] < CLS || yh[1] > ny - CLS;
 
-  const int i = min(xl[0] + lane, xh[0] - 1);
-  // offset of this lane's point of row j
-  auto at = [&](int j) { return TR ? (long)i * a.pitch + a.xoff + j : (long)j * a.pitch + a.xoff + i; };
-  // x taps of this lane: closure columns read a table row from their end of
-  // the line; interior ones the interior row, whose padding taps re-read the
-  // centre (a point that is certainly valid) with coefficient zero
+  const StepArgs<T> &a;
+  T *const s;  // a lane's x taps may reach R slots outside its row: garbage that no used value depends on
+  const int nx, ny;
+  const T hl, hr;  // of the lane and row axes
+  const int lane, wv;
+  int xl[NST + 1], xh[NST + 1], yl[NST + 1], yh[NST + 1];  // regions evaluated in stages 1 .. NST ([NST]: the patch), and loaded ([0])
+  bool xedge, yedge;  // closure columns (rows) among the region's
+  int i;
   T cf[TAPS];
-  int xt = lane - R, xpad = lane;
-  if (xedge) {
-    const bool lo = i < CLS, hi = i >= nx - CLS;
-    const int row = lo ? i : (hi ? CLS + (nx - 1 - i) : 2 * CLS);
+  int xt, xpad;
+  double xc = 0, c3c = 0, s3c = 0;
+
+  __device__ __forceinline__ Patch(const StepArgs<T> &args, T *s_, int i0, int i1, int j0, int j1)
+      : a(args), s(s_ + R), nx(TR ? args.ny : args.nx), ny(TR ? args.nx : args.ny), hl(TR ? args.hiy : args.hix),
+        hr(TR ? args.hix : args.hiy), lane(threadIdx.x & 63), wv(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6))
+  {
+    xl[NST] = i0, xh[NST] = i1, yl[NST] = j0, yh[NST] = j1;
 #pragma unroll
-    for (int t = 0; t < TAPS; t++) cf[t] = c_edge<T, ORDER>.c[row][t];
-    if (lo || hi) {
-      xt = min(max((lo ? 0 : nx - TAPS) - xl[0], 0), kStepLanes - TAPS);
-      xpad = -1;
+    for (int k = NST - 1; k >= 0; k--) {
+      xl[k] = xl[k + 1], xh[k] = xh[k + 1], yl[k] = yl[k + 1], yh[k] = yh[k + 1];
+      stencil_reach<ORDER>(xl[k], xh[k], nx);
+      stencil_reach<ORDER>(yl[k], yh[k], ny);
+    }
+    xedge = xl[1] < CLS || xh[1] > nx - CLS;
+    yedge = yl[1] < CLS || yh[1] > ny - CLS;
+    i = min(xl[0] + lane, xh[0] - 1);
+    // x taps of this lane: closure columns read a table row from their end of
+    // the line; interior ones the interior row, whose padding taps re-read the
+    // centre (a point that is certainly valid) with coefficient zero
+    xt = lane - R, xpad = lane;
+    if (xedge) {
+      const bool lo = i < CLS, hi = i >= nx - CLS;
+      const int row = lo ? i : (hi ? CLS + (nx - 1 - i) : 2 * CLS);
+#pragma unroll
+      for (int t = 0; t < TAPS; t++) cf[t] = c_edge<T, ORDER>.c[row][t];
+      if (lo || hi) {
+        xt = min(max((lo ? 0 : nx - TAPS) - xl[0], 0), kStepLanes - TAPS);
+        xpad = -1;
+      }
+    }
+    if constexpr (MAT == M_REF) {
+      xc = a.xs[i];
+      c3c = a.c3x[i];
+      s3c = a.s3x[i];
     }
   }
 
-  T U[KR][C], P[KR][C], Y[KR][C], ri[KR], Kb[KR], cmp[KR][C];
-  double xc = 0, c3c = 0, s3c = 0;
-  if constexpr (MAT == M_REF) {
-    xc = a.xs[i];
-    c3c = a.c3x[i];
-    s3c = a.s3x[i];
+  // grid row of region row r (clamped: rows past the region repeat its last)
+  __device__ __forceinline__ int row(int k) const { return min(yl[0] + wv + NW * k, yh[0] - 1); }
+  // offset of this lane's point of row j
+  __device__ __forceinline__ long at(int j) const
+  {
+    return TR ? (long)i * a.pitch + a.xoff + j : (long)j * a.pitch + a.xoff + i;
   }
-#pragma unroll
-  for (int k = 0; k < KR; k++) {
-    const int j = min(yl[0] + wv + NW * k, yh[0] - 1);
-    const long o = at(j);
-#pragma unroll
-    for (int c = 0; c < C; c++) U[k][c] = a.u[c * a.plane + o];
-    ri[k] = Kb[k] = T(1);
-    if constexpr (MAT == M_ARR) {
-      ri[k] = (AC ? a.rinv : a.velx)[o];
-      Kb[k] = (AC ? a.bulk : a.vely)[o];
-    }
-    if constexpr (KAHAN) {
-#pragma unroll
-      for (int c = 0; c < C; c++) cmp[k][c] = a.comp[c * a.plane + o];
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < KR; k++)
-#pragma unroll
-    for (int c = 0; c < C; c++) {
-      Y[k][c] = U[k][c];
-      P[k][c] = T(0);
-      s[c * FS + (wv + NW * k) * kStepLanes + lane] = U[k][c];
-    }
-  __syncthreads();
+  __device__ __forceinline__ bool own() const { return xl[0] + lane >= xl[NST] && xl[0] + lane < xh[NST]; }
+  __device__ __forceinline__ T *slot(int b, int r) const { return s + b * BS + r * kStepLanes + lane; }
 
   // Right-hand side at row j = region row r of buffer b, centre values Yc.
-  auto rhs = [&](auto XE, int b, int r, int j, const T *Yc, T rik, T Kk, double c5, T *K) {
-    constexpr bool xe = decltype(XE)::value;
+  template <bool xe>
+  __device__ __forceinline__ void rhs(int b, int r, int j, const T *Yc, T rik, T Kk, double c5, T *K) const
+  {
     constexpr int NX = xe ? TAPS : 2 * R + 1;
     const T *f = s + b * BS, *fp = AC ? f + 2 * FS : f;
     // u differentiated in x, v in y, p in both
@@ -144,7 +133,8 @@ __device__ __forceinline__ void step_patch(const StepArgs<T> &a, T *s_, int i0, 
     const bool yc = yedge && (j < CLS || j >= ny - CLS);  // closure row
     const int ry = yc ? (j < CLS ? 0 : ny - TAPS) - yl[0] : r - R;
     const T *py = fp + ry * kStepLanes + lane, *vy = f + (TR ? 0 : FS) + ry * kStepLanes + lane;
-    T ax[NX], bx[NX], ay[TAPS], by[TAPS];  // p (or the one field) and u / v along the lanes; p and v / u across
+    // p (or the one field) and u / v along the lanes; p and v / u across
+    T ax[NX], bx[NX], ay[TAPS], by[TAPS];
 #pragma unroll
     for (int t = 0; t < NX; t++) {
       const int q = xe ? (t < 2 * R + 1 || xpad < 0 ? xt + t : xpad) : lane - R + t;
@@ -226,34 +216,67 @@ __device__ __forceinline__ void step_patch(const StepArgs<T> &a, T *s_, int i0, 
       }
       K[0] = k;
     }
-  };
+  }
+};
+
+// The RK4 step of a patch.
+template <typename T, int ORDER, int PHYS, int MAT, bool KAHAN, bool TR, int NW, int H>
+__device__ __forceinline__ void step_patch(const StepArgs<T> &a, T *s_, int i0, int i1, int j0, int j1)
+{
+  using Pt = Patch<T, ORDER, PHYS, MAT, TR, NW, H, 4>;
+  constexpr int KR = Pt::KR, C = Pt::C;
+  constexpr bool AC = Pt::AC;
+  const Pt pt(a, s_, i0, i1, j0, j1);
+
+  T U[KR][C], P[KR][C], Y[KR][C], ri[KR], Kb[KR], cmp[KR][C];
+#pragma unroll
+  for (int k = 0; k < KR; k++) {
+    const long o = pt.at(pt.row(k));
+#pragma unroll
+    for (int c = 0; c < C; c++) U[k][c] = a.u[c * a.plane + o];
+    ri[k] = Kb[k] = T(1);
+    if constexpr (MAT == M_ARR) {
+      ri[k] = (AC ? a.rinv : a.velx)[o];
+      Kb[k] = (AC ? a.bulk : a.vely)[o];
+    }
+    if constexpr (KAHAN) {
+#pragma unroll
+      for (int c = 0; c < C; c++) cmp[k][c] = a.comp[c * a.plane + o];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < KR; k++)
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+      Y[k][c] = U[k][c];
+      P[k][c] = T(0);
+      pt.slot(0, pt.wv + NW * k)[c * Pt::FS] = U[k][c];
+    }
+  __syncthreads();
 
   // (unrolled: fewer registers, so two blocks per CU; 513^2 18.9 against 27 us)
   auto stages = [&](auto XE) {
-    const int y1l = yl[1], y1h = yh[1], y2l = yl[2], y2h = yh[2], y3l = yl[3], y3h = yh[3];
 #pragma unroll
     for (int st = 1; st <= 4; st++) {
       const int b = (st - 1) & 1;
       const double c5 = st == 1 ? a.c5[0] : (st == 4 ? a.c5[2] : a.c5[1]);
       const T cy = st == 3 ? a.c3 : a.c12, w = st == 2 ? T(2) : T(1);
-      const int ylo = st == 1 ? y1l : (st == 2 ? y2l : (st == 3 ? y3l : j0));
-      const int yhi = st == 1 ? y1h : (st == 2 ? y2h : (st == 3 ? y3h : j1));
 #pragma unroll
       for (int k = 0; k < KR; k++) {
-        const int r = wv + NW * k, j = yl[0] + r;
-        if (j < ylo || j >= yhi) continue;  // (the whole wave)
+        const int r = pt.wv + NW * k, j = pt.yl[0] + r;
+        if (j < pt.yl[st] || j >= pt.yh[st]) continue;  // (the whole wave)
         T K[C];
-        rhs(XE, b, r, j, Y[k], ri[k], Kb[k], c5, K);
+        pt.template rhs<decltype(XE)::value>(b, r, j, Y[k], ri[k], Kb[k], c5, K);
         if (st < 4) {
 #pragma unroll
           for (int c = 0; c < C; c++) {
             const T y = mad(cy, K[c], U[k][c]);
             P[k][c] = P[k][c] + w * (y - U[k][c]);  // exact products: Y2-U, + 2 (Y3-U), + (Y4-U)
             Y[k][c] = y;
-            s[(b ^ 1) * BS + c * FS + r * kStepLanes + lane] = y;
+            pt.slot(b ^ 1, r)[c * Pt::FS] = y;
           }
-        } else if (xl[0] + lane >= i0 && xl[0] + lane < i1) {
-          const long o = at(j);
+        } else if (pt.own()) {
+          const long o = pt.at(j);
 #pragma unroll
           for (int c = 0; c < C; c++) {
             const T inc = mad(P[k][c], a.third, a.ca * K[c]);
@@ -271,7 +294,7 @@ __device__ __forceinline__ void step_patch(const StepArgs<T> &a, T *s_, int i0, 
       __syncthreads();
     }
   };
-  if (!TR && xedge) stages(std::integral_constant<bool, !TR>{});
+  if (!TR && pt.xedge) stages(std::integral_constant<bool, !TR>{});
   else stages(std::false_type{});
 }
 
@@ -294,15 +317,15 @@ struct StepPlan {
   bool ok;
   int px, pw, py, ph;
 };
-template <int ORDER> inline StepPlan step_plan_t(int nx, int ny)
+// stages of the method, most rows a block loads, most rows of a patch
+template <int ORDER> inline StepPlan patch_plan(int nx, int ny, int stages, int rows, int most)
 {
-  constexpr int rows = kStepWaves * step_rows(ORDER);
-  // parts of `len` points of a line of n whose four-stage regions hold at most `most`
-  auto fits = [](int n, int len, int most) {
+  // parts of `len` points of a line of n whose regions hold at most `cap`
+  auto fits = [=](int n, int len, int cap) {
     for (int p = 0; p < n; p += len) {
       int lo = p, hi = p + len < n ? p + len : n;
-      for (int k = 0; k < 4; k++) stencil_reach<ORDER>(lo, hi, n);
-      if (hi - lo > most) return false;
+      for (int k = 0; k < stages; k++) stencil_reach<ORDER>(lo, hi, n);
+      if (hi - lo > cap) return false;
     }
     return true;
   };
@@ -316,7 +339,7 @@ template <int ORDER> inline StepPlan step_plan_t(int nx, int ny)
   p.px = (nx + p.pw - 1) / p.pw;
   constexpr int kCus = 256;
   int best = 0;
-  for (p.ph = 1; p.ph <= 8; p.ph++) {
+  for (p.ph = 1; p.ph <= most; p.ph++) {
     if (!fits(ny, p.ph, rows)) continue;
     best = p.ph;
     if ((long)p.px * ((ny + p.ph - 1) / p.ph) <= kCus) break;
@@ -326,6 +349,10 @@ template <int ORDER> inline StepPlan step_plan_t(int nx, int ny)
   p.py = (ny + p.ph - 1) / p.ph;
   p.ok = true;
   return p;
+}
+template <int ORDER> inline StepPlan step_plan_t(int nx, int ny)
+{
+  return patch_plan<ORDER>(nx, ny, 4, kStepWaves * step_rows(ORDER), 8);
 }
 inline StepPlan step_plan(int order, int nx, int ny)
 {
