@@ -168,8 +168,8 @@ bool step_default(const sbp_ctx *c)
 
 // Marched steps (sbp_march.hpp) replace both from the sizes where their lead-in
 // and frame cost less than the passes they save (us per step, march / before):
-// order 4 FP64 301^2 12.8 / 11.5, 401^2 13.2 / 15.4, 1025^2 30.8 / 47.5, 4097^2
-// 251 / 452; FP32 401^2 10.1 / 9.7, 513^2 11.9 / 14.2, 4097^2 121 / 236; order 2
+// order 4 FP64 301^2 12.8 / 11.5, 401^2 13.2 / 15.4, 1025^2 27.1 / 47.5, 4097^2
+// 226 / 452; FP32 401^2 10.1 / 9.7, 513^2 11.9 / 14.2, 4097^2 121 / 236; order 2
 // FP64 201^2 6.3 / 5.8, 257^2 6.5 / 7.3; order 6 FP64 301^2 21.9 / 20.1, 513^2
 // 30.3 / 36.7, FP32 301^2 15.2 / 17.2.  Ribbons leave most of a strip's columns
 // or rows to the lead-in: 64 x 4096 31.7 / 16.1, 2048 x 128 19.1 / 17.8, 128 x

@@ -22,12 +22,15 @@
 // every stage is an interior point of the operator; the D-deep frame is cut
 // into patches that blocks of the same launch step on chip (sbp_step.hpp).
 //
-// What bounds it: order 4 FP64, 4097^2, takes 251 us per step (452 as two
-// launches): 806 MB of U and U' are 147 us at what a copy reaches, the 200
-// vector instructions per row and wave 120 us of every SIMD, the halo columns
-// and lead-in rows a quarter more of those.  Small grids wait for the lead-in
-// and the frame (1025^2 30.8 us, 47.5 before).  FP32 4097^2 121 (236), order 6
-// FP32 + compensation with rho/K arrays 272 (442), order 6 FP64 416 (570: its
+// What bounds it: order 4 FP64, 4097^2, takes 226 us per step (452 as two
+// launches).  806 MB of U and U' are 147 us at what a copy reaches; a row costs
+// a CU's LDS 0.6 us for the neighbours (32 words read and 8 written per column)
+// and its SIMDs 0.8 us for 200 instructions, which the barrier of each row lets
+// overlap in part; halo columns and lead-in rows add a fifth.  Constant LDS
+// addresses (15 instructions less per row, at a longer unrolling) and more rows
+// of loads in flight (3, 4) gain nothing.  Small grids wait for the lead-in
+// and the frame (1025^2 27 us, 47.5 before).  FP32 4097^2 117 (236), order 6
+// FP32 + compensation with rho/K arrays 272 (442), order 6 FP64 413 (570: its
 // rings fill the register file, one wave per SIMD).  Stores are cached: 2049^2
 // FP64 74.6 us, 78.5 nontemporal, and the next step reads them.  A version
 // whose waves exchange columns through DPP alone, with no LDS and no barrier,
@@ -68,9 +71,15 @@ template <typename T, int WN, int N> struct LaneRing<T, WN, N, true> {
   template <int S> __device__ __forceinline__ void set(int c, T x) { p[(S * N + c) * kMarchThreads] = x; }
 };
 
-// Whether the ring S lives in LDS: FP64 acoustics of order 4 and 6 would need
-// more than 256 registers with it (order 4: 188 without, so two waves per SIMD).
-constexpr bool march_s_lds(int esz, int order, bool acoustic) { return esz == 8 && acoustic && order >= 4; }
+// Whether the ring S lives in LDS: where FP64 acoustics would need more than
+// 256 registers with it, two waves per SIMD (order 4 with arrays; 39 us per step
+// at 1025^2 in registers, 33 in LDS) or all the more of the second half of the
+// file (order 6).  LDS is the scarcer where they suffice: order 4 without
+// arrays 27.1 / 30.2 us at 1025^2, 67 / 74 at 2049^2, 226 / 236 at 4097^2.
+constexpr bool march_s_lds(int esz, int order, bool acoustic, bool arrays)
+{
+  return esz == 8 && acoustic && (order == 6 || (order == 4 && arrays));
+}
 // LDS values per block of that ring, and of the exchanged rows: R+1 slots of
 // the differentiated fields of the four operands, R columns beyond either end
 constexpr int march_ring(int order, int comps) { return comps * (order + 1) * kMarchThreads; }
@@ -97,7 +106,7 @@ __device__ __forceinline__ void march_strip(const StepArgs<T> &a, T *lds, int st
   T *const x = lds + R + t;  // this thread's column of the exchanged rows
 
   T U1[WN][C], U2[WN][C], Y2[WN][C], Y3[WN][C], Y4[WN][C], q[WN][C];
-  LaneRing<T, WN, C, march_s_lds(sizeof(T), ORDER, AC)> S(lds + march_rows(ORDER, C) + t);
+  LaneRing<T, WN, C, march_s_lds(sizeof(T), ORDER, AC, LD_M)> S(lds + march_rows(ORDER, C) + t);
   // materials (or velocities) of rows r-R .. r-3R, and of r-3R .. r-4R
   T M1[WN][2], M2[WN][2];
   T qr[WN], qk[WN], qc[WN][C];
@@ -261,9 +270,10 @@ __device__ __forceinline__ void march_frame_patch(const StepArgs<T> &a, T *s, in
 }
 
 // values of a block's LDS: a marching block's, or a frame patch's
-template <typename T> constexpr int march_block_lds(int order, int comps)
+template <typename T> constexpr int march_block_lds(int order, int comps, bool arrays)
 {
-  const int m = march_rows(order, comps) + (march_s_lds(sizeof(T), order, comps == 3) ? march_ring(order, comps) : 0);
+  const int m =
+      march_rows(order, comps) + (march_s_lds(sizeof(T), order, comps == 3, arrays) ? march_ring(order, comps) : 0);
   const int f = step_lds(order, comps, march_frame_rows(order));
   return m > f ? m : f;
 }
@@ -272,7 +282,7 @@ template <typename T, int ORDER, int PHYS, int MAT, bool KAHAN>
 __global__ __launch_bounds__(kMarchThreads) void march2d_kernel(StepArgs<T> a, int frame)
 {
   constexpr int D = march_depth(ORDER), NC = PHYS == PH_ACOUSTIC ? 3 : 1;
-  __shared__ T lds[march_block_lds<T>(ORDER, NC)];
+  __shared__ T lds[march_block_lds<T>(ORDER, NC, MAT == M_ARR)];
   if ((int)blockIdx.x < frame) {
     march_frame_patch<T, ORDER, PHYS, MAT, KAHAN>(a, lds, blockIdx.x);
     return;
@@ -327,7 +337,7 @@ __global__ __launch_bounds__(kMarchThreads) void batch_march_kernel(const BatchI
                                                                    const int2 *__restrict__ work)
 {
   constexpr int D = march_depth(ORDER);
-  __shared__ T lds[march_block_lds<T>(ORDER, 3)];
+  __shared__ T lds[march_block_lds<T>(ORDER, 3, MAT == M_ARR)];
   const int2 chunk = work[blockIdx.x % kNumXcd];
   const int w = blockIdx.x / kNumXcd;
   if (w >= chunk.y) return;

@@ -378,7 +378,7 @@ __host__ __device__ inline int march_frame(int order, int px, int ny)
 // / 45, 1025^2 21 / 17 / 17 / 19): as many blocks per CU, at most `resident`,
 // as make (rows + lead) (1 + w / 4) smallest.  A frame of few patches takes
 // its place within them, so that all blocks of a launch run at once (1025^2
-// FP64: 31 us per step, 36 with another 88 blocks to wait for); a larger one is
+// FP64: 31 us per step, 36 with another 88 blocks to wait for; both with S in LDS); a larger one is
 // worth a longer launch (4097^2 FP64 255 / 288).
 struct MarchPlan {
   bool ok;
