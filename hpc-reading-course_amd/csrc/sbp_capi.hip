@@ -18,6 +18,7 @@
 #include "../../include/sbp_hip.h"
 #include "sbp_ctx.hpp"
 #include "sbp_host.hpp"
+#include "sbp_rhs.hpp"
 #include "sbp_kernels.hpp"
 #include "sbp_ts.hpp"
 
@@ -442,6 +443,18 @@ template <typename T> hipError_t launch_whole_t(sbp_ctx *c, double t, double dt)
   return e;
 }
 
+// The right-hand side of the vector in aos, to rhs_out.
+hipError_t launch_rhs_host(sbp_ctx *c, double t)
+{
+  auto go = [&](auto a) {
+    a.px = c->rhs_plan.px;
+    a.pw = c->rhs_plan.pw;
+    a.ph = c->rhs_plan.ph;
+    return c->rhs_launch(&a, std::cos(5 * kPi * t), c->aos, c->rhs_out, c->rhs_plan.px * c->rhs_plan.py, c->stream);
+  };
+  return c->esz == 8 ? go(step_args_t<double>(c)) : go(step_args_t<float>(c));
+}
+
 hipError_t launch_step(sbp_ctx *c, double t, double dt)
 {
   if (is1d(c->phys)) {
@@ -717,6 +730,7 @@ void release(sbp_ctx *c)
   for (void *p : c->rkw)
     if (p) (void)hipFree(p);
   if (c->rk_host) (void)hipHostFree(c->rk_host);
+  if (c->rhs_out) (void)hipHostFree(c->rhs_out);
   for (hipEvent_t &e : c->ev)
     if (e) (void)hipEventDestroy(e);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -831,6 +845,17 @@ int build_ctx(const sbp_problem *desc, sbp_ctx *c)
     if ((rc = dalloc(&c->aos, aos_bytes))) return rc;
   } else {
     HIP_OR_FAIL(hipHostMalloc(reinterpret_cast<void **>(&c->aos), aos_bytes, hipHostMallocDefault));
+    if (!is1d(c->phys)) {
+      c->rhs_plan = rhs_plan(c->order, c->nx, c->ny);
+      if (c->rhs_plan.ok) {
+        RhsLaunchFn (*reg)(int, int) =
+            c->esz == 8 ? (c->order == 2 ? rhs_launcher_o2_f64 : (c->order == 4 ? rhs_launcher_o4_f64 : rhs_launcher_o6_f64))
+                        : (c->order == 2 ? rhs_launcher_o2_f32 : (c->order == 4 ? rhs_launcher_o4_f32 : rhs_launcher_o6_f32));
+        c->rhs_launch = reg(c->phys, c->mat);
+      }
+    }
+    if (c->rhs_launch)
+      HIP_OR_FAIL(hipHostMalloc(reinterpret_cast<void **>(&c->rhs_out), aos_bytes, hipHostMallocDefault));
   }
   c->npartials = 1024;
   if ((rc = dalloc(&c->partials, sizeof(double) * c->npartials)) || (rc = dalloc(&c->scalar, 2 * sizeof(double))))
@@ -1152,6 +1177,13 @@ int sbp_rhs(sbp_ctx *ctx, double t, const double *src, double *dst)
 {
   if (!ctx || !src || !dst) return fail(SBP_EINVAL, "null argument");
   int rc;
+  if (ctx->rhs_launch) {
+    if ((rc = upload_aos(ctx, src))) return rc;
+    HIP_OR_FAIL(launch_rhs_host(ctx, t));
+    HIP_OR_FAIL(hipStreamSynchronize(ctx->stream));
+    std::memcpy(dst, ctx->rhs_out, sizeof(double) * (size_t)ctx->C * ctx->nx * ctx->ny);
+    return SBP_OK;
+  }
   if ((rc = upload_aos(ctx, src)) || (rc = aos_to_planar(ctx, ctx->Y1, nullptr))) return rc;
   HIP_OR_FAIL(launch_stage(ctx, MODE_RHS, 0.0, t, ctx->Y1, ctx->Y0));
   if ((rc = planar_to_aos(ctx, ctx->Y0, nullptr))) return rc;

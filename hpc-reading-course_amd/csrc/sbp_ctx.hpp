@@ -40,6 +40,10 @@ struct sbp_ctx {
   // while nobody has chosen one with sbp_set_fused.
   sbp::StepLaunchFn step_launch = nullptr;
   sbp::StepPlan step_plan{}, rkf_plan{};
+  // one right-hand side of vectors in host memory in one launch (sbp_rhs.hpp)
+  sbp::RhsLaunchFn rhs_launch = nullptr;
+  sbp::StepPlan rhs_plan{};
+  double *rhs_out = nullptr;  // its result (pinned host memory)
   bool whole = false;
   // whole steps march along the grid (sbp_march.hpp)
   sbp::MarchFns march_fns{};

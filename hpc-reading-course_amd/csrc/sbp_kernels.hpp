@@ -1513,6 +1513,16 @@ StepLaunchFn step_launcher_o6_f64(int phys, int mat);
 StepLaunchFn step_launcher_o2_f32(int phys, int mat, bool kahan);
 StepLaunchFn step_launcher_o4_f32(int phys, int mat, bool kahan);
 StepLaunchFn step_launcher_o6_f32(int phys, int mat, bool kahan);
+// Right-hand sides on vectors in host memory (sbp_rhs.hpp; nullptr where none
+// is built): cos(5 pi t), the vectors, blocks.
+using RhsLaunchFn = hipError_t (*)(const void *args, double c5, const double *in, double *out, int grid, hipStream_t s);
+RhsLaunchFn rhs_launcher_o2_f64(int phys, int mat);
+RhsLaunchFn rhs_launcher_o4_f64(int phys, int mat);
+RhsLaunchFn rhs_launcher_o6_f64(int phys, int mat);
+RhsLaunchFn rhs_launcher_o2_f32(int phys, int mat);
+RhsLaunchFn rhs_launcher_o4_f32(int phys, int mat);
+RhsLaunchFn rhs_launcher_o6_f32(int phys, int mat);
+
 // Marched whole steps (sbp_march.hpp; null where none is built): launch, and the
 // blocks a CU holds.
 struct MarchFns {

@@ -125,7 +125,7 @@ __global__ __launch_bounds__(64 * kStepWaves) void rkf_patch_kernel(RkfArgs ra)
 // an attempt's patches
 template <int ORDER> inline StepPlan rkf_plan_t(int nx, int ny)
 {
-  return patch_plan<ORDER>(nx, ny, 6, kStepWaves * rkf_rows(ORDER), 20);
+  return patch_plan<ORDER>(nx, ny, 6, kStepWaves * rkf_rows(ORDER), 1, 20);
 }
 inline StepPlan rkf_plan(int order, int nx, int ny)
 {

@@ -317,8 +317,8 @@ struct StepPlan {
   bool ok;
   int px, pw, py, ph;
 };
-// stages of the method, most rows a block loads, most rows of a patch
-template <int ORDER> inline StepPlan patch_plan(int nx, int ny, int stages, int rows, int most)
+// stages of the method, most rows a block loads, least and most rows of a patch
+template <int ORDER> inline StepPlan patch_plan(int nx, int ny, int stages, int rows, int least, int most)
 {
   // parts of `len` points of a line of n whose regions hold at most `cap`
   auto fits = [=](int n, int len, int cap) {
@@ -339,7 +339,7 @@ template <int ORDER> inline StepPlan patch_plan(int nx, int ny, int stages, int 
   p.px = (nx + p.pw - 1) / p.pw;
   constexpr int kCus = 256;
   int best = 0;
-  for (p.ph = 1; p.ph <= most; p.ph++) {
+  for (p.ph = least; p.ph <= most; p.ph++) {
     if (!fits(ny, p.ph, rows)) continue;
     best = p.ph;
     if ((long)p.px * ((ny + p.ph - 1) / p.ph) <= kCus) break;
@@ -352,7 +352,7 @@ template <int ORDER> inline StepPlan patch_plan(int nx, int ny, int stages, int 
 }
 template <int ORDER> inline StepPlan step_plan_t(int nx, int ny)
 {
-  return patch_plan<ORDER>(nx, ny, 4, kStepWaves * step_rows(ORDER), 8);
+  return patch_plan<ORDER>(nx, ny, 4, kStepWaves * step_rows(ORDER), 1, 8);
 }
 inline StepPlan step_plan(int order, int nx, int ny)
 {
