@@ -254,15 +254,33 @@ struct NetEnergyArgs {
   int order, band;
 };
 
-// Blocks of fused_net_kernel per image and the rows of each block's chunk.
-inline int net_chunk_rows(int H)
+// Rows of each block's chunk (at most FUSED_MAX_ROWS, chunks as even as
+// possible) and the blocks, for nb images.  A block runs its rows and
+// FUSED_HALO more in whole groups of six steps; a step takes 0.55 us where a CU
+// has one block and 0.43 us per block where it has more.  The split of the
+// least total is taken: tall chunks for many images, low ones that spread a few
+// over the chip (64 corrected steps of one 257^2 image 4.2 ms with chunks of 29
+// rows, 3.1 with 6; a training step of one 172 and 142 us).
+inline int net_chunk_rows(int nb, int H, int W)
 {
-  const int nchunks = (H + FUSED_MAX_ROWS - 1) / FUSED_MAX_ROWS;  // at most FUSED_MAX_ROWS rows, chunks as even as possible
-  return (H + nchunks - 1) / nchunks;
+  constexpr int kCus = 256;
+  const long strips = (long)nb * ((W + FOUT - 1) / FOUT);
+  int best = 1;
+  double least = 1e300;
+  for (int n = (H + FUSED_MAX_ROWS - 1) / FUSED_MAX_ROWS; n <= H; n++) {
+    const int rows = (H + n - 1) / n;
+    const long blocks = strips * ((H + rows - 1) / rows);
+    const double cost = (rows + FUSED_HALO + 5) / 6 * 6 * std::max(0.55, 0.43 * (double)((blocks + kCus - 1) / kCus));
+    if (cost < least) {
+      least = cost;
+      best = rows;
+    }
+  }
+  return best;
 }
-inline long net_blocks_per_image(int H, int W)
+inline long net_blocks_per_image(int nb, int H, int W)
 {
-  const int rows = net_chunk_rows(H);
+  const int rows = net_chunk_rows(nb, H, W);
   return (long)((W + FOUT - 1) / FOUT) * ((H + rows - 1) / rows);
 }
 
@@ -271,7 +289,7 @@ inline long net_blocks_per_image(int H, int W)
 // training forward; each block its own rows and 58 columns): 78 us for 16
 // images of 257^2 against 289 us for one convolution launch per layer.
 template <typename T, bool KEEP>
-__global__ __launch_bounds__(256) void fused_net_kernel(const bf16 *__restrict__ X, int nimg, int H, int W, int rows,
+__global__ __launch_bounds__(256, 3) void fused_net_kernel(const bf16 *__restrict__ X, int nimg, int H, int W, int rows,
                                                         const bf16 *__restrict__ w1, const float *__restrict__ b1,
                                                         const bf16 *__restrict__ w2, const float *__restrict__ b2,
                                                         const bf16 *__restrict__ w3, const float *__restrict__ b3,
@@ -349,8 +367,8 @@ __global__ __launch_bounds__(256) void fused_net_kernel(const bf16 *__restrict__
 
   // Step t with ring slot P = t % 2: X completes its rows, Y is one row
   // behind, Z starts.
-  auto step = [&](int t, auto P, FusedRows &Xr, FusedRows &Yr, FusedRows &Zr) {
-    constexpr int ws = decltype(P)::value, rs = ws ^ 1;
+  auto step = [&](auto SEGS, int t, auto P, FusedRows &Xr, FusedRows &Yr, FusedRows &Zr) {
+    constexpr int nu = decltype(SEGS)::value, ws = decltype(P)::value, rs = ws ^ 1;
     // input row y0 - 3 + t -> slot ws, and the load of the row of step t + 2
     if (threadIdx.x < FIN_PARTS) {
       const int ri = y0 - 3 + t;
@@ -359,11 +377,16 @@ __global__ __launch_bounds__(256) void fused_net_kernel(const bf16 *__restrict__
     }
     in_q[ws] = load_in(y0 - 1 + t);
     // layer 1: input rows y0-3 .. y1+2 (steps 1 .. rows+6); completes row y0-5+t
-    if (t >= 1 && t <= nsteps - 3) {
+    // (KEEP runs every layer in every step: what the others skip only reaches
+    // rows that nothing reads, and without the branches the kernel keeps to 168
+    // registers, three waves per SIMD, not two; a training step 381 -> 365 us
+    // with fused_back_kernel likewise.  Plain inference has them either way,
+    // and the products skipped are worth more: 55 and 60 us)
+    if (KEEP || (t >= 1 && t <= nsteps - 3)) {
       const int r = y0 - 5 + t;
       const bool rin = r >= 0 && r < H;
 #pragma unroll
-      for (int u = 0; u < 2; u++) {
+      for (int u = 0; u < nu; u++) {
         const int sg = sA + 2 * u;
         // lanes kg = 3 meet zero weights: they re-read column tap 2
         const bf16x8 a = *reinterpret_cast<const bf16x8 *>(s_in[rs] + (16 * sg + m + min(kg, 2)) * C_INP);
@@ -377,11 +400,11 @@ __global__ __launch_bounds__(256) void fused_net_kernel(const bf16 *__restrict__
       }
     }
     // layer 2: layer-1 rows y0-2 .. y1+1 (steps 4 .. rows+7); completes row y0-7+t
-    if (t >= 4 && t <= nsteps - 2) {
+    if (KEEP || (t >= 4 && t <= nsteps - 2)) {
       const int r = y0 - 7 + t;
       const bool rin = r >= 0 && r < H;
 #pragma unroll
-      for (int u = 0; u < 2; u++) {
+      for (int u = 0; u < nu; u++) {
         const int sg = sA + 2 * u;
         bf16x8 a[3];
 #pragma unroll
@@ -402,7 +425,7 @@ __global__ __launch_bounds__(256) void fused_net_kernel(const bf16 *__restrict__
     }
     // layer 3: layer-2 rows y0-1 .. y1 (steps 7 .. rows+8); completes output
     // row y0-9+t, staged from step 9 on
-    if (t >= 7 && t < nsteps) {
+    if ((KEEP || (t >= 7 && t < nsteps)) && (nu == 2 || wv < 2)) {
       const int sg = wv;
       bf16x8 a[3];
 #pragma unroll
@@ -413,7 +436,7 @@ __global__ __launch_bounds__(256) void fused_net_kernel(const bf16 *__restrict__
       for (int dx = 0; dx < 3; dx++) acc = mfma32(bw3[dx], a[dx], acc);
       q3 = acc;
       const int w = 16 * sg + m;
-      if (t >= FUSED_HALO && kg < C_OUT && w >= 3 && w < FW - 3)
+      if (t >= FUSED_HALO && t < nsteps && kg < C_OUT && w >= 3 && w < FW - 3)
         s_out[((t - FUSED_HALO) * FOUT + w - 3) * C_OUT + kg] = acc[2] + bv3;
     }
     // this step's rows become readable, and the slots read in this step may
@@ -426,14 +449,20 @@ __global__ __launch_bounds__(256) void fused_net_kernel(const bf16 *__restrict__
   for (int u = 0; u < 2; u++) ra.l1[u] = rb.l1[u] = rc.l1[u] = ra.l2[u] = rb.l2[u] = rc.l2[u] = zero;
   // whole groups of six steps (the ones past nsteps only load and wait), so
   // every step issues its load and the wait for it is the same on every path
-  for (int t = 0; t < nsteps; t += 6) {
-    step(t, IC<0>{}, ra, rb, rc);
-    step(t + 1, IC<1>{}, rb, rc, ra);
-    step(t + 2, IC<0>{}, rc, ra, rb);
-    step(t + 3, IC<1>{}, ra, rb, rc);
-    step(t + 4, IC<0>{}, rb, rc, ra);
-    step(t + 5, IC<1>{}, rc, ra, rb);
-  }
+  auto march = [&](auto SEGS) {
+    for (int t = 0; t < nsteps; t += 6) {
+      step(SEGS, t, IC<0>{}, ra, rb, rc);
+      step(SEGS, t + 1, IC<1>{}, rb, rc, ra);
+      step(SEGS, t + 2, IC<0>{}, rc, ra, rb);
+      step(SEGS, t + 3, IC<1>{}, ra, rb, rc);
+      step(SEGS, t + 4, IC<0>{}, rb, rc, ra);
+      step(SEGS, t + 5, IC<1>{}, rc, ra, rb);
+    }
+  };
+  // a window whose second half lies outside the image leaves its zeros there
+  // (the last of five at 257 columns: a tenth of the products)
+  if (c0 + FW / 2 < W) march(IC<2>{});
+  else march(IC<1>{});
 
   // corrected-candidate energy (T != void): this block's U and materials,
   // loaded before the output is written out
@@ -521,7 +550,7 @@ __device__ __forceinline__ uint2 mask_pack4(f32x4 acc, uint2 a, bool in)
 
 constexpr int BACK_HALO = 6;  // row steps beyond the chunk's rows
 
-__global__ __launch_bounds__(256) void fused_back_kernel(const bf16 *__restrict__ dY3, int H, int W, int rows,
+__global__ __launch_bounds__(256, 3) void fused_back_kernel(const bf16 *__restrict__ dY3, int H, int W, int rows,
                                                          const bf16 *__restrict__ w3t, const bf16 *__restrict__ w2t,
                                                          const bf16 *__restrict__ A2, const bf16 *__restrict__ A1,
                                                          bf16 *__restrict__ dP2, bf16 *__restrict__ dP1)
@@ -577,8 +606,8 @@ __global__ __launch_bounds__(256) void fused_back_kernel(const bf16 *__restrict_
     }
   __syncthreads();
 
-  auto step = [&](int t, auto P, FusedRows &Xr, FusedRows &Yr, FusedRows &Zr) {
-    constexpr int ws = decltype(P)::value, rs = ws ^ 1;
+  auto step = [&](auto SEGS, int t, auto P, FusedRows &Xr, FusedRows &Yr, FusedRows &Zr) {
+    constexpr int nu = decltype(SEGS)::value, ws = decltype(P)::value, rs = ws ^ 1;
     if (threadIdx.x < FIN_PARTS) {
       const int ri = y0 - 2 + t;
       const bool in = iload && ri >= 0 && ri < H;
@@ -594,10 +623,10 @@ __global__ __launch_bounds__(256) void fused_back_kernel(const bf16 *__restrict_
       m1[ws][u] = load_mask(A1, u, y0 - 4 + t);
     }
     // layer 3's transpose: dY3 rows y0-2 .. y1+1 (steps 1 .. rows+4); completes dP2 row y0-4+t
-    if (t >= 1 && t <= nsteps - 2) {
+    {
       const int r = y0 - 4 + t;
 #pragma unroll
-      for (int u = 0; u < 2; u++) {
+      for (int u = 0; u < nu; u++) {
         const int w = 16 * (sA + 2 * u) + m;
         const bf16x8 a = *reinterpret_cast<const bf16x8 *>(s_in[rs] + (w + min(kg, 2)) * C_D3);
         Zr.l1[u] = mfma32(bw3[0], a, zero);
@@ -610,10 +639,10 @@ __global__ __launch_bounds__(256) void fused_back_kernel(const bf16 *__restrict_
       }
     }
     // layer 2's transpose: dP2 rows y0-1 .. y1 (steps 4 .. rows+5); completes dP1 row y0-6+t
-    if (t >= 4 && t < nsteps) {
+    {
       const int r = y0 - 6 + t;
 #pragma unroll
-      for (int u = 0; u < 2; u++) {
+      for (int u = 0; u < nu; u++) {
         const int w = 16 * (sA + 2 * u) + m;
         bf16x8 a[3];
 #pragma unroll
@@ -634,14 +663,19 @@ __global__ __launch_bounds__(256) void fused_back_kernel(const bf16 *__restrict_
   FusedRows ra, rb, rc;
 #pragma unroll
   for (int u = 0; u < 2; u++) ra.l1[u] = rb.l1[u] = rc.l1[u] = ra.l2[u] = rb.l2[u] = rc.l2[u] = zero;
-  for (int t = 0; t < nsteps; t += 6) {
-    step(t, IC<0>{}, ra, rb, rc);
-    step(t + 1, IC<1>{}, rb, rc, ra);
-    step(t + 2, IC<0>{}, rc, ra, rb);
-    step(t + 3, IC<1>{}, ra, rb, rc);
-    step(t + 4, IC<0>{}, rb, rc, ra);
-    step(t + 5, IC<1>{}, rc, ra, rb);
-  }
+  auto march = [&](auto SEGS) {
+    for (int t = 0; t < nsteps; t += 6) {
+      step(SEGS, t, IC<0>{}, ra, rb, rc);
+      step(SEGS, t + 1, IC<1>{}, rb, rc, ra);
+      step(SEGS, t + 2, IC<0>{}, rc, ra, rb);
+      step(SEGS, t + 3, IC<1>{}, ra, rb, rc);
+      step(SEGS, t + 4, IC<0>{}, rb, rc, ra);
+      step(SEGS, t + 5, IC<1>{}, rc, ra, rb);
+    }
+  };
+  // a window whose second half lies outside the image leaves its zeros there
+  if (c0 + FW / 2 < W) march(IC<2>{});
+  else march(IC<1>{});
 }
 
 // --------------------------------------------------------------------------
@@ -1277,7 +1311,7 @@ struct sbp_corrector {
   double *lpart = nullptr, *scalars = nullptr;  // scalars: [0] loss, [1] E_old
   int *rejected = nullptr, *idx = nullptr;
   double *bpart = nullptr, *be_old = nullptr;  // batched energies: per-block partials, reference energies
-  double *cpart = nullptr;                      // candidate energies: per-block partials (at most one per 256 points)
+  double *cpart = nullptr;                      // candidate energies: per-block partials
   int *brej = nullptr;
   float *ds_raw = nullptr, *ds_tgt = nullptr;
   int ds_n = 0;
@@ -1321,9 +1355,9 @@ int prepare(sbp_corrector *c)
 template <typename T = void, bool KEEP = false>
 void launch_infer(sbp_corrector *c, int nb, hipStream_t stream, NetEnergyArgs ea = NetEnergyArgs{})
 {
-  const long blocks = (long)nb * net_blocks_per_image(c->H, c->W);
+  const long blocks = (long)nb * net_blocks_per_image(nb, c->H, c->W);
   hipLaunchKernelGGL((fused_net_kernel<T, KEEP>), dim3((unsigned)blocks), dim3(256), 0, stream, c->X0, nb, c->H, c->W,
-                     net_chunk_rows(c->H), c->w1, c->b1, c->w2, c->b2, c->w3, c->b3, c->Yo, c->A1, c->A2, ea);
+                     net_chunk_rows(nb, c->H, c->W), c->w1, c->b1, c->w2, c->b2, c->w3, c->b3, c->Yo, c->A1, c->A2, ea);
 }
 
 // Training forward of nb images packed in X0: Yo, and the activations A1, A2.
@@ -1358,8 +1392,8 @@ int backward(sbp_corrector *c, int nb)
   const double inv_n = 1.0 / (double)(npix * C_OUT);
   hipLaunchKernelGGL(loss_kernel, dim3(lblocks), dim3(256), 0, c->stream, c->Yo, c->Tg, npix, c->H, c->W, c->band, inv_n,
                      c->dY3, c->lpart);
-  hipLaunchKernelGGL(fused_back_kernel, dim3((unsigned)(nb * net_blocks_per_image(c->H, c->W))), dim3(256), 0, c->stream,
-                     c->dY3, c->H, c->W, net_chunk_rows(c->H), c->w3t, c->w2t, c->A2, c->A1, c->dP2, c->dP1);
+  hipLaunchKernelGGL(fused_back_kernel, dim3((unsigned)(nb * net_blocks_per_image(nb, c->H, c->W))), dim3(256), 0, c->stream,
+                     c->dY3, c->H, c->W, net_chunk_rows(nb, c->H, c->W), c->w3t, c->w2t, c->A2, c->A1, c->dP2, c->dP1);
   WgradReduce r{};
   r.part[0] = c->wpart;
   r.part[1] = r.part[0] + (long)WG_BLOCKS * wg_len(C_INP, C_H);
@@ -1441,7 +1475,9 @@ int sbp_corr_create(int nx, int ny, int batch, sbp_corrector **out)
   if (!rc) rc = dmalloc(&c->rejected, sizeof(int));
   if (!rc) rc = dmalloc(&c->idx, sizeof(int) * batch);
   if (!rc) rc = dmalloc(&c->bpart, sizeof(double) * batch * 64);
-  if (!rc) rc = dmalloc(&c->cpart, sizeof(double) * batch * net_blocks_per_image(ny, nx));
+  long cparts = 0;  // (fewer images may take more blocks each)
+  for (int n = 1; n <= batch; n++) cparts = std::max(cparts, n * net_blocks_per_image(n, ny, nx));
+  if (!rc) rc = dmalloc(&c->cpart, sizeof(double) * cparts);
   if (!rc) rc = dmalloc(&c->be_old, sizeof(double) * batch);
   if (!rc) rc = dmalloc(&c->brej, sizeof(int) * batch);
   if (!rc) {
@@ -1742,7 +1778,7 @@ int sbp_corr_advance_batch(sbp_corrector *c, sbp_batch *b, const double *dt, lon
   if (rc) return rc;
   const int count = b->count, bpi = 64;
   // candidate-energy partials per instance: one per inference block
-  const int cbpi = (int)net_blocks_per_image(c->H, c->W);
+  const int cbpi = (int)net_blocks_per_image(count, c->H, c->W);
   const int pth_ = b->esz == 8 ? pth<double> : pth<float>;
   const int ptiles = ((c->W + PTW - 1) / PTW) * ((c->H + pth_ - 1) / pth_);
   const long npix = (long)count * c->H * c->W;
@@ -1758,7 +1794,7 @@ int sbp_corr_advance_batch(sbp_corrector *c, sbp_batch *b, const double *dt, lon
   hipLaunchKernelGGL(batch_energy_final_kernel, dim3((count + 63) / 64), dim3(64), 0, s, c->bpart, count, bpi, c->be_old);
   HIP_OR_FAIL(hipGetLastError());
   // one corrected step: plain RK4 stages, features, network, candidate
-  // energy, guarded update -- kernel launches only, so it can be captured
+  // energy, guarded update
   // (descriptors of the parity after the step: a two-stage step moves the
   // state into the Y0 pool)
   auto enqueue_step = [&]() -> hipError_t {
@@ -1781,34 +1817,10 @@ int sbp_corr_advance_batch(sbp_corrector *c, sbp_batch *b, const double *dt, lon
     }
     return hipGetLastError();
   };
-  // Runs of kGraphSteps corrected steps are captured once per call and
-  // replayed (no memset nodes: counters are cleared above, outside it).
-  constexpr long kGraphSteps = 16;
-  long done = 0;
-  if (nsteps >= 2 * kGraphSteps) {
-    hipGraph_t g = nullptr;
-    hipGraphExec_t ge = nullptr;
-    const int par0 = b->par;  // captured two-stage steps flip the batch's parity as if they had run
-    HIP_OR_FAIL(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    hipError_t le = hipSuccess;
-    for (long k = 0; k < kGraphSteps && le == hipSuccess; k++) le = enqueue_step();
-    hipError_t ce = hipStreamEndCapture(s, &g);
-    if (le != hipSuccess || ce != hipSuccess) {
-      b->par = par0;
-      if (g) (void)hipGraphDestroy(g);
-      return fail(SBP_EHIP, std::string("corrector graph capture: ") + hipGetErrorString(le != hipSuccess ? le : ce));
-    }
-    hipError_t ie = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(g);
-    if (ie != hipSuccess) return fail(SBP_EHIP, std::string("corrector graph instantiate: ") + hipGetErrorString(ie));
-    hipError_t re = hipSuccess;
-    for (; done + kGraphSteps <= nsteps && re == hipSuccess; done += kGraphSteps) re = hipGraphLaunch(ge, s);
-    hipError_t se = hipStreamSynchronize(s);
-    (void)hipGraphExecDestroy(ge);
-    if (re != hipSuccess || se != hipSuccess)
-      return fail(SBP_EHIP, std::string("corrector graph launch: ") + hipGetErrorString(re != hipSuccess ? re : se));
-  }
-  for (; done < nsteps; done++) HIP_OR_FAIL(enqueue_step());
+  // (launched one by one: a step's four kernels take longer than their launches
+  // even for one small image, and a captured graph of them would be instantiated
+  // on every call: 32 steps of one 257^2 image 2080 us launched, 2235 replayed)
+  for (long k = 0; k < nsteps; k++) HIP_OR_FAIL(enqueue_step());
   std::vector<int> rej(count, 0);
   HIP_OR_FAIL(hipMemcpyAsync(rej.data(), c->brej, sizeof(int) * count, hipMemcpyDeviceToHost, s));
   HIP_OR_FAIL(hipStreamSynchronize(s));
