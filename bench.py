@@ -41,8 +41,8 @@ PEAK_HBM_GBS = 8000.0
 # 2.0 + WRITE_SIZE x 1.0 KiB (the factors that turn the counters of a 1 GiB
 # plain copy in the same runs into the bytes it reads and writes):
 # profiles/march2d_acoustic_4097sq_order4_fp64_hbm_counters.md.
-MEASURED_TRAFFIC = {}
-MEASURED_AT = None
+MEASURED_TRAFFIC = {(4097, 4, 0, "whole step", 1): (237420 * 2.0 + 395820 * 1.0) * 1024}
+MEASURED_AT = "c5497f2"
 
 
 def pkg(sub):
@@ -204,12 +204,13 @@ def batched(count=256, steps=500, warmup=10, prec=1):
     dofs = sum(sp.nx * sp.ny * 3 for sp in specs)
     bpd = bytes_per_dof(prec, materials=True)
     achieved = dofs * bpd * steps / (ev_ms * 1e-3) / 1e9
-    kbpd = sum(sum(launch_bytes(sp, TWO if cfg.get("two_stage", False) else ONE)) for sp in specs) / dofs
+    schedule = TWO if cfg["two_stage"] else (WHOLE if cfg["blocks_per_cu"] == 0 else ONE)
+    kbpd = sum(sum(launch_bytes(sp, schedule)) for sp in specs) / dofs
     return {"instances": count, "dofs": dofs, "steps": steps, "precision": ["fp64", "fp32", "fp32_kahan"][prec],
             "dof_updates_per_s": dofs * steps / wall, "ms_per_step": wall / steps * 1e3,
             "event_ms_per_step": ev_ms / steps, "bytes_per_dof": bpd, "achieved_gbs": achieved,
             "frac": achieved / PEAK_HBM_GBS, "kernel_bytes_per_dof": kbpd,
-            "kernel_frac": achieved * kbpd / bpd / PEAK_HBM_GBS, "autotune_choice": choice, "config": cfg,
+            "kernel_frac": achieved * kbpd / bpd / PEAK_HBM_GBS, "autotune_choice": choice, "config": cfg, "schedule": schedule,
             "setup_s": setup_s, "energy_head": e_end}
 
 

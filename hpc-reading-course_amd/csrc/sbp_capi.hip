@@ -169,16 +169,23 @@ bool step_default(const sbp_ctx *c)
 
 // Marched steps (sbp_march.hpp) replace both from the sizes where their lead-in
 // and frame cost less than the passes they save (us per step, march / before):
-// order 4 FP64 301^2 12.8 / 11.5, 401^2 13.2 / 15.4, 1025^2 27.1 / 47.5, 4097^2
-// 226 / 452; FP32 401^2 10.1 / 9.7, 513^2 11.9 / 14.2, 4097^2 121 / 236; order 2
-// FP64 201^2 6.3 / 5.8, 257^2 6.5 / 7.3; order 6 FP64 301^2 21.9 / 20.1, 513^2
-// 30.3 / 36.7, FP32 301^2 15.2 / 17.2.  Ribbons leave most of a strip's columns
-// or rows to the lead-in: 64 x 4096 31.7 / 16.1, 2048 x 128 19.1 / 17.8, 128 x
-// 2048 22.8 / 20.6, 2000 x 200 22.1 / 23.4; longer ones are still better
-// marched (64 x 60000 201 / 338, 60000 x 64 87 / 176).
+// order 4 FP64 301^2 12.8 / 11.5, 401^2 12.0 / 15.4, 1025^2 27.1 / 47.5, 4097^2
+// 226 / 452, and with rho/K arrays or of advection, whose steps on chip slow
+// down earlier, 301^2 13.4 / 15.2 and 7.8 / 7.9; FP32 401^2 10.1 / 9.7, 513^2
+// 11.9 / 14.2, 4097^2 117 / 236, advection 401^2 7.0 / 7.4; order 2 FP64 201^2
+// 6.3 / 5.8, 257^2 6.5 / 7.3; order 6 FP64 301^2 21.9 / 20.1, 513^2 30.3 / 36.7,
+// FP32 301^2 15.2 / 17.2.  Ribbons leave most of a strip's columns or rows to
+// the lead-in: 64 x 4096 31.7 / 16.1, 2048 x 128 19.1 / 17.8, 128 x 2048 22.8 /
+// 20.6, 2000 x 200 22.1 / 23.4; longer ones are still better marched (64 x 60000
+// 201 / 338, 60000 x 64 87 / 176).
 bool march_default(const sbp_ctx *c)
 {
-  const long least = std::min(c->nx, c->ny) <= 128 ? 700 : (c->order == 2 ? 260 : 380);
+  const bool adv = c->phys == SBP_ADVECTION_2D, arr = c->mat == SBP_MAT_ARRAYS;
+  long least = 380;
+  if (c->order == 2) least = 260;
+  if (c->order == 4 && c->esz == 8 && (adv || arr)) least = 300;
+  if (c->order == 4 && c->esz == 4 && !adv) least = 440;
+  if (std::min(c->nx, c->ny) <= 128) least = 700;
   return c->march_plan.ok && (long)c->nx * c->ny >= least * least;
 }
 
