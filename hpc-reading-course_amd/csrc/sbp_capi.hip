@@ -169,8 +169,8 @@ bool step_default(const sbp_ctx *c)
 
 // Marched steps (sbp_march.hpp) replace both from the sizes where their lead-in
 // and frame cost less than the passes they save (us per step, march / before):
-// order 4 FP64 301^2 12.8 / 11.5, 401^2 12.0 / 15.4, 1025^2 27.1 / 47.5, 4097^2
-// 226 / 452, and with rho/K arrays or of advection, whose steps on chip slow
+// order 4 FP64 301^2 12.8 / 11.5, 401^2 12.0 / 15.4, 1025^2 26.3 / 47.5, 4097^2
+// 223 / 452, and with rho/K arrays or of advection, whose steps on chip slow
 // down earlier, 301^2 13.4 / 15.2 and 7.8 / 7.9; FP32 401^2 10.1 / 9.7, 513^2
 // 11.9 / 14.2, 4097^2 117 / 236, advection 401^2 7.0 / 7.4; order 2 FP64 201^2
 // 6.3 / 5.8, 257^2 6.5 / 7.3; order 6 FP64 301^2 21.9 / 20.1, 513^2 30.3 / 36.7,

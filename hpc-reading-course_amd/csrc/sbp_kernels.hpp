@@ -18,9 +18,11 @@
 // step instead of the 16 of a 3-register (U, Y, accumulator) scheme.  The
 // Kahan form compensates the final U += increment with one more register.
 // The 1D kernel (line_kernel) runs whole steps on chip and follows
-// RK4_custom's operation order exactly.  Large 2D grids run the two-stage schedule further down
-// (pair2d_kernel: stages 1-2 and 3-4 in one launch each, the inner stage on
-// chip, 5 words per value and step) with the same arithmetic per point.
+// RK4_custom's operation order exactly.  2D grids run whole steps by default
+// (sbp_step.hpp, sbp_march.hpp), large ones with the forcing the two-stage
+// schedule further down (pair2d_kernel: stages 1-2 and 3-4 in one launch each,
+// the inner stage on chip, 5 words per value and step), with the same
+// arithmetic per point.
 //
 // Layout in HBM: one plane per component, rows of `pitch` elements, column i
 // stored at xoff + i with xoff chosen so that the first interior column

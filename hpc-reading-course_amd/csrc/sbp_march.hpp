@@ -22,15 +22,15 @@
 // every stage is an interior point of the operator; the D-deep frame is cut
 // into patches that blocks of the same launch step on chip (sbp_step.hpp).
 //
-// What bounds it: order 4 FP64, 4097^2, takes 226 us per step (452 as two
+// What bounds it: order 4 FP64, 4097^2, takes 223 us per step (452 as two
 // launches).  806 MB of U and U' are 147 us at what a copy reaches; a row costs
 // a CU's LDS 0.6 us for the neighbours (32 words read and 8 written per column)
 // and its SIMDs 0.8 us for 200 instructions, which the barrier of each row lets
 // overlap in part; halo columns and lead-in rows add a fifth.  Constant LDS
 // addresses (15 instructions less per row, at a longer unrolling) and more rows
 // of loads in flight (3, 4) gain nothing.  Small grids wait for the lead-in
-// and the frame (1025^2 27 us, 47.5 before).  FP32 4097^2 117 (236), order 6
-// FP32 + compensation with rho/K arrays 272 (442), order 6 FP64 413 (570: its
+// and the frame (1025^2 26 us, 47.5 before).  FP32 4097^2 116 (236), order 6
+// FP32 + compensation with rho/K arrays 273 (442), order 6 FP64 347 (570: its
 // rings fill the register file, one wave per SIMD).  Stores are cached: 2049^2
 // FP64 74.6 us, 78.5 nontemporal, and the next step reads them.  A version
 // whose waves exchange columns through DPP alone, with no LDS and no barrier,
@@ -128,21 +128,35 @@ __device__ __forceinline__ void march_strip(const StepArgs<T> &a, T *lds, int st
     }
   };
 
-  // right-hand side of stage ST at ring slot s of its operand rows Y, whose
-  // centre row lies in the exchange slot at xr
-  auto rhs = [&](const T (&Y)[WN][C], auto SLOT, auto ST, const T *xr, T ri, T Kb, T *F) {
-    constexpr int s = decltype(SLOT)::value, st = decltype(ST)::value - 1;
-    auto ddx = [&](int f, int c) {
-      const T *l = xr + (st * NF + f) * XW;
-      return dint<T, ORDER>([&](int n) { return n == R ? Y[s][c] : l[n - R]; }, a.hix);
+  // x neighbours of one exchanged field (unit: stage and field) of the row at xr
+  auto fetch = [&](int unit, const T *xr, T (&o)[2 * R]) {
+    const T *l = xr + unit * XW;
+#pragma unroll
+    for (int n = 0; n < 2 * R; n++) o[n] = l[n < R ? n - R : n - R + 1];
+  };
+  // right-hand side of stage ST (of NS running) at ring slot s of its operand
+  // rows Y, whose centre row lies in the exchange slot at xr.  The neighbours of
+  // a field are fetched while the field before it is differentiated, behind a
+  // scheduling barrier: left to itself the compiler moves each fetch to its use
+  // and waits for LDS eight times per row (order 6 FP64, one wave per SIMD, 413
+  // us per step at 4097^2, 347 so; order 4 FP64 27.2 and 26.3 at 1025^2).  A
+  // whole stage ahead would take order 4 FP64 past 256 registers.
+  auto rhs = [&](const T (&Y)[WN][C], auto SLOT, auto ST, auto NS, T (&nb)[2][2 * R], const T *xr, T ri, T Kb, T *F) {
+    constexpr int s = decltype(SLOT)::value, st = decltype(ST)::value - 1, units = decltype(NS)::value * NF;
+    auto ddx = [&](auto FIELD, int c) {
+      constexpr int u = st * NF + decltype(FIELD)::value;
+      if constexpr (u + 1 < units) fetch(u + 1, xr, nb[(u + 1) & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+      const T (&l)[2 * R] = nb[u & 1];
+      return dint<T, ORDER>([&](int n) { return n == R ? Y[s][c] : l[n < R ? n : n - 1]; }, a.hix);
     };
     auto ddy = [&](int c) { return dint<T, ORDER>([&](int n) { return Y[(s + n + WN - R) % WN][c]; }, a.hiy); };
     if constexpr (AC) {
-      const T dxp = ddx(1, 2), dyp = ddy(2), dxu = ddx(0, 0), dyv = ddy(1);
+      const T dxu = ddx(Int<0>{}, 0), dyv = ddy(1), dxp = ddx(Int<1>{}, 2), dyp = ddy(2);
       acoustic_F<T, MAT>(dxp, dyp, dxu, dyv, ri, Kb, T(0), T(0), F[0], F[1], F[2]);
     } else {
       const T va = LD_M ? ri : a.ax, vb = LD_M ? Kb : a.ay;
-      F[0] = -mad(va, ddx(0, 0), vb * ddy(0));
+      F[0] = -mad(va, ddx(Int<0>{}, 0), vb * ddy(0));
     }
   };
   // a new operand row of stage ST into the exchange slot at xw
@@ -175,15 +189,16 @@ __device__ __forceinline__ void march_strip(const StepArgs<T> &a, T *lds, int st
       M1[s1][1] = mk;
     }
     load(k + PF, (kp + PF) % WN);
-    T F[C];
+    T F[C], nb[2][2 * R];
     if constexpr (ns >= 1) {
-      rhs(U1, Int<s1>{}, Int<1>{}, xr, mr, mk, F);
+      fetch(0, xr, nb[0]);
+      rhs(U1, Int<s1>{}, Int<1>{}, NS, nb, xr, mr, mk, F);
 #pragma unroll
       for (int c = 0; c < C; c++) Y2[s1][c] = mad(a.c12, F[c], U1[s1][c]);
       share(Int<2>{}, xw, Y2[s1]);
     }
     if constexpr (ns >= 2) {
-      rhs(Y2, Int<s2>{}, Int<2>{}, xr, LD_M ? M1[s2][0] : T(1), LD_M ? M1[s2][1] : T(1), F);
+      rhs(Y2, Int<s2>{}, Int<2>{}, NS, nb, xr, LD_M ? M1[s2][0] : T(1), LD_M ? M1[s2][1] : T(1), F);
 #pragma unroll
       for (int c = 0; c < C; c++) {
         const T U = U1[s2][c];
@@ -198,7 +213,7 @@ __device__ __forceinline__ void march_strip(const StepArgs<T> &a, T *lds, int st
         M2[s3][0] = m3r;
         M2[s3][1] = m3k;
       }
-      rhs(Y3, Int<s3>{}, Int<3>{}, xr, m3r, m3k, F);
+      rhs(Y3, Int<s3>{}, Int<3>{}, NS, nb, xr, m3r, m3k, F);
 #pragma unroll
       for (int c = 0; c < C; c++) {
         const T U = U2[s3][c];
@@ -208,7 +223,7 @@ __device__ __forceinline__ void march_strip(const StepArgs<T> &a, T *lds, int st
       share(Int<4>{}, xw, Y4[s3]);
     }
     if constexpr (ns >= 4) {
-      rhs(Y4, Int<s4>{}, Int<4>{}, xr, LD_M ? M2[s4][0] : T(1), LD_M ? M2[s4][1] : T(1), F);
+      rhs(Y4, Int<s4>{}, Int<4>{}, NS, nb, xr, LD_M ? M2[s4][0] : T(1), LD_M ? M2[s4][1] : T(1), F);
       const long o = (long)(rs + k - 4 * R) * a.pitch;
       if (out && rs + k - 4 * R < j1) {
         T *__restrict__ p = a.uo + o;
