@@ -318,7 +318,8 @@ def _problem_struct(spec, keep):
 
 class Batch:
     """Ensemble of independent 2D acoustic problems advanced together
-    (sbp_batch in C): one persistent kernel per RK4 stage, graph-replayed steps."""
+    (sbp_batch in C): one persistent kernel per RK4 stage or pair of stages, or
+    one launch per whole step, as configured; graph-replayed steps."""
 
     def __init__(self, specs):
         lib = load_library()

@@ -70,7 +70,8 @@ template <typename T, int ORDER, int PHYS, int MAT, bool TR, int NW, int H, int 
   const int nx, ny;
   const T hl, hr;  // of the lane and row axes
   const int lane, wv;
-  int xl[NST + 1], xh[NST + 1], yl[NST + 1], yh[NST + 1];  // regions evaluated in stages 1 .. NST ([NST]: the patch), and loaded ([0])
+  // regions evaluated in stages 1 .. NST ([NST]: the patch), and loaded ([0])
+  int xl[NST + 1], xh[NST + 1], yl[NST + 1], yh[NST + 1];
   bool xedge, yedge;  // closure columns (rows) among the region's
   int i;
   T cf[TAPS];
