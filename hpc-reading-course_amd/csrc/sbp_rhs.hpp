@@ -12,6 +12,17 @@ namespace sbp {
 
 constexpr int kRhsWaves = 4, kRhsRows = 16;  // waves of a block, most rows it loads
 
+// LDS values pass between lanes of one wave: what any lane wrote before is read
+// as written by any lane after.  A wave's LDS operations complete in order, so
+// the fences cost no wait; they keep the compiler, to which the barrier alone
+// says nothing about memory, from moving the accesses across it.
+__device__ __forceinline__ void wave_handover()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <typename T, int ORDER, int PHYS, int MAT>
 __global__ __launch_bounds__(64 * kRhsWaves) void rhs_patch_kernel(StepArgs<T> a, double c5, const double *__restrict__ in,
                                                                    double *__restrict__ out)
@@ -62,21 +73,21 @@ __global__ __launch_bounds__(64 * kRhsWaves) void rhs_patch_kernel(StepArgs<T> a
 #pragma unroll
       for (int c = 0; c < C; c++) Yc[c] = pt.slot(0, r)[c * Pt::FS];
       pt.template rhs<decltype(XE)::value>(0, r, j, Yc, ri[k], Kb[k], c5, F);
-      // a wave's own row of results: its LDS operations complete in order
+      // a row of results that only this wave writes and reads
       double *o = so[pt.wv];
       if (pt.own()) {
         const int col = pt.xl[0] + pt.lane - i0;
 #pragma unroll
         for (int c = 0; c < C; c++) o[col * C + c] = F[c];
       }
-      __builtin_amdgcn_wave_barrier();
+      wave_handover();
       double *row = out + ((long)j * a.nx + i0) * C;
 #pragma unroll
       for (int c = 0; c < C; c++) {
         const int q = pt.lane + kStepLanes * c;
         if (q < (i1 - i0) * C) row[q] = o[q];
       }
-      __builtin_amdgcn_wave_barrier();
+      wave_handover();
     }
   };
   if (pt.xedge) rows(std::true_type{});
