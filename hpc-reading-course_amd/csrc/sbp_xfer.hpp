@@ -23,7 +23,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 
 namespace sbp {
@@ -84,7 +84,7 @@ class Staging {
     int started = 1;
     try {
       for (; started < kSlots; started++) th[started] = std::thread(drain, started);
-    } catch (const std::system_error &) {  // no more threads: those there are take the rest
+    } catch (const std::exception &) {  // no more threads, or no memory for one: those there are take the rest
     }
     drain(0);
     for (int k = 1; k < started; k++) th[k].join();
