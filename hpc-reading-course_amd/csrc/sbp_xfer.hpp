@@ -60,13 +60,19 @@ class Staging {
   hipError_t to_host(void *dst, const void *src, size_t bytes, hipStream_t s)
   {
     const long chunks = (long)((bytes + kChunk - 1) / kChunk);
-    int device = 0;
-    hipError_t e = hipGetDevice(&device);
+    // the stream's device, which need not be the calling thread's
+    int device = 0, callers = 0;
+    hipError_t e = hipStreamGetDevice(s, &device);
+    if (e == hipSuccess) e = hipGetDevice(&callers);
+    if (e == hipSuccess) e = hipSetDevice(device);
     for (int k = 0; k < kSlots && e == hipSuccess; k++) {
       if (!ev_[k]) e = hipEventCreateWithFlags(&ev_[k], hipEventDisableTiming);
       if (e == hipSuccess && !pin_[k]) e = hipHostMalloc(reinterpret_cast<void **>(&pin_[k]), kChunk, hipHostMallocDefault);
     }
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess) {
+      (void)hipSetDevice(callers);
+      return e;
+    }
     std::atomic<long> next{0};
     std::atomic<int> failed{hipSuccess};
     auto drain = [&](int k) {
@@ -88,6 +94,8 @@ class Staging {
     }
     drain(0);
     for (int k = 1; k < started; k++) th[k].join();
+    const hipError_t back = hipSetDevice(callers);
+    if (failed == hipSuccess) failed = back;
     return static_cast<hipError_t>(failed.load());
   }
 };

@@ -1,6 +1,7 @@
 // drain CASE: a result of several chunks through sbp::host::get on the host
 // stand-in of the runtime (hip/hip_runtime.h here); prints ok, exits 0.
 //   plain         as it is
+//   other-device  the calling thread's device is not the stream's (and stays the thread's)
 //   no-memory     the second thread's own allocation throws std::bad_alloc
 #include <hip/hip_runtime.h>
 
@@ -27,7 +28,7 @@ int main(int, char **argv)
   const size_t n = sbp::host::kThreadedBytes + (5 << 20) + 12345;
   std::vector<char> src(n), dst(n);
   for (size_t k = 0; k < n; k++) src[k] = (char)(k * 2654435761u >> 13);
-  FakeStream stream{0};
+  FakeStream stream{how == "other-device" ? 3 : 0};
   sbp::host::Staging staging;
   for (int pass = 0; pass < 2; pass++) {
     std::memset(dst.data(), 0, n);
@@ -36,6 +37,7 @@ int main(int, char **argv)
     t_throw_at = 0;
     if (e != hipSuccess) return std::printf("error %d\n", (int)e), 1;
     if (dst != src) return std::printf("wrong bytes\n"), 1;
+    if (t_device != 0) return std::printf("the thread's device changed\n"), 1;
     if (hipGetLastError() != hipSuccess) return std::printf("an error is left behind\n"), 1;
   }
   std::printf("ok\n");

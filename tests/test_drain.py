@@ -31,3 +31,9 @@ def test_threads_that_cannot_be_allocated(drain):
     """An exception of any kind while a thread is started must not reach the C
     entry, nor leave started threads behind unjoined."""
     assert drain("no-memory") == (0, "ok")
+
+
+def test_result_of_another_device(drain):
+    """A context made on one device, read by a thread whose current device is
+    another (a thread's first device is 0): copy calls take the stream's."""
+    assert drain("other-device") == (0, "ok")
