@@ -65,13 +65,19 @@ class Staging {
     hipError_t e = hipStreamGetDevice(s, &device);
     if (e == hipSuccess) e = hipGetDevice(&callers);
     if (e == hipSuccess) e = hipSetDevice(device);
-    for (int k = 0; k < kSlots && e == hipSuccess; k++) {
-      if (!ev_[k]) e = hipEventCreateWithFlags(&ev_[k], hipEventDisableTiming);
-      if (e == hipSuccess && !pin_[k]) e = hipHostMalloc(reinterpret_cast<void **>(&pin_[k]), kChunk, hipHostMallocDefault);
+    if (e != hipSuccess) return e;
+    int slots = 0;
+    for (; slots < kSlots && e == hipSuccess; slots += e == hipSuccess) {
+      if (!ev_[slots]) e = hipEventCreateWithFlags(&ev_[slots], hipEventDisableTiming);
+      if (e == hipSuccess && !pin_[slots])
+        e = hipHostMalloc(reinterpret_cast<void **>(&pin_[slots]), kChunk, hipHostMallocDefault);
     }
-    if (e != hipSuccess) {
-      (void)hipSetDevice(callers);
-      return e;
+    if (slots < kSlots) (void)hipGetLastError();  // fewer chunks, or none: a copy call
+    if (slots == 0) {
+      e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
+      if (e == hipSuccess) e = hipStreamSynchronize(s);
+      const hipError_t back = hipSetDevice(callers);
+      return e == hipSuccess ? back : e;
     }
     std::atomic<long> next{0};
     std::atomic<int> failed{hipSuccess};
@@ -89,7 +95,7 @@ class Staging {
     std::thread th[kSlots];
     int started = 1;
     try {
-      for (; started < kSlots; started++) th[started] = std::thread(drain, started);
+      for (; started < slots; started++) th[started] = std::thread(drain, started);
     } catch (const std::exception &) {  // no more threads, or no memory for one: those there are take the rest
     }
     drain(0);

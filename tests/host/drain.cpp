@@ -2,6 +2,7 @@
 // stand-in of the runtime (hip/hip_runtime.h here); prints ok, exits 0.
 //   plain         as it is
 //   other-device  the calling thread's device is not the stream's (and stays the thread's)
+//   no-pinned     no pinned chunk to be had; one-pinned: a single one
 //   no-memory     the second thread's own allocation throws std::bad_alloc
 #include <hip/hip_runtime.h>
 
@@ -29,6 +30,8 @@ int main(int, char **argv)
   std::vector<char> src(n), dst(n);
   for (size_t k = 0; k < n; k++) src[k] = (char)(k * 2654435761u >> 13);
   FakeStream stream{how == "other-device" ? 3 : 0};
+  if (how == "no-pinned") g_pinned_most = 0;
+  if (how == "one-pinned") g_pinned_most = 1;
   sbp::host::Staging staging;
   for (int pass = 0; pass < 2; pass++) {
     std::memset(dst.data(), 0, n);

@@ -37,3 +37,10 @@ def test_result_of_another_device(drain):
     """A context made on one device, read by a thread whose current device is
     another (a thread's first device is 0): copy calls take the stream's."""
     assert drain("other-device") == (0, "ok")
+
+
+@pytest.mark.parametrize("case", ["no-pinned", "one-pinned"])
+def test_pinned_memory_that_cannot_be_allocated(drain, case):
+    """The chunks are a means of speed: without them the copy call remains, and
+    the failed allocation is not reported by a later call."""
+    assert drain(case) == (0, "ok")
