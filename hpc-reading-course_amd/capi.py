@@ -42,6 +42,9 @@ class SbpProblem(C.Structure):
 _ARRAY_FIELDS = ("rho_inv", "bulk", "vel_x", "vel_y")  # copied by sbp_create / sbp_batch_create
 
 
+SCHEDULES = ("stages", "pairs", "patches", "march", "line")  # sbp_schedule
+
+
 class SbpError(RuntimeError):
     def __init__(self, code, msg):
         super().__init__("sbp error %d: %s" % (code, msg))
@@ -57,6 +60,8 @@ EXPORTS = {
     "sbp_set_tile_rows": (C.c_int, [C.c_void_p, C.c_int]),
     "sbp_set_fused": (C.c_int, [C.c_void_p, C.c_int, C.c_int]),
     "sbp_get_fused": (C.c_int, [C.c_void_p]),
+    "sbp_get_schedule": (C.c_int, [C.c_void_p]),
+    "sbp_reset_schedule": (C.c_int, [C.c_void_p]),
     "sbp_set_store_policy": (C.c_int, [C.c_void_p, C.c_int]),
     "sbp_tune_fused": (C.c_int, [C.c_void_p, C.c_double, C.POINTER(C.c_int)]),
     "sbp_batch_set_store_policy": (C.c_int, [C.c_void_p, C.c_int]),
@@ -254,17 +259,31 @@ class Context:
         return out
 
     def set_tile_rows(self, rows: int):
+        """Interior tile height of the right-hand side and of one launch per stage."""
         _check(load_library().sbp_set_tile_rows(self._h, int(rows)))
 
     def set_fused(self, on: bool = True, rows: int = 0):
         """Two-stage stepping: stages 1-2 and 3-4 in one launch each, interior
         tiles and boundary-frame patches alike (2D acoustics with any material
-        model, 2D advection); rows = tile height, 0 = chosen from the grid."""
+        model, 2D advection); rows = tile height, 0 = chosen from the grid.
+        False: one launch per stage.  Either replaces a default of whole steps
+        until reset_schedule()."""
         _check(load_library().sbp_set_fused(self._h, int(bool(on)), int(rows)))
 
     @property
     def fused(self) -> bool:
         return bool(load_library().sbp_get_fused(self._h))
+
+    @property
+    def schedule(self) -> str:
+        """How steps run: one of SCHEDULES."""
+        k = load_library().sbp_get_schedule(self._h)
+        _check(min(k, 0))
+        return SCHEDULES[k]
+
+    def reset_schedule(self):
+        """Back to the schedule the context was created with."""
+        _check(load_library().sbp_reset_schedule(self._h))
 
     def set_store_policy(self, policy: int):
         """Two-stage tile stores: 0 by streamed size (default), 1 cached, 2 nontemporal."""

@@ -1099,6 +1099,26 @@ int sbp_set_fused(sbp_ctx *ctx, int on, int rows)
 
 int sbp_get_fused(const sbp_ctx *ctx) { return ctx && ctx->fused ? 1 : 0; }
 
+int sbp_get_schedule(const sbp_ctx *ctx)
+{
+  if (!ctx) return fail(SBP_EINVAL, "null context");
+  if (is1d(ctx->phys)) return SBP_SCHEDULE_LINE;
+  if (ctx->whole) return ctx->march ? SBP_SCHEDULE_MARCH : SBP_SCHEDULE_PATCHES;
+  return ctx->fused ? SBP_SCHEDULE_PAIRS : SBP_SCHEDULE_STAGES;
+}
+
+int sbp_reset_schedule(sbp_ctx *ctx)
+{
+  if (!ctx) return fail(SBP_EINVAL, "null context");
+  HIP_OR_FAIL(hipStreamSynchronize(ctx->stream));
+  drop_graph(ctx);
+  ctx->fused = pair_default(ctx);
+  ctx->whole = ctx->march || step_default(ctx);
+  ctx->p_ty_rows = default_pair_rows(ctx);
+  compute_pair_geometry(ctx);
+  return SBP_OK;
+}
+
 int sbp_tune_fused(sbp_ctx *ctx, double dt, int *rows)
 {
   if (!ctx || !(dt > 0)) return fail(SBP_EINVAL, "bad argument");

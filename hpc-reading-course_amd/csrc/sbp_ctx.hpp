@@ -37,7 +37,7 @@ struct sbp_ctx {
   sbp::PairLaunchFn pair_launch = nullptr;
   bool fused = false;
   // Whole steps in one launch (sbp_step.hpp), in place of either schedule
-  // while nobody has chosen one with sbp_set_fused.
+  // unless one was chosen with sbp_set_fused (until sbp_reset_schedule).
   sbp::StepLaunchFn step_launch = nullptr;
   sbp::StepPlan step_plan{}, rkf_plan{};
   // one right-hand side of vectors in host memory in one launch (sbp_rhs.hpp)

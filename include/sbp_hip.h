@@ -103,8 +103,10 @@ int  sbp_destroy(sbp_ctx *ctx);
 int  sbp_components(const sbp_ctx *ctx);
 long sbp_vector_length(const sbp_ctx *ctx);
 
-/* Interior tile height in rows (default: chosen from the grid size).  A
- * tuning knob with no reference counterpart; results do not depend on it. */
+/* Interior tile height in rows (default: chosen from the grid size) of the
+ * right-hand side and of a step of one launch per stage (SBP_SCHEDULE_STAGES);
+ * whole steps and pairs of stages do not take it.  A tuning knob with no
+ * reference counterpart; results do not depend on it. */
 int  sbp_set_tile_rows(sbp_ctx *ctx, int rows);
 
 /* Two-stage stepping (on = 1): each RK4 step runs stages 1-2 and stages 3-4
@@ -112,16 +114,29 @@ int  sbp_set_tile_rows(sbp_ctx *ctx, int rows);
  * patches of the (CLS+R)-deep boundary frame that evaluate both stages
  * themselves; 5 array passes per step instead of 13, same arithmetic per
  * point.  2D acoustic contexts (every material model) and 2D advection
- * contexts (constant or per-point velocity); SBP_EINVAL otherwise.  On by
- * default for grids of at least 450^2 interior points (where it was
- * measured faster).  rows: tile height of the two-stage tiles
+ * contexts (constant or per-point velocity); SBP_EINVAL otherwise.
+ * on = 0: one launch per stage.  rows: tile height of the two-stage tiles
  * (0 = chosen from the grid).  A performance knob with no reference
  * counterpart: it changes how ts_rk4's steps are scheduled on the device
- * (ts_rk.cpp:54-65), not what they compute.  Until this is called a context
- * runs whole steps in one launch where that was measured faster than the
- * schedule sbp_get_fused reports; the call chooses one of the two schedules. */
+ * (ts_rk.cpp:54-65), not what they compute.  The call chooses one of the two;
+ * until then, and again after sbp_reset_schedule, a context runs whole steps in
+ * one launch where that was measured faster than both. */
 int  sbp_set_fused(sbp_ctx *ctx, int on, int rows);
+/* 1: two-stage stepping is what the context runs, or would run without whole
+ * steps (by default from 450^2 interior points).  sbp_get_schedule tells what
+ * it runs. */
 int  sbp_get_fused(const sbp_ctx *ctx);
+/* How the context's steps run. */
+typedef enum {
+  SBP_SCHEDULE_STAGES  = 0, /* one launch per RK4 stage                                   */
+  SBP_SCHEDULE_PAIRS   = 1, /* two stages per launch                                      */
+  SBP_SCHEDULE_PATCHES = 2, /* a whole step per launch, on-chip patches of a small 2D grid */
+  SBP_SCHEDULE_MARCH   = 3, /* a whole step per launch, marched along a large 2D grid      */
+  SBP_SCHEDULE_LINE    = 4  /* 1D: many steps per launch                                   */
+} sbp_schedule;
+int  sbp_get_schedule(const sbp_ctx *ctx); /* an sbp_schedule; SBP_EINVAL for a null context */
+/* Back to the schedule (and two-stage tile height) the context was created with. */
+int  sbp_reset_schedule(sbp_ctx *ctx);
 /* Time the two-stage schedule's candidate tile heights (8 .. 136 rows) on
  * this grid for step dt and keep the fastest; *rows (optional) receives it
  * (0 when sbp_get_fused is 0).  A context that runs whole steps keeps doing so
@@ -132,7 +147,7 @@ int  sbp_tune_fused(sbp_ctx *ctx, double dt, int *rows);
 /* Store hint of the two-stage tiles' outputs: 0 (default) chooses from the
  * bytes a step streams (cached stores while U, Y2, Y3 and the materials fit
  * the 256 MB Infinity Cache, nontemporal ones beyond), 1 forces cached and 2
- * nontemporal stores.  A performance knob with no reference counterpart;
+ * nontemporal stores.  Other schedules do not take it.  A performance knob with no reference counterpart;
  * results do not depend on it (it selects between two builds of the same
  * kernel, which is how tests run both on small grids). */
 int  sbp_set_store_policy(sbp_ctx *ctx, int policy);
