@@ -379,8 +379,13 @@ __host__ __device__ inline int march_frame(int order, int px, int ny)
 // / 45, 1025^2 21 / 17 / 17 / 19): as many blocks per CU, at most `resident`,
 // as make (rows + lead) (1 + w / 4) smallest.  A frame of few patches takes
 // its place within them, so that all blocks of a launch run at once (1025^2
-// FP64: 31 us per step, 36 with another 88 blocks to wait for; both with S in LDS); a larger one is
-// worth a longer launch (4097^2 FP64 255 / 288).
+// FP64: 31 us per step, 36 with another 88 blocks to wait for; both with S in
+// LDS); a larger one is worth a longer launch (4097^2 FP64 255 / 288).  Where a
+// CU holds one block (order 6 FP64) patches that follow wait for whole blocks
+// and cost about as much as 3 order rows, so the cheaper of the two is taken,
+// rows counted as they run, in whole groups of order + 1 (us per step, within /
+// after the strips' blocks: 1133 x 132 22 / 36, 1395 x 129 23 / 36, 500 x 800 29
+// / 42; 3428 x 140 43 / 38, 1111 x 1053 with arrays 65 / 61).
 struct MarchPlan {
   bool ok;
   int strips, segs, seg_rows;
@@ -394,14 +399,22 @@ inline MarchPlan march_plan(int order, int nx, int ny, int px, int resident)
   p.strips = (w + march_cols(order) - 1) / march_cols(order);
   const int nf = march_frame(order, px, ny);
   double least = 1e300;
-  for (int per = 1; per <= resident; per++) {
-    const int all = kCus * per, blocks = 4 * nf <= all ? all - nf : all;
+  auto consider = [&](int per, int blocks, int group, int late) {
     const int segs = blocks > p.strips ? blocks / p.strips : 1;
     const int rows = (h + segs - 1) / segs;
-    const double cost = (rows + 4.0 * order) * (4 + per);
+    const double cost = ((rows + group - 1) / group * group + 4.0 * order + late) * (4 + per);
     if (cost < least) {
       least = cost;
       p.seg_rows = rows;
+    }
+  };
+  for (int per = 1; per <= resident; per++) {
+    const int all = kCus * per;
+    if (resident > 1) {
+      consider(per, 4 * nf <= all ? all - nf : all, 1, 0);
+    } else {
+      if (all - nf >= p.strips) consider(per, all - nf, order + 1, 0);
+      consider(per, all, order + 1, 3 * order);
     }
   }
   p.segs = (h + p.seg_rows - 1) / p.seg_rows;
