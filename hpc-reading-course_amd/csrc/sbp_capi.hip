@@ -156,37 +156,54 @@ bool pair_default(const sbp_ctx *c)
   return pair_supported(c) && (long)(c->nx - 2 * D) * (c->ny - 2 * D) >= 450L * 450L;
 }
 
-// Whole steps in one launch (sbp_step.hpp) are the default where they were
-// measured faster than the schedule they replace (us per step, whole /
-// schedule): order 4 FP64 641^2 24.4 / 29.5 and with rho/K arrays 27 / 35,
-// rho = 2 + xy 43 / 48, 2D advection 14.7 / 18.5; 769^2 31.4 / 32.3.  Order 6
-// grows twelve rows and columns per patch: 257^2 13.5 / 19.9, 321^2 21.8 / 20.4.
-bool step_default(const sbp_ctx *c)
-{
-  const long most = c->order == 6 ? 300 : 700;
-  return c->step_launch && c->step_plan.ok && (long)c->nx * c->ny <= most * most;
-}
-
-// Marched steps (sbp_march.hpp) replace both from the sizes where their lead-in
-// and frame cost less than the passes they save (us per step, march / before):
-// order 4 FP64 301^2 12.8 / 11.5, 401^2 12.0 / 15.4, 1025^2 26.3 / 47.5, 4097^2
-// 223 / 452, and with rho/K arrays or of advection, whose steps on chip slow
-// down earlier, 301^2 13.4 / 15.2 and 7.8 / 7.9; FP32 401^2 10.1 / 9.7, 513^2
-// 11.9 / 14.2, 4097^2 117 / 236, advection 401^2 7.0 / 7.4; order 2 FP64 201^2
-// 6.3 / 5.8, 257^2 6.5 / 7.3; order 6 FP64 301^2 21.9 / 20.1, 513^2 30.3 / 36.7,
-// FP32 301^2 15.2 / 17.2.  Ribbons leave most of a strip's columns or rows to
-// the lead-in: 64 x 4096 31.7 / 16.1, 2048 x 128 19.1 / 17.8, 128 x 2048 22.8 /
-// 20.6, 2000 x 200 22.1 / 23.4; longer ones are still better marched (64 x 60000
-// 201 / 338, 60000 x 64 87 / 176).
-bool march_default(const sbp_ctx *c)
+// Marched steps (sbp_march.hpp) are the default from the sizes where their
+// lead-in and frame cost less than the passes they save (us per step, march /
+// before): order 4 FP64 301^2 12.8 / 11.5, 401^2 12.0 / 15.4, 1025^2 26.3 /
+// 47.5, 4097^2 223 / 452, and with rho/K arrays or of advection, whose steps on
+// chip slow down earlier, 301^2 13.4 / 15.2 and 7.8 / 7.9; FP32 401^2 10.1 /
+// 9.7, 513^2 11.9 / 14.2, 4097^2 117 / 236, advection 401^2 7.0 / 7.4; order 2
+// FP64 201^2 6.3 / 5.8, 257^2 6.5 / 7.3; order 6 FP64 301^2 21.9 / 20.1, 513^2
+// 30.3 / 36.7.  Order 6 FP32 leads in with 24 rows whatever the grid: FP32 1133
+// x 132 19.7 / 18.5 and in patches 12.6, compensated with arrays 256 x 570 20.7
+// / 19.0 and 15.7, 1141 x 179 23.7 / 20.9 and 19.4, 512 x 471 20.6 / 26.7 and
+// 21.1.  Returns the least size as the side of a square.
+long march_side(const sbp_ctx *c)
 {
   const bool adv = c->phys == SBP_ADVECTION_2D, arr = c->mat == SBP_MAT_ARRAYS;
-  long least = 380;
-  if (c->order == 2) least = 260;
-  if (c->order == 4 && c->esz == 8 && (adv || arr)) least = 300;
-  if (c->order == 4 && c->esz == 4 && !adv) least = 440;
-  if (std::min(c->nx, c->ny) <= 128) least = 700;
+  if (c->order == 2) return 260;
+  if (c->order == 4 && c->esz == 8 && (adv || arr)) return 300;
+  if (c->order == 4 && c->esz == 4 && !adv) return 440;
+  if (c->order == 6 && c->esz == 4 && !adv) return arr && c->prec == SBP_FP32_KAHAN ? 470 : 400;
+  return 380;
+}
+
+// Ribbons leave most of a strip's columns or rows to the lead-in: 64 x 4096 31.7
+// / 16.1, 2048 x 128 19.1 / 17.8, 128 x 2048 22.8 / 20.6, 2000 x 200 22.1 /
+// 23.4; longer ones are still better marched (64 x 60000 201 / 338, 60000 x 64
+// 87 / 176).  With rho/K arrays order 4 FP64 patches cost more than two launches
+// on wide ones already from 280000 points: 3125 x 96 marched 18.9, patches 29.4,
+// launches 25.8; tall ones not (96 x 3125 36, 37, 49).
+bool march_default(const sbp_ctx *c)
+{
+  long least = march_side(c);
+  if (std::min(c->nx, c->ny) <= 128) {
+    const bool wide = c->nx > c->ny && c->order == 4 && c->esz == 8 && c->phys == SBP_ACOUSTIC_2D && c->mat == SBP_MAT_ARRAYS;
+    least = wide ? 530 : 700;
+  }
   return c->march_plan.ok && (long)c->nx * c->ny >= least * least;
+}
+
+// Steps in patches on chip (sbp_step.hpp) are the default on smaller grids,
+// where they were measured faster than the launches they replace (us per step,
+// patches / launches): order 4 FP64 641^2 24.4 / 29.5 and with rho/K arrays 27 /
+// 35, rho = 2 + xy 43 / 48, 2D advection 14.7 / 18.5; 769^2 31.4 / 32.3.  Order 6
+// grows twelve rows and columns per patch: FP64 257^2 13.5 / 19.9, 321^2 21.8 /
+// 20.4; FP32 acoustics up to where marching begins (above).
+bool step_default(const sbp_ctx *c)
+{
+  long most = 700;
+  if (c->order == 6) most = c->esz == 4 && c->march_fns.launch && c->phys == SBP_ACOUSTIC_2D ? march_side(c) : 300;
+  return c->step_launch && c->step_plan.ok && (long)c->nx * c->ny <= most * most;
 }
 
 int default_ty_rows(int nx, int ny, int cls)
@@ -817,7 +834,6 @@ int build_ctx(const sbp_problem *desc, sbp_ctx *c)
                                       : (c->order == 4 ? step_launcher_o4_f32 : step_launcher_o6_f32))(
           c->phys, c->mat, c->prec == SBP_FP32_KAHAN);
     c->step_plan = step_plan(c->order, c->nx, c->ny);
-    c->whole = step_default(c);
     if (c->prec == SBP_FP64)
       c->march_fns = (c->order == 2 ? march_launcher_o2_f64
                                     : (c->order == 4 ? march_launcher_o4_f64 : march_launcher_o6_f64))(c->phys, c->mat);
@@ -830,8 +846,8 @@ int build_ctx(const sbp_problem *desc, sbp_ctx *c)
       HIP_OR_FAIL(c->march_fns.resident(&resident));
       if (c->step_plan.ok) c->march_plan = march_plan(c->order, c->nx, c->ny, c->step_plan.px, resident);
       c->march = march_default(c);
-      c->whole = c->whole || c->march;
     }
+    c->whole = c->march || step_default(c);
   }
 
   HIP_OR_FAIL(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));

@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from problems_helper import P
+from test_gpu_step import problem
 
 pytestmark = pytest.mark.gpu
 
@@ -60,3 +61,25 @@ def test_forced_grids_beyond_the_patches(capi):
         ctx.set_fused(False)
         ctx.reset_schedule()
         assert ctx.schedule == "pairs"
+
+
+@pytest.mark.parametrize("kind,order,prec,nx,ny,want", [
+    # order 6 in FP32: patches up to the size marching begins at
+    ("arrays", 6, P.FP32_KAHAN, 256, 570, "patches"), ("arrays", 6, P.FP32_KAHAN, 1141, 179, "patches"),
+    ("arrays", 6, P.FP32_KAHAN, 471, 471, "march"), ("unit", 6, P.FP32_KAHAN, 399, 399, "patches"),
+    ("unit", 6, P.FP32, 1133, 132, "patches"), ("unit", 6, P.FP32, 401, 401, "march"),
+    ("unit", 6, P.FP64, 299, 299, "patches"), ("unit", 6, P.FP64, 301, 301, "stages"), ("unit", 6, P.FP64, 381, 381, "march"),
+    # ribbons: order 4 FP64 with arrays marches wide ones earlier
+    ("arrays", 4, P.FP64, 3125, 96, "march"), ("arrays", 4, P.FP64, 96, 3125, "patches"),
+    ("arrays", 4, P.FP64, 2100, 128, "patches"), ("unit", 4, P.FP64, 3125, 96, "patches"),
+    ("arrays", 4, P.FP64, 96, 5200, "march")])
+def test_lines_between_the_schedules(capi, kind, order, prec, nx, ny, want):
+    """Either side of the lines, and the bits of one launch per stage there."""
+    print("line between schedules", kind, order, prec, nx, ny, flush=True)
+    spec, v, _ = problem(kind, order, nx, ny, P.BC_WALL, prec)
+    dt = 0.2 / max(spec.hix, spec.hiy)
+    with capi.Context(spec) as ctx:
+        assert ctx.schedule == want
+        got = ctx.rk4_advance(v, 0.0, dt, 3)
+        ctx.set_fused(False)
+        assert np.array_equal(ctx.rk4_advance(v, 0.0, dt, 3), got)
