@@ -27,6 +27,7 @@
 
 #include "../../include/sbp_hip.h"
 #include "sbp_batch_impl.hpp"
+#include "sbp_corr_plan.hpp"
 #include "sbp_ctx.hpp"
 #include "sbp_host.hpp"
 
@@ -210,11 +211,8 @@ using vbf8 = __attribute__((ext_vector_type(8))) __bf16;
 using vbf2 = __attribute__((ext_vector_type(2))) __bf16;
 using f32x2 = __attribute__((ext_vector_type(2))) float;
 using vi16x2 = __attribute__((ext_vector_type(2))) short;
-constexpr int FW = 64, FOUT = FW - 6;  // window width, output columns
 constexpr int FPX = FW + 2;            // pixels per LDS row (one zero pad each side)
 constexpr int F1S = 40;                // LDS channel stride of the 32-channel rows (80 B)
-constexpr int FUSED_HALO = 9;          // row steps beyond the chunk's rows
-constexpr int FUSED_MAX_ROWS = 32;     // output rows per block (LDS staging)
 constexpr int FIN_PARTS = FPX * C_INP / 4;  // 8-byte parts of an input row
 
 __device__ __forceinline__ f32x4 mfma32(bf16x8 a, bf16x8 b, f32x4 c)
@@ -253,36 +251,6 @@ struct NetEnergyArgs {
   double *partial;
   int order, band;
 };
-
-// Rows of each block's chunk (at most FUSED_MAX_ROWS, chunks as even as
-// possible) and the blocks, for nb images.  A block runs its rows and
-// FUSED_HALO more in whole groups of six steps; a step takes 0.55 us where a CU
-// has one block and 0.43 us per block where it has more.  The split of the
-// least total is taken: tall chunks for many images, low ones that spread a few
-// over the chip (64 corrected steps of one 257^2 image 4.2 ms with chunks of 29
-// rows, 3.1 with 6; a training step of one 172 and 142 us).
-inline int net_chunk_rows(int nb, int H, int W)
-{
-  constexpr int kCus = 256;
-  const long strips = (long)nb * ((W + FOUT - 1) / FOUT);
-  int best = 1;
-  double least = 1e300;
-  for (int n = (H + FUSED_MAX_ROWS - 1) / FUSED_MAX_ROWS; n <= H; n++) {
-    const int rows = (H + n - 1) / n;
-    const long blocks = strips * ((H + rows - 1) / rows);
-    const double cost = (rows + FUSED_HALO + 5) / 6 * 6 * std::max(0.55, 0.43 * (double)((blocks + kCus - 1) / kCus));
-    if (cost < least) {
-      least = cost;
-      best = rows;
-    }
-  }
-  return best;
-}
-inline long net_blocks_per_image(int nb, int H, int W)
-{
-  const int rows = net_chunk_rows(nb, H, W);
-  return (long)((W + FOUT - 1) / FOUT) * ((H + rows - 1) / rows);
-}
 
 // T: type of the state whose corrected energy the epilogue reduces; void for
 // plain inference.  KEEP: also store the activations of layers 1 and 2 (the
@@ -1475,9 +1443,7 @@ int sbp_corr_create(int nx, int ny, int batch, sbp_corrector **out)
   if (!rc) rc = dmalloc(&c->rejected, sizeof(int));
   if (!rc) rc = dmalloc(&c->idx, sizeof(int) * batch);
   if (!rc) rc = dmalloc(&c->bpart, sizeof(double) * batch * 64);
-  long cparts = 0;  // (fewer images may take more blocks each)
-  for (int n = 1; n <= batch; n++) cparts = std::max(cparts, n * net_blocks_per_image(n, ny, nx));
-  if (!rc) rc = dmalloc(&c->cpart, sizeof(double) * cparts);
+  if (!rc) rc = dmalloc(&c->cpart, sizeof(double) * batch * net_most_blocks(ny, nx));
   if (!rc) rc = dmalloc(&c->be_old, sizeof(double) * batch);
   if (!rc) rc = dmalloc(&c->brej, sizeof(int) * batch);
   if (!rc) {
