@@ -754,7 +754,6 @@ void release(sbp_ctx *c)
   for (void *p : c->rkw)
     if (p) (void)hipFree(p);
   if (c->rk_host) (void)hipHostFree(c->rk_host);
-  if (c->rhs_out) (void)hipHostFree(c->rhs_out);
   for (hipEvent_t &e : c->ev)
     if (e) (void)hipEventDestroy(e);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -867,7 +866,6 @@ int build_ctx(const sbp_problem *desc, sbp_ctx *c)
   if (!c->aos_host) {
     if ((rc = dalloc(&c->aos, aos_bytes))) return rc;
   } else {
-    HIP_OR_FAIL(hipHostMalloc(reinterpret_cast<void **>(&c->aos), aos_bytes, hipHostMallocDefault));
     if (!is1d(c->phys)) {
       c->rhs_plan = rhs_plan(c->order, c->nx, c->ny);
       if (c->rhs_plan.ok) {
@@ -877,8 +875,11 @@ int build_ctx(const sbp_problem *desc, sbp_ctx *c)
         c->rhs_launch = reg(c->phys, c->mat);
       }
     }
-    if (c->rhs_launch)
-      HIP_OR_FAIL(hipHostMalloc(reinterpret_cast<void **>(&c->rhs_out), aos_bytes, hipHostMallocDefault));
+    // one allocation for both vectors: a pinned one costs 25 us to make and give
+    // back, whatever its size, and was half of a small context's cost
+    const size_t step = (aos_bytes + 255) / 256 * 256;
+    HIP_OR_FAIL(hipHostMalloc(reinterpret_cast<void **>(&c->aos), c->rhs_launch ? 2 * step : step, hipHostMallocDefault));
+    if (c->rhs_launch) c->rhs_out = c->aos + step / sizeof(double);
   }
   c->npartials = 1024;
   if ((rc = dalloc(&c->partials, sizeof(double) * c->npartials)) || (rc = dalloc(&c->scalar, 2 * sizeof(double))))

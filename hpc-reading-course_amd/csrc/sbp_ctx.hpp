@@ -43,7 +43,7 @@ struct sbp_ctx {
   // one right-hand side of vectors in host memory in one launch (sbp_rhs.hpp)
   sbp::RhsLaunchFn rhs_launch = nullptr;
   sbp::StepPlan rhs_plan{};
-  double *rhs_out = nullptr;  // its result (pinned host memory)
+  double *rhs_out = nullptr;  // its result (behind aos in its allocation)
   bool whole = false;
   // whole steps march along the grid (sbp_march.hpp)
   sbp::MarchFns march_fns{};
