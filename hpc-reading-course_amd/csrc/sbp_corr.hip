@@ -37,7 +37,6 @@ using sbp::host::fail;
 
 namespace {
 
-using bf16x4 = __attribute__((ext_vector_type(4))) short;
 using f32x4 = __attribute__((ext_vector_type(4))) float;
 typedef unsigned short bf16;
 
@@ -62,8 +61,6 @@ __device__ __forceinline__ bf16 f2bf(float f)
   u += 0x7fffu + ((u >> 16) & 1u);  // round to nearest even
   return (bf16)(u >> 16);
 }
-
-__device__ __forceinline__ float bf2f(bf16 h) { return __uint_as_float(((unsigned)h) << 16); }
 
 // Whether the correction acts at grid point (i, j) of an H x W image: the
 // points closer than `band` to a wall (the boundary-closure rows) keep the
@@ -1560,7 +1557,6 @@ int sbp_corr_gradients(sbp_corrector *c, const float *raw, const float *target, 
   if (!raw || !target || !grads) return fail(SBP_EINVAL, "null argument");
   const long npix = (long)nb * c->H * c->W;
   float *draw = nullptr, *dtgt = nullptr;
-  int *didx = nullptr;
   if ((rc = dmalloc(&draw, sizeof(float) * npix * C_IN))) return rc;
   if ((rc = dmalloc(&dtgt, sizeof(float) * npix * C_OUT))) {
     (void)hipFree(draw);
@@ -1573,7 +1569,6 @@ int sbp_corr_gradients(sbp_corrector *c, const float *raw, const float *target, 
       hipMemcpyAsync(dtgt, target, sizeof(float) * npix * C_OUT, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
       hipMemcpyAsync(c->idx, idx.data(), sizeof(int) * nb, hipMemcpyHostToDevice, c->stream) != hipSuccess)
     rc = fail(SBP_EHIP, "upload failed");
-  (void)didx;
   if (!rc) {
     hipLaunchKernelGGL(gather_kernel, dim3(grid_for(npix)), dim3(256), 0, c->stream, draw, dtgt, c->idx, nb,
                        (long)c->H * c->W, c->norm, c->norm + NORM_OUT, c->X0, c->Tg);
