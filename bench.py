@@ -69,11 +69,21 @@ def bytes_per_dof(precision, materials=False, C=3):
 WHOLE, TWO, ONE = "whole step", "two-stage", "one stage per launch"
 
 
-def schedule_of(fused, stage_ms):
-    """A context's schedule: a whole step is timed into the first slot alone."""
-    if stage_ms[0] > 0 and not np.any(np.asarray(stage_ms[1:]) > 0):
-        return WHOLE
-    return TWO if fused else ONE
+# what a context's schedule (capi.SCHEDULES) moves through memory
+SCHEDULE = {"line": WHOLE, "patches": WHOLE, "march": WHOLE, "pairs": TWO, "stages": ONE}
+
+
+def kernel_names(sched):
+    """The kernel in each of a step's four stage slots."""
+    if sched == "stages":
+        return {k: "stage2d_kernel, RK4 stage %d" % k for k in range(1, 5)}
+    if sched == "pairs":
+        return {1: "pair2d_kernel, RK4 stages 1-2 (interior tiles and frame patches)", 2: "(no launch)",
+                3: "pair2d_kernel, RK4 stages 3-4 (interior tiles and frame patches)", 4: "(no launch)"}
+    return {1: {"march": "march2d_kernel, a whole RK4 step (strips and frame patches)",
+                "patches": "step2d_kernel, a whole RK4 step (patches on chip)",
+                "line": "line_kernel, whole RK4 steps"}[sched],
+            2: "(no launch)", 3: "(no launch)", 4: "(no launch)"}
 
 
 def launch_bytes(spec, schedule):
@@ -139,9 +149,8 @@ def gpu_run(spec, v0, dt, steps, warmup, stage_steps=None, fused=None):
     try:
         if fused is not None:
             ctx.set_fused(fused)
-        fused = ctx.fused
         ctx.set_state(v0)
-        if fused and TILE_ROWS:
+        if ctx.fused and TILE_ROWS:
             ctx.set_fused(True, TILE_ROWS)
             rows = TILE_ROWS
         else:
@@ -154,19 +163,20 @@ def gpu_run(spec, v0, dt, steps, warmup, stage_steps=None, fused=None):
         wall = time.perf_counter() - t0
         stage_ms = ctx.time_stages(dt, stage_steps or max(3, min(steps, 20)))
         energy = ctx.state_energy()
+        sched = ctx.schedule
     finally:
         ctx.close()
-    return wall, ev_ms, stage_ms, energy, fused, rows
+    return wall, ev_ms, stage_ms, energy, sched, rows
 
 
 def measure(spec, v0, dt, steps, warmup, fused=None):
-    wall, ev_ms, stage_ms, energy, fused, rows = gpu_run(spec, v0, dt, steps, warmup, fused=fused)
+    wall, ev_ms, stage_ms, energy, sched, rows = gpu_run(spec, v0, dt, steps, warmup, fused=fused)
     dofs = spec.nx * spec.ny * spec.components
     mat = spec.material == 2
     bpd = bytes_per_dof(spec.precision, mat, spec.components)
     step_kernel_s = float(np.sum(stage_ms)) * 1e-3
     achieved = dofs * bpd / step_kernel_s / 1e9
-    schedule = schedule_of(fused, stage_ms)
+    schedule = SCHEDULE[sched]
     lb = launch_bytes(spec, schedule)
     k_achieved = sum(lb) / step_kernel_s / 1e9
     dom = int(np.argmax(stage_ms))
@@ -177,7 +187,7 @@ def measure(spec, v0, dt, steps, warmup, fused=None):
         bytes_per_dof=bpd, achieved_gbs=achieved, frac=achieved / PEAK_HBM_GBS, energy=energy,
         kernel_bytes_per_dof=sum(lb) / dofs, kernel_achieved_gbs=k_achieved, kernel_frac=k_achieved / PEAK_HBM_GBS,
         launch_bytes=lb, dominant_launch=dom + 1, dominant_gbs=dom_gbs, dominant_frac=dom_gbs / PEAK_HBM_GBS,
-        schedule=schedule, tile_rows=rows if schedule == TWO else None)
+        schedule=schedule, kernels=kernel_names(sched), tile_rows=rows if schedule == TWO else None)
 
 
 def batched(count=256, steps=500, warmup=10, prec=1):
@@ -233,10 +243,9 @@ def reflection_2d(steps=2000, warmup=0):
             wall = time.perf_counter() - t0
             finals[name] = ctx.get_state()
             stage_ms = ctx.time_stages(dt, 5)
-            fused = ctx.fused
+            schedule = SCHEDULE[ctx.schedule]
         dofs = spec.nx * spec.ny * 3
         bpd = bytes_per_dof(prec, True)
-        schedule = schedule_of(fused, stage_ms)
         lb = launch_bytes(spec, schedule)
         kbpd = sum(lb) / dofs
         step_s = float(np.sum(stage_ms)) * 1e-3
@@ -414,13 +423,6 @@ def main():
     stream_gbs = capi.stream_bandwidth(plane_bytes, nr, nw, 5)
     log("flat stream, %d planes read + %d written: %.0f GB/s" % (nr, nw, stream_gbs))
     traffic = MEASURED_TRAFFIC.get((spec.nx, spec.order, spec.precision, main_m["schedule"], dom))
-    if main_m["schedule"] == WHOLE:
-        names = {1: "march2d_kernel, a whole RK4 step (strips and frame patches)"}
-    elif main_m["schedule"] == TWO:
-        names = {1: "pair2d_kernel, RK4 stages 1-2 (interior tiles and frame patches)", 2: "(no launch)",
-                 3: "pair2d_kernel, RK4 stages 3-4 (interior tiles and frame patches)", 4: "(no launch)"}
-    else:
-        names = {k: "stage2d_kernel, RK4 stage %d" % k for k in range(1, 5)}
     out = {
         "metric": "DOF-updates/s & % HBM roofline; time to L2 err 1e-4: chosen vs plain FP64",
         "value": main_m["dof_updates_per_s"],
@@ -440,7 +442,7 @@ def main():
                    "parallelism": "single GPU"},
         "roofline": {"bound": "hbm", "achieved": main_m["dominant_gbs"], "peak": PEAK_HBM_GBS,
                      "unit": "GB/s", "frac": main_m["dominant_frac"], "traffic": traffic,
-                     "kernel": names[dom], "schedule": main_m["schedule"],
+                     "kernel": main_m["kernels"][dom], "schedule": main_m["schedule"],
                      "algorithmic_bytes_per_launch": main_m["launch_bytes"][dom - 1],
                      "mean_launch_ms": main_m["stage_ms"][dom - 1],
                      "bytes_basis": "each value the launch must read or write, once (bench.launch_bytes)",
