@@ -41,8 +41,8 @@ PEAK_HBM_GBS = 8000.0
 # 2.0 + WRITE_SIZE x 1.0 KiB (the factors that turn the counters of a 1 GiB
 # plain copy in the same runs into the bytes it reads and writes):
 # profiles/march2d_acoustic_4097sq_order4_fp64_hbm_counters.md.
-MEASURED_TRAFFIC = {(4097, 4, 0, "whole step", 1): (237420 * 2.0 + 395820 * 1.0) * 1024}
-MEASURED_AT = "c5497f2"
+MEASURED_TRAFFIC = {(4097, 4, 0, "whole step", 1): (237798 * 2.0 + 396911 * 1.0) * 1024}
+MEASURED_AT = "8d4cdde"
 
 
 def pkg(sub):
