@@ -51,7 +51,8 @@ enum {
 // interior beyond its (CLS+3R)-deep frame: low segments fill the chip where
 // there are few instances, high ones lead in less often (FP32 with rho/K
 // arrays, us per step at 8, 32 and 128 rows, best two-stage: 16 x 257^2 25 / 33
-// / 90, 37; 48 of 129^2 .. 1025^2 298 / 224 / 199, 421).
+// / 90, 37; 48 of 129^2 .. 1025^2 298 / 224 / 199, 421).  A segment's rows run in
+// whole groups of 2R+1 (8 as 10 at order 4, 128 as 130).
 constexpr BatchConfig kConfigs[] = {
     {256, 32, 4, 1, 0}, {256, 64, 4, 1, 0}, {256, 16, 4, 1, 0}, {256, 32, 2, 1, 0}, {256, 32, 8, 1, 0},
     {256, 64, 2, 1, 0}, {128, 32, 8, 1, 0}, {128, 64, 8, 1, 0}, {128, 16, 8, 1, 0}, {128, 32, 4, 1, 0},

@@ -251,7 +251,7 @@ struct NetEnergyArgs {
 
 // T: type of the state whose corrected energy the epilogue reduces; void for
 // plain inference.  KEEP: also store the activations of layers 1 and 2 (the
-// training forward; each block its own rows and 58 columns): 78 us for 16
+// training forward; each block its own rows and 58 columns): 59 us for 16
 // images of 257^2 against 289 us for one convolution launch per layer.
 template <typename T, bool KEEP>
 __global__ __launch_bounds__(256, 3) void fused_net_kernel(const bf16 *__restrict__ X, int nimg, int H, int W, int rows,
@@ -662,7 +662,7 @@ __global__ __launch_bounds__(256, 3) void fused_back_kernel(const bf16 *__restri
 // chunks; the partials are summed in a fixed order (wgrad_reduce_kernel).
 //
 // Bound: the LDS reads and transposing writes around each row's barrier.  16
-// images of 257^2, layers 3 / 2 / 1: 37 / 47 / 28 us; with 2-byte gathers of both operands from global memory and
+// images of 257^2, layers 3 / 2 / 1: 36 / 46 / 28 us; with 2-byte gathers of both operands from global memory and
 // 16-pixel MFMAs 651 / 710 / 278 us, and 1228 us more for each layer's bias
 // gradient in a kernel of its own.  The reduction of all partials takes 9 us
 // (three launches of one serial sum per entry: 271 us each).

@@ -83,8 +83,8 @@ template <typename T> struct StageArgs {
 
 template <typename T, int ORDER> __constant__ EdgeTable<T, ORDER> c_edge = make_edge_table<T, ORDER>();
 
-// a * b + c: one rounding in FP32, two in FP64.  Every unit is compiled without
-// contraction and multiply-adds are written with this, so the FP64 kernels
+// a * b + c: one rounding in FP32, two in FP64.  The solver units (*_f64, *_f32)
+// are compiled without contraction and multiply-adds are written with this, so the FP64 kernels
 // round like the reference's loops and every kernel (one launch per stage, two
 // stages, whole steps, ensembles) forms the same FP32 values from the same
 // operands, whatever the compiler makes of the code around them.
@@ -1121,8 +1121,8 @@ __global__ __launch_bounds__(256) void rhs1d_kernel(StageArgs<T> a)
 //   stage 4: U = U + dt/6 (S + k4)   (Kahan form: the increment is compensated)
 // Bound: the latency of one stage (LDS taps, a serial sum, a barrier).
 // One launch per stage took 7.0 us per step on 201 points (order 4 advection)
-// and 10.8 on 5001 (order 6 reflection), launch latency; this takes 0.64 and
-// 1.63.
+// and 10.8 on 5001 (order 6 reflection), launch latency; this takes 0.63 and
+// 1.62.
 template <typename T> struct LineArgs {
   const T *u, *comp;  // state read
   T *uo, *co;         // state written (the same arrays when one block holds the line)

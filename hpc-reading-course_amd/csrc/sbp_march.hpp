@@ -22,7 +22,7 @@
 // every stage is an interior point of the operator; the D-deep frame is cut
 // into patches that blocks of the same launch step on chip (sbp_step.hpp).
 //
-// What bounds it: order 4 FP64, 4097^2, takes 223 us per step (452 as two
+// What bounds it: order 4 FP64, 4097^2, takes 217 us per step (452 as two
 // launches).  806 MB of U and U' are 147 us at what a copy reaches; a row costs
 // a CU's LDS 0.6 us for the neighbours (32 words read and 8 written per column)
 // and its SIMDs 0.8 us for 200 instructions, which the barrier of each row lets
@@ -253,7 +253,9 @@ __device__ __forceinline__ void march_strip(const StepArgs<T> &a, T *lds, int st
   };
   each_int(lead, std::make_integer_sequence<int, 8 * R>{});
   // (a segment has at least one row; a loop that might not run would let the
-  // compiler sink the leading rows' results into it, with all their operands)
+  // compiler sink the leading rows' results into it, with all their operands.
+  // Rows run in whole groups of 2R+1: the last group's surplus is computed and
+  // dropped, so 12 rows of order 4 cost 15)
   const int nk = (j1 - j0) + 8 * R;
   int k = 8 * R;
   auto row = [&](auto N) { iter(Int<(8 * R + decltype(N)::value) % WN>{}, Int<4>{}, k + decltype(N)::value); };

@@ -7,7 +7,8 @@
 //
 // What bounds it: a block's chain of six stages with a barrier each, and the
 // points evaluated for their neighbours (order 4: 64 x 32 loaded for 40 x 8).
-// 201^2, order 4: 27 us per attempt, thirteen launches 70 (and 90 when the
+// 201^2, order 4: 27 us per attempt (the kernel 16, then the host's sum and
+// decision), thirteen launches 70 (and 90 when the
 // error came back through a copy call).
 #pragma once
 #include "sbp_step.hpp"

@@ -375,12 +375,12 @@ __host__ __device__ inline int march_frame(int order, int px, int ny)
 // The cut of the marched region into strips and segments.  A segment costs its
 // rows and the 4 order rows it leads in with, and each further block per CU
 // slows the others down by about a quarter of what one alone takes (4097^2
-// FP32 190 / 130 / 128 / 126 us per step at 1 .. 4 per CU, 2049^2 58 / 43 / 41
-// / 45, 1025^2 21 / 17 / 17 / 19): as many blocks per CU, at most `resident`,
+// FP32 172 / 122 / 126 / 116 us per step at 1 .. 4 per CU, 2049^2 51 / 38 / 38
+// / 38, 1025^2 21 / 19 / 18 / 21): as many blocks per CU, at most `resident`,
 // as make (rows + lead) (1 + w / 4) smallest.  A frame of few patches takes
 // its place within them, so that all blocks of a launch run at once (1025^2
-// FP64: 31 us per step, 36 with another 88 blocks to wait for; both with S in
-// LDS); a larger one is worth a longer launch (4097^2 FP64 255 / 288).  Where a
+// FP64: 28.5 us per step, 31.7 with another 88 blocks to wait for); a larger one
+// is worth a longer launch (4097^2 FP64 216 / 302).  Where a
 // CU holds one block (order 6 FP64) patches that follow wait for whole blocks
 // and cost about as much as 3 order rows, so the cheaper of the two is taken,
 // rows counted as they run, in whole groups of order + 1 (us per step, within /
