@@ -182,7 +182,8 @@ long march_side(const sbp_ctx *c)
 // 23.4; longer ones are still better marched (64 x 60000 201 / 338, 60000 x 64
 // 87 / 176).  With rho/K arrays order 4 FP64 patches cost more than two launches
 // on wide ones already from 280000 points: 3125 x 96 marched 18.9, patches 29.4,
-// launches 25.8; tall ones not (96 x 3125 36, 37, 49).
+// launches 25.8; tall ones gain in patches as the others do (61 x 3697 marched
+// 34, patches 28, launches 61).
 bool march_default(const sbp_ctx *c)
 {
   long least = march_side(c);
